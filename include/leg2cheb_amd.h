@@ -188,7 +188,11 @@ int l2c_plan_graph(fmm_plan *plan, int enable);
  * per 65,535 lines; any nlines).  Line l (l < nlines) has first element at
  * (l / n0) * line_stride1 + (l % n0) * line_stride0 and its elements at that
  * offset + i * elem_stride.  Device pointers.  With n0 = nlines,
- * line_stride0 = distance between consecutive lines. */
+ * line_stride0 = distance between consecutive lines.
+ * Calls of two lines and more of plans of N <= 1536 (128 lines and more up to
+ * N = 2048) run as one dense product on blocks that create_fmm builds
+ * (N^2 / 2 doubles per direction; environment L2C_DENSE_MAXN at plan creation
+ * lowers the bound, 0 keeps the FMM, as L2C_DIRECT_MAXN = 0 does). */
 int l2c_execute_lines_device(fmm_plan *plan, const double *d_in, double *d_out,
                              size_t direction, size_t nlines, size_t n0,
                              size_t line_stride0, size_t line_stride1,

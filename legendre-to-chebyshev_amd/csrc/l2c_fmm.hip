@@ -2757,6 +2757,24 @@ __global__ void __launch_bounds__(256) k_direct_band(const double *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
+// two doubles at any 8-byte boundary, moved as one 16-byte access
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+// Buffer descriptor of n doubles at p (both wave-uniform): raw buffer loads
+// check each dword against the length and return zero past it.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t line_rsrc(const double *p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 8 * n, 0x00020000);
+}
+__device__ __forceinline__ double load_one(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+}
+// The two doubles at byte voff (per lane) + soff (uniform) of the buffer.
+__device__ __forceinline__ d2 load_pair(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+  return __builtin_bit_cast(d2, v);
+}
+
 // Batched lines of the direct path (N <= kDenseMaxN) as dense products on FP64
 // MFMA: per parity p, OUT_p (NPP x LT) = K_p (NPP x NPP) IN_p (NPP x LT) for a
 // tile of LT lines, K_p upper triangular (the direct sums of
@@ -2950,25 +2968,33 @@ static size_t dense_shared_bytes(int NPP) {
 
 // Batched lines of the direct path with kDenseMaxN < N <= kGemmMaxN: the same
 // parity blocks K_p (NPP up to 2048) as a tiled product on FP64 MFMA.  A
-// work-group owns 64 pair-rows (row tiles 4 rt + wave, one per wave) of one
-// parity p for 32 lines and walks the columns c >= 64 rt in chunks of 64:
-// the chunk's inputs 2c + p of its 32 lines are staged in LDS [c][line], then
-// each wave runs v_mfma_f64_16x16x4f64 with A = K_p fragments (global
-// memory, L2/MALL-resident) and B = the staged rows, two 16-line column
-// tiles.  The next chunk's inputs and fragments load into registers during
-// the current chunk's products.  The results go out through the same LDS
-// tile.  The two parities are separate work-groups: twice as many, each
-// with half the registers and LDS of one holding both, and row tile 0 (which
-// walks all NPP / 64 chunks) splits its chain in two.  Grid (2 x line
-// tiles, row tiles), the parity in the lowest bit of blockIdx.x:
-// the long row tiles of both parities are dispatched first, and consecutive
-// work-groups share a row tile's K rows.
-// LDS row stride 33 doubles: the staging writes (lanes along c) and the
-// result reads step 66 dwords, two banks apart, while each 16-lane row of an
-// MFMA operand read stays contiguous
-constexpr int kGemmRT = 64, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmLTP = 33;
+// work-group owns 32 pair-rows of both parities for 32 lines (wave: parity
+// wave & 1, 16-row tile wave >> 1, two 16-line column tiles) and walks the
+// columns c >= its first row in chunks of 64 pairs: the chunk's inputs
+// 2c, 2c + 1 of its 32 lines are staged in LDS [parity][line][c], then each
+// wave runs v_mfma_f64_16x16x4f64 with A = K_p fragments (global memory,
+// L2/MALL-resident) and B = the staged rows.  The next chunk's inputs and
+// fragments load into registers during the current chunk's products.
+// LDS row stride KC + 2 = 66 doubles: the writes of contiguous lines (lanes
+// along c) and the operand reads (16 lines x 2 columns per half-wave, 132
+// dwords apart) fall in distinct banks.
+// Contiguous lines move both parities of a column as one 16-byte access;
+// strided ones 32 lines of one element per half-wave, and their results go
+// out of the accumulators as they are (16 lines of one element per store).
+// Grid (line tiles, row tiles): the long row tiles are dispatched first, and
+// consecutive work-groups share a row tile's K rows.
+// Bound by the matrix cores on large calls (4096 lines of 1024 41 TFLOP/s,
+// 2048 lines of 3000 54 TFLOP/s of the 72 that a large FP64 product reaches;
+// L2 carries 64 KB of fragments and inputs per 128 products of a wave), by
+// the chain of chunks, about 1.4 us each, on small ones.  One parity per
+// work-group of 64 rows, inputs [c][line] at stride 33 with lanes along c for
+// strided lines too, masked fragment loads, measured before it: 1024 lines of
+// 1024 24.0 -> 19.4 us, 4096 lines of 2048 212 -> 177, 32 lines of 2048 35 ->
+// 27.  Splitting a tile's columns over two or four groups of waves: 4 lines of
+// 2048 26 -> 24 us, but 1024 lines of 1024 19.4 -> 20.5 and 25.5.
+constexpr int kGemmRT = 32, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmKP = kGemmKC + 2;
 constexpr size_t kGemmFewLines = 16384;
-// The work of tile (bx, by) of the tiled dense product (grid (2 x line tiles,
+// The work of tile (bx, by) of the tiled dense product (grid (line tiles,
 // row tiles)); k_lines_gemm runs one grid of them, k_lines_gemm_multi the
 // grids of several size classes in one launch.
 template <bool CONTIG>
@@ -2977,12 +3003,12 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
                                                 size_t nlines, int N, int NPP,
                                                 const double *__restrict__ K, unsigned bx,
                                                 unsigned by, double *sm) {
-  constexpr int LTP = kGemmLTP, KC = kGemmKC, LT = kGemmLT;
+  constexpr int KP = kGemmKP, KC = kGemmKC, LT = kGemmLT;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rt = (int)by, p = bx & 1;
-  const size_t l0 = (size_t)(bx >> 1) * LT;
-  size_t *toff = (size_t *)(sm + KC * LTP);
+  const int rt = (int)by, p = wave & 1;
+  const size_t l0 = (size_t)bx * LT;
+  size_t *toff = (size_t *)(sm + 2 * LT * KP);
   int *tlen = (int *)(toff + LT);
   if (tid < LT) {
     const size_t line = l0 + tid;
@@ -2990,96 +3016,145 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     tlen[tid] = line < nlines ? line_len(lm, line, N) : 0;
   }
   __syncthreads();
-  const int NR = NPP >> 4, nkt = NPP >> 2, R = 4 * rt + wave;
+  const int NR = NPP >> 4, nkt = NPP >> 2, R = 2 * rt + (wave >> 1);
   const bool active = R < NR;  // the last row tile may be partly past NPP
   const size_t es = CONTIG ? 1 : lm.es;
   const d4 z = {0.0, 0.0, 0.0, 0.0};
-  d4 D0 = z, D1 = z;  // 16-line halves
-  const double *Bp = sm + (lane >> 4) * LTP + (lane & 15);
-  const double *Kp = K + ((size_t)(p * NR + R) * nkt) * 64 + lane;
-  constexpr int QS = KC * LT / kGemmNT;  // staged inputs per thread per chunk
-  static_assert(KC == 64 && kGemmRT == 64 && kGemmNT == 256, "thread q-th line is 4 q + wave");
-  // this thread's lines in every chunk and in the results: 4 q + wave (q <
-  // QS), column c0 + lane (row 64 rt + lane); their starts and lengths are
-  // wave-uniform and kept in scalar registers
-  const double *src[QS];
-  double *dst[QS];
-  int len[QS];
+  // sums of the two 16-line halves: each chunk's own, added to the total (one
+  // long chain over up to 1024 columns would lose a digit: 2-norm error
+  // against double-double sums at N = 2000 1.3-1.8e-15 in one chain)
+  d4 D0 = z, D1 = z;
+  const double *Bp = sm + (p * LT + (lane & 15)) * KP + (lane >> 4);
+  // the fragments of row tile R (zeros past NPP, and for a row tile past it)
+  const __amdgpu_buffer_rsrc_t Kr =
+      line_rsrc(K + (size_t)(p * NR + (active ? R : 0)) * nkt * 64, active ? 64 * nkt : 0);
+  static_assert(KC == 64 && LT == 32 && kGemmRT == 32 && kGemmNT == 256, "thread maps below");
+  // staged inputs of this thread in every chunk.  CONTIG: pair c0 + lane of
+  // lines 4 q + wave, read through a buffer descriptor of the line's length
+  // (reads past its end return zero); else element 2 (c0 + wave + 4 q) +
+  // lane / 32 of line lane % 32 (a line past nlines reads line 0 and stores
+  // nothing).
+  constexpr int QL = CONTIG ? 8 : 1, QE = 16;
+  __amdgpu_buffer_rsrc_t src[QL];
+  const double *src0 = nullptr;
+  if constexpr (CONTIG) {
 #pragma unroll
-  for (int q = 0; q < QS; q++) {
-    const size_t o = toff[4 * q + wave];
-    const size_t ou = (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)o) |
-                      ((size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(o >> 32)) << 32);
-    len[q] = __builtin_amdgcn_readfirstlane(tlen[4 * q + wave]);
-    src[q] = in + ou + p * es;
-    dst[q] = out + ou + p * es;
+    for (int q = 0; q < QL; q++) {
+      const size_t o = toff[4 * q + wave];
+      const size_t ou = (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)o) |
+                        ((size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(o >> 32)) << 32);
+      src[q] = line_rsrc(in + ou, __builtin_amdgcn_readfirstlane(tlen[4 * q + wave]));
+    }
+  } else {
+    src0 = in + toff[lane & 31] + (size_t)(2 * wave + (lane >> 5)) * es;
   }
-  // chunk c0's inputs of this thread and this wave's fragments, into registers
-  double e[QS], an[KC / 4];
-  auto fetch = [&](int c0) {
-    const int ks0 = c0 == kGemmRT * rt ? 4 * wave : 0, nks = min(KC, NPP - c0) >> 2;
-    if (active && ks0 == 0 && nks == KC / 4) {
+  double e[QE], a[KC / 4];
+  // the loads of chunk c0 (past NPP: zeros).  The empty asm keeps the
+  // compiler from carrying one address register per load through the loop.
+  auto fetch_in = [&](int c0) {
+    asm volatile("" : "+s"(c0));
+    if constexpr (CONTIG) {
 #pragma unroll
-      for (int ks = 0; ks < KC / 4; ks++) an[ks] = Kp[((c0 >> 2) + ks) * 64];
+      for (int q = 0; q < QL; q++) {
+        const d2 t = load_pair(src[q], 16 * lane, 16 * c0);
+        e[2 * q] = t.x;
+        e[2 * q + 1] = t.y;
+      }
+    } else {
+      const double *s0 = src0 + (size_t)(2 * c0) * es;
+      if (2 * (c0 + KC) <= N) {
+#pragma unroll
+        for (int q = 0; q < QE; q++) e[q] = s0[(size_t)(8 * q) * es];
+      } else {
+        const int i0 = 2 * (c0 + wave) + (lane >> 5);
+#pragma unroll
+        for (int q = 0; q < QE; q++) e[q] = i0 + 8 * q < N ? s0[(size_t)(8 * q) * es] : 0.0;
+      }
+    }
+  };
+  auto fragment = [&](int c0, int ks) { return load_one(Kr, 8 * lane + 512 * (ks & 7), 128 * c0 + 512 * (ks & 8)); };
+  fetch_in(kGemmRT * rt);
+#pragma unroll
+  for (int ks = 0; ks < KC / 4; ks++) a[ks] = fragment(kGemmRT * rt, ks);
+  // one k-step: its products, then the same step's fragment of chunk cn
+  d4 S0, S1;
+  auto step = [&](int ks, int cn) {
+    const double *b = Bp + 4 * ks;
+    S0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[0], S0, 0, 0, 0);
+    S1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[16 * KP], S1, 0, 0, 0);
+    a[ks] = fragment(cn, ks);
+    // (the scheduler would gather the loads and hold both chunks' fragments)
+    if (ks & 1) __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int c0 = kGemmRT * rt; c0 < NPP; c0 += KC) {
+    if constexpr (CONTIG) {
+#pragma unroll
+      for (int q = 0; q < QL; q++) {
+        sm[(4 * q + wave) * KP + lane] = e[2 * q];
+        sm[(LT + 4 * q + wave) * KP + lane] = e[2 * q + 1];
+      }
     } else {
 #pragma unroll
-      for (int ks = 0; ks < KC / 4; ks++)
-        an[ks] = active && ks >= ks0 && ks < nks ? Kp[((c0 >> 2) + ks) * 64] : 0.0;
+      for (int q = 0; q < QE; q++)
+        sm[((lane >> 5) * LT + (lane & 31)) * KP + wave + 4 * q] = e[q];
     }
-    const int c = c0 + lane;
-#pragma unroll
-    for (int q = 0; q < QS; q++) e[q] = 2 * c + p < len[q] ? src[q][(size_t)(2 * c) * es] : 0.0;
-  };
-  fetch(kGemmRT * rt);
-  for (int c0 = kGemmRT * rt; c0 < NPP; c0 += KC) {
-    // k-steps of this chunk for this wave: from its diagonal in the first
-    // chunk (K_p is zero below it), up to NPP in the last
-    const int ks0 = c0 == kGemmRT * rt ? 4 * wave : 0;
-    const int nks = min(KC, NPP - c0) >> 2;
-    double a[KC / 4];
-#pragma unroll
-    for (int q = 0; q < QS; q++) sm[lane * LTP + 4 * q + wave] = e[q];
-#pragma unroll
-    for (int ks = 0; ks < KC / 4; ks++) a[ks] = an[ks];
     __syncthreads();
-    // the next chunk's loads run during this chunk's products
-    if (c0 + KC < NPP) fetch(c0 + KC);
-    if (active && ks0 == 0 && nks == KC / 4) {
+    // the next chunk's inputs load during this chunk's products
+    int cn = c0 + KC;
+    fetch_in(cn);
+    asm volatile("" : "+s"(cn));
+    S0 = S1 = z;
+    // the tile's second row tile starts 16 columns on (K_p is zero before)
+    if (c0 != kGemmRT * rt || wave < 2) {
 #pragma unroll
-      for (int ks = 0; ks < KC / 4; ks++) {
-        const double *b = Bp + 4 * ks * LTP;
-        D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[0], D0, 0, 0, 0);
-        D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[16], D1, 0, 0, 0);
-      }
-    } else if (active) {
+      for (int ks = 0; ks < 4; ks++) step(ks, cn);
+    } else {
 #pragma unroll
-      for (int ks = 0; ks < KC / 4; ks++) {
-        if (ks < ks0 || ks >= nks) continue;
-        const double *b = Bp + 4 * ks * LTP;
-        D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[0], D0, 0, 0, 0);
-        D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ks], b[16], D1, 0, 0, 0);
-      }
+      for (int ks = 0; ks < 4; ks++) a[ks] = fragment(cn, ks);
     }
+#pragma unroll
+    for (int ks = 4; ks < KC / 4; ks++) step(ks, cn);
+    D0 += S0;
+    D1 += S1;
     __syncthreads();  // the tile is free for the next chunk
   }
-  // results: row 16 wave + lane/16 + 4 v of the tile, line 16 h + lane % 16
-  {
-    double *o = sm + (16 * wave + (lane >> 4)) * LTP + (lane & 15);
+  // results: row 16 (wave >> 1) + lane / 16 + 4 v of the tile, line 16 h +
+  // lane % 16
+  if constexpr (CONTIG) {
+    double *o = sm + (p * LT + (lane & 15)) * KP + 16 * (wave >> 1) + (lane >> 4);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      o[4 * v * LTP] = D0[v];
-      o[4 * v * LTP + 16] = D1[v];
+      o[4 * v] = D0[v];
+      o[4 * v + 16 * KP] = D1[v];
+    }
+    __syncthreads();
+    // pairs 32 rt + lane % 32 of lines 2 wave + lane / 32 + 8 q
+    const int r = lane & 31, i = 2 * (kGemmRT * rt + r);
+#pragma unroll
+    for (int q = 0; q < LT / 8; q++) {
+      const int l = 2 * wave + (lane >> 5) + 8 * q, n = tlen[l];
+      double *dst = out + toff[l] + i;
+      const d2u t = {sm[l * KP + r], sm[(LT + l) * KP + r]};
+      if (i + 1 < n)
+        *reinterpret_cast<d2u *>(dst) = t;
+      else if (i < n)
+        dst[0] = t.x;
+    }
+  } else {
+    const int i0 = 2 * (16 * R + (lane >> 4)) + p;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int l = 16 * h + (lane & 15), n = tlen[l];
+      double *dst = out + toff[l];
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (active && i0 + 8 * v < n) dst[(size_t)(i0 + 8 * v) * es] = (h ? D1 : D0)[v];
     }
   }
-  __syncthreads();
-  const int r = kGemmRT * rt + lane;
-#pragma unroll
-  for (int q = 0; q < QS; q++)
-    if (r < NPP && 2 * r + p < len[q]) dst[q][(size_t)(2 * r) * es] = sm[lane * LTP + 4 * q + wave];
 }
 
 template <bool CONTIG>
-__global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(4)))
     k_lines_gemm(const double *__restrict__ in, double *__restrict__ out, LineMap lm,
                  size_t nlines, int N, int NPP, const double *__restrict__ K) {
   extern __shared__ double sm[];
@@ -3096,14 +3171,14 @@ struct DenseClass {
   const int *n;
   size_t nlines;
   int N, NPP;
-  unsigned bxs, tiles;  // 2 x line tiles; bxs x row tiles
+  unsigned bxs, tiles;  // line tiles; bxs x row tiles
 };
 constexpr int kMaxDenseClasses = 8;
 struct DenseClasses {
   DenseClass c[kMaxDenseClasses];
   int count;
 };
-__global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(4)))
     k_lines_gemm_multi(const double *__restrict__ in, double *__restrict__ out, DenseClasses dc) {
   extern __shared__ double sm[];
   unsigned t = blockIdx.x;
@@ -3116,7 +3191,7 @@ __global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(3)
 }
 
 size_t gemm_shared_bytes() {
-  return 8 * (size_t)kGemmKC * kGemmLTP + kGemmLT * (sizeof(size_t) + sizeof(int));
+  return 8 * 2 * (size_t)kGemmLT * kGemmKP + kGemmLT * (sizeof(size_t) + sizeof(int));
 }
 
 // One transform by direct sums from the Lambda tables a, an, dn (those of a
@@ -3198,7 +3273,7 @@ int run_dense_classes(const DenseItem *items, int count, const double *d_in, dou
     c.nlines = items[i].nlines;
     c.N = (int)dp->N;
     c.NPP = dp->NPP;
-    c.bxs = (unsigned)(2 * ((c.nlines + kGemmLT - 1) / kGemmLT));
+    c.bxs = (unsigned)((c.nlines + kGemmLT - 1) / kGemmLT);
     c.tiles = c.bxs * (unsigned)((dp->NPP + kGemmRT - 1) / kGemmRT);
     total += c.tiles;
   }
@@ -3209,20 +3284,23 @@ int run_dense_classes(const DenseItem *items, int count, const double *d_in, dou
   return 0;
 }
 
+// Lines through the parity blocks K (NPP) of length N on the tiled dense
+// product, one launch for any number of lines.
+static void launch_lines_gemm(Prof *prof, const double *K, int NPP, int N, const double *d_in,
+                              double *d_out, const LineMap &lm, size_t nlines, hipStream_t st) {
+  const dim3 grid((unsigned)((nlines + kGemmLT - 1) / kGemmLT),
+                  (unsigned)((NPP + kGemmRT - 1) / kGemmRT));
+  launch_k(prof, lm.es == 1 ? k_lines_gemm<true> : k_lines_gemm<false>, grid, kGemmNT,
+           gemm_shared_bytes(), st, d_in, d_out, lm, nlines, N, NPP, K);
+}
+
 // Batched lines through a direct plan: dense MFMA products when the plan has
 // them and the batch is large enough, else one row per thread.
 static int launch_direct_lines(const direct_plan_s *dp, const double *d_in, double *d_out,
                                size_t dir, const LineMap &lm, size_t nlines, hipStream_t st) {
   const int N = (int)dp->N;
   if (dense_tiled(dp, dir, nlines)) {
-    const size_t nb = (nlines + kGemmLT - 1) / kGemmLT;
-    const dim3 grid((unsigned)(2 * nb), (unsigned)((dp->NPP + kGemmRT - 1) / kGemmRT));
-    if (lm.es == 1)
-      launch_k(dp->prof, k_lines_gemm<true>, grid, kGemmNT, gemm_shared_bytes(), st, d_in, d_out,
-          lm, nlines, N, dp->NPP, dp->d_K[dir]);
-    else
-      launch_k(dp->prof, k_lines_gemm<false>, grid, kGemmNT, gemm_shared_bytes(), st, d_in, d_out,
-          lm, nlines, N, dp->NPP, dp->d_K[dir]);
+    launch_lines_gemm(dp->prof, dp->d_K[dir], dp->NPP, N, d_in, d_out, lm, nlines, st);
   } else if (dp->d_K[dir] && nlines >= 4) {
     const size_t nb = (nlines + kDenseLT - 1) / kDenseLT;
     if (lm.es == 1)
@@ -3557,6 +3635,19 @@ static bool direct_lines(const fmm_plan_s *p, size_t nlines) {
   return p->N <= (size_t)p->direct_max_n && nlines * p->N <= (size_t)p->direct_line_elems;
 }
 
+// Whether a line call of an FMM plan runs as the tiled dense product on the
+// plan's parity blocks (plans of N <= dense_max_n, plain FP64).  The product
+// costs N / 2 multiply-adds an element against the FMM's fixed cost per line
+// and per call.  Per call, FMM / dense (us, contiguous lines): N = 300 with
+// 64 lines 23.6 / 7.7, 4096 lines 298 / 12.4; 512 with 1024 lines 138 / 9.8;
+// 1024 with 64 lines 25.6 / 15.1, 4096 lines 567 / 52.6; 1500 with 64 lines
+// 27.1 / 21.0, 1024 lines 110 / 33.1; 2048 with 64 lines 24.9 / 26.9, 256
+// lines 53.0 / 30.9, 4096 lines 601 / 177.  Above 2048 the blocks would take
+// more than 17 MB of HBM per direction for gains that end near N = 4096.
+static bool dense_lines(const fmm_plan_s *p, size_t dir, size_t nlines) {
+  return p->d_K[dir] && p->precision == 0 && nlines >= (p->N <= 1536 ? 2 : 128);
+}
+
 int run_lines(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size_t nlines,
               size_t n0, size_t ls0, size_t ls1, size_t es, hipStream_t st) {
   prof_step(p->prof);
@@ -3574,6 +3665,13 @@ int run_lines(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size
     prof_begin(p->prof, K_DIRECT, st);
     launch_direct_one(p->prof, (int)p->N, dir, p->t.a, p->t.an, p->t.dn, d_in, d_out, lm, st,
                       p->direct_band, (unsigned)nlines);
+    prof_end(p->prof, st);
+    L2C_HIP(hipGetLastError(), -1);
+    return 0;
+  }
+  if (dense_lines(p, dir, nlines)) {
+    prof_begin(p->prof, K_DIRECT, st);
+    launch_lines_gemm(p->prof, p->d_K[dir], p->NPP, (int)p->N, d_in, d_out, lm, nlines, st);
     prof_end(p->prof, st);
     L2C_HIP(hipGetLastError(), -1);
     return 0;
@@ -3635,6 +3733,11 @@ static int run_lines_scratch(fmm_plan_s *p, double *scr, const double *d_in, dou
   if (direct_lines(p, nlines)) {  // as l2c_execute_lines_device: no workspace
     launch_direct_one(p->prof, (int)p->N, dir, p->t.a, p->t.an, p->t.dn, d_in, d_out, lm, st,
                       p->direct_band, (unsigned)nlines);
+    L2C_HIP(hipGetLastError(), -1);
+    return 0;
+  }
+  if (dense_lines(p, dir, nlines)) {  // nor here
+    launch_lines_gemm(p->prof, p->d_K[dir], p->NPP, (int)p->N, d_in, d_out, lm, nlines, st);
     L2C_HIP(hipGetLastError(), -1);
     return 0;
   }

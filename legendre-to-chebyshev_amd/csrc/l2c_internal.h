@@ -300,6 +300,12 @@ struct fmm_plan_s {
   // line calls of such plans of at most this many elements (lines x N) take
   // the same direct sums, all lines in one launch; L2C_DIRECT_LINES
   int direct_line_elems = 16384;
+  // line calls of plans of N up to this (and up to direct_max_n) run as the
+  // tiled dense product on parity blocks d_K (as a direct plan's), built at
+  // plan creation; 0: always the FMM; L2C_DENSE_MAXN
+  int dense_max_n = 2048;
+  double *d_K[2] = {nullptr, nullptr};
+  int NPP = 0;
   // M2L of the blocks below the top levels from At (rows in registers, no
   // LDS staging: k_m2l_t) for the VALU M2L; L2C_M2L_T=0: k_m2l from A
   bool m2l_t = true;

@@ -454,6 +454,21 @@ static int build_lambda_tables(size_t N, bool c2l, double **a, double **an, doub
   return 0;
 }
 
+// The dense parity blocks of length N for the planned directions, from the
+// Lambda tables: K[d] 2 x NPP x NPP, filled on st.  Returns 0 or -1; K[d] set
+// so far stays with the caller.
+static int build_dense(size_t N, size_t direction, const double *a, const double *an,
+                       const double *dn, double *K[2], int *NPP, hipStream_t st, size_t *acct) {
+  *NPP = (int)(((N + 1) / 2 + 15) / 16 * 16);
+  for (int d = 0; d < 2; d++) {
+    if (direction != BOTH && direction != (size_t)d) continue;
+    if (dmalloc(&K[d], 2 * (size_t)*NPP * *NPP, acct)) return -1;
+    k_build_dense<<<dim3(*NPP, 2), 64, 0, st>>>(K[d], a, an, dn, (int)N, *NPP, d);
+    L2C_HIP(hipGetLastError(), -1);
+  }
+  return 0;
+}
+
 direct_plan_s *make_direct(size_t N, size_t direction, size_t precompute) {
   direct_plan_s *dp = new direct_plan_s();
   dp->N = N;
@@ -475,21 +490,13 @@ direct_plan_s *make_direct(size_t N, size_t direction, size_t precompute) {
     destroy_direct(dp);
     return nullptr;
   }
-  if (N <= (size_t)kGemmMaxN) {
-    dp->NPP = (int)(((N + 1) / 2 + 15) / 16 * 16);
-    const size_t nk = 2 * (size_t)dp->NPP * dp->NPP;
-    for (int d = 0; d < 2; d++) {
-      if ((d == L2C && direction == C2L) || (d == C2L && !c2l)) continue;
-      if (dmalloc(&dp->d_K[d], nk, nullptr)) {
-        destroy_direct(dp);
-        return nullptr;
-      }
-      k_build_dense<<<dim3(dp->NPP, 2), 64, 0, dp->stream>>>(dp->d_K[d], dp->d_a, dp->d_an,
-                                                             dp->d_dn, (int)N, dp->NPP, d);
-      L2C_HIP(hipGetLastError(), (destroy_direct(dp), nullptr));
-    }
-    L2C_HIP(hipStreamSynchronize(dp->stream), (destroy_direct(dp), nullptr));
+  if (N <= (size_t)kGemmMaxN &&
+      build_dense(N, direction, dp->d_a, dp->d_an, dp->d_dn, dp->d_K, &dp->NPP, dp->stream,
+                  nullptr)) {
+    destroy_direct(dp);
+    return nullptr;
   }
+  L2C_HIP(hipStreamSynchronize(dp->stream), (destroy_direct(dp), nullptr));
   return dp;
 }
 
@@ -533,6 +540,8 @@ static void destroy_fmm(fmm_plan_s *p) {
   dfree(p->t.Q);
   dfree(p->t.head[0]);
   dfree(p->t.head[1]);
+  dfree(p->d_K[0]);
+  dfree(p->d_K[1]);
   dfree(p->d_w);
   dfree(p->d_wl);
   for (double *r : p->wl_retired) dfree(r);
@@ -618,6 +627,7 @@ fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, s
   if (const char *e = getenv("L2C_DIRECT_MAXN")) p->direct_max_n = std::max(0, atoi(e));
   if (const char *e = getenv("L2C_DIRECT_BAND")) p->direct_band = atoi(e) != 0;
   if (const char *e = getenv("L2C_DIRECT_LINES")) p->direct_line_elems = std::max(0, atoi(e));
+  if (const char *e = getenv("L2C_DENSE_MAXN")) p->dense_max_n = std::max(0, atoi(e));
   if (const char *e = getenv("L2C_M2L_T")) p->m2l_t = atoi(e) != 0;
   (void)hipGetDevice(&p->device);
   if (hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -683,6 +693,11 @@ fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, s
   const bool l2c = direction == L2C || direction == BOTH;
   const bool c2l = direction == C2L || direction == BOTH;
   if (build_lambda_tables(N, c2l, &p->t.a, &p->t.an, &p->t.dn, st, acct)) {
+    destroy_fmm(p);
+    return nullptr;
+  }
+  if (N <= (size_t)p->dense_max_n && N <= (size_t)p->direct_max_n &&
+      build_dense(N, direction, p->t.a, p->t.an, p->t.dn, p->d_K, &p->NPP, st, acct)) {
     destroy_fmm(p);
     return nullptr;
   }
