@@ -2775,195 +2775,227 @@ __device__ __forceinline__ d2 load_pair(__amdgpu_buffer_rsrc_t r, int voff, int 
   return __builtin_bit_cast(d2, v);
 }
 
+__device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int voff) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
+}
+
 // Batched lines of the direct path (N <= kDenseMaxN) as dense products on FP64
 // MFMA: per parity p, OUT_p (NPP x LT) = K_p (NPP x NPP) IN_p (NPP x LT) for a
 // tile of LT lines, K_p upper triangular (the direct sums of
 // src/C/leg2cheb.c:152-234 with scaling and C2L weights folded in).
 //
-// The two parities run one after the other through one LDS tile [c][line]
-// (row stride kDenseLTP: 36 KB at NPP = 128) and the kernel fits 128 VGPRs,
-// so four work-groups share a CU and one's loads overlap another's products.
-// v_mfma_f64_16x16x4f64 with A =
-// K_p from global memory (the plan's table, L2-resident, in fragment order,
-// streamed kDenseKG k-steps ahead) and B = the input rows from LDS.  Wave w
-// owns row tiles w and NR-1-w, so every wave runs the same number of k-steps;
-// results go back through the LDS tile so that the stores keep the loads'
-// coalescing.
-//
-// CONTIG (lines with unit element stride): lanes run along element pairs
-// (2c, 2c+1), loaded and stored as one 16-byte access; the odd parity's
-// inputs wait in registers during the even parity's products, and the even
-// parity's outputs wait in registers during the odd one's.  Strided lines
-// (lanes along the lines) load and store one parity at a time.
-constexpr int kDenseLT = 32, kDenseLTP = 36, kDenseNT = 256, kDenseKG = 4;
-template <bool CONTIG>
-__global__ void __launch_bounds__(kDenseNT) __attribute__((amdgpu_waves_per_eu(4)))
+// A work-group holds whole lines in LDS [parity][line][c] and every row tile
+// of their outputs, so each element is read and written once, and K (NPP <=
+// 16 NRM) stays in registers: a wave has a parity and the row tiles w and
+// NR-1-w, so that every wave runs the same 4 (NR + 1) k-steps of
+// v_mfma_f64_16x16x4f64.  The work-groups stay and walk the line tiles, the
+// next tile's inputs in flight in registers during the current one's
+// products: HBM-bound.  Row stride 16 NRM + 2 doubles: the writes of contiguous
+// lines and the operand reads fall in distinct banks.
+//   CONTIG (unit element stride): both parities (NP = 2) of a column move as
+//   one 16-byte access, through buffer descriptors of the lines' lengths
+//   (reads past the end return zero, writes past it are dropped).
+//   Strided lines move 32 lines of one element per half-wave, and their
+//   results leave the accumulators as they are (16 lines of one element per
+//   store); wide lines then take one parity per work-group (NP = 1), which
+//   costs them nothing and leaves three work-groups, out of step with each
+//   other, to a CU.
+// 65,536 lines, contiguous / strided (us): N = 256 57.5 / 57.7 (4.7 TB/s of
+// the 4.9 that a large copy reaches), 160 37.7 / 38.9, 128 24.7 / 24.8 (5.4
+// TB/s), 64 17.1 / 13.5; before, one parity after the other through one tile
+// with K from L2 for each of them, 83.8 / 71.6, 55.1 / 48.2, 45.6 / 40.8,
+// 29.2 / 23.8.  Not staying on the CU (512 threads, K from L2): N = 256
+// strided 85.3; staying with both parities of 32 strided lines in one
+// work-group of eight waves per CU: 82.6 (its loads, products and stores take
+// turns).
+template <bool CONTIG, int NRM, int LT, int NP>
+__global__ void __launch_bounds__(32 * NRM * NP)
+    __attribute__((amdgpu_waves_per_eu(CONTIG && NRM == 8 ? 4 : 3)))
     k_lines_dense(const double *__restrict__ in, double *__restrict__ out, LineMap lm,
                   size_t nlines, int N, int NPP, const double *__restrict__ K) {
   extern __shared__ double sm[];
+  constexpr int NW = NRM / 2 * NP, NH = LT / 16;  // waves, 16-line halves
+  static_assert(CONTIG ? NP == 2 : LT == 32, "line moves below");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const size_t l0 = (size_t)blockIdx.x * kDenseLT;
-  const int LTP = kDenseLTP;
-  constexpr bool contig = CONTIG;
-  // start and length of the tile's lines, computed once (line_off divides)
-  size_t *toff = (size_t *)(sm + NPP * LTP);
-  int *tlen = (int *)(toff + kDenseLT);
-  if (tid < kDenseLT) {
-    const size_t line = l0 + tid;
-    toff[tid] = line < nlines ? line_off(lm, line) : 0;
-    tlen[tid] = line < nlines ? line_len(lm, line, N) : 0;
+  const size_t es = CONTIG ? 1 : lm.es;
+  constexpr int KP = 16 * NRM + 2;
+  // work items: line tiles, per parity when NP = 1
+  const unsigned nitem = (unsigned)((nlines + LT - 1) / LT) * (3 - NP);
+  // NP = 1: the grid is even, so a work-group keeps its parity
+  const int p = NP == 2 ? wave & 1 : blockIdx.x & 1;
+  // start and length of an item's lines (line_off divides), of this item, the
+  // next and the one after
+  size_t *toff = (size_t *)(sm + NP * LT * KP);
+  int *tlen = (int *)(toff + 3 * LT);
+  auto offsets = [&](unsigned t, int slot) {
+    if (tid >= LT || t >= nitem) return;
+    const size_t line = (size_t)(NP == 2 ? t : t >> 1) * LT + tid;
+    toff[slot * LT + tid] = line < nlines ? line_off(lm, line) : 0;
+    tlen[slot * LT + tid] = line < nlines ? line_len(lm, line, N) : 0;
+  };
+  unsigned item = blockIdx.x;
+  offsets(item, 0);
+  offsets(item + gridDim.x, 1);
+  const int NR = NPP >> 4, nkt = NPP >> 2;
+  // row tiles R0 and R1 of NRM; groups of four k-steps (one 16-column tile):
+  // NRM - R0 of R0, then NRM - R1 of R1, columns from the diagonal on.  Tiles
+  // past NR read as zero.
+  const int R0 = NP == 2 ? wave >> 1 : wave, R1 = NRM - 1 - R0;
+  constexpr int NG = NRM + 1;
+  double a[NG][4];
+  const __amdgpu_buffer_rsrc_t Kr = line_rsrc(K + (size_t)p * NR * nkt * 64, NR * nkt * 64);
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    const int row = g < NRM - R0 ? R0 : R1, col = g < NRM - R0 ? R0 + g : R1 + g - (NRM - R0);
+    const int base = col < NR ? row * nkt + 4 * col : NR * nkt;
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) a[g][kk] = load_one(Kr, 8 * lane + 512 * kk, base * 512);
   }
+  // moves of a thread: CONTIG line wave + NW (q / QH), pair lane + 64 (q %
+  // QH); else column c0 + cs q (and the half-wave's own parity when NP = 2)
+  // of line lane % 32
+  constexpr int QH = NRM == 8 ? 2 : 1, QL = LT / NW * QH;
+  constexpr int NE = CONTIG ? 2 * QL : 16;
+  const int c0 = NP == 2 ? wave : 2 * wave + (lane >> 5);
+  constexpr int cs = NP == 2 ? NW : 2 * NW;
+  const int i0 = 2 * c0 + (NP == 2 ? lane >> 5 : p);
+  double e[NE];
+  // buffer descriptor of line l of an item
+  auto rsrc = [&](const double *base, int slot, int l) {
+    const size_t o = toff[slot * LT + l];
+    const size_t ou = (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)o) |
+                      ((size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(o >> 32)) << 32);
+    return line_rsrc(base + ou, __builtin_amdgcn_readfirstlane(tlen[slot * LT + l]));
+  };
+  auto fetch = [&](int slot) {
+    if constexpr (CONTIG) {
+#pragma unroll
+      for (int q = 0; q < QL; q++) {
+        const d2 t = load_pair(rsrc(in, slot, wave + NW * (q / QH)), 16 * lane + 1024 * (q % QH), 0);
+        e[2 * q] = t.x;
+        e[2 * q + 1] = t.y;
+      }
+    } else {
+      // (a line past nlines reads line 0 and stores nothing).  One running
+      // address: the empty asm keeps the compiler from holding all sixteen
+      // steps through the item loop.
+      const double *line = in + toff[slot * LT + (lane & 31)], *src = line + (size_t)i0 * es;
+      size_t step = 2 * cs * es;
+      asm volatile("" : "+s"(step));
+      if (N == 32 * NRM) {
+#pragma unroll
+        for (int q = 0; q < NE; q++, src += step) e[q] = *src;
+      } else {
+#pragma unroll
+        for (int q = 0; q < NE; q++, src += step) {
+          const bool ok = i0 + 2 * cs * q < N;
+          const double v = *(ok ? src : line);
+          e[q] = ok ? v : 0.0;
+        }
+      }
+    }
+  };
+  auto stage = [&]() {
+    if constexpr (CONTIG) {
+#pragma unroll
+      for (int q = 0; q < QL; q++) {
+        const int l = wave + NW * (q / QH), c = lane + 64 * (q % QH);
+        if (64 * QH <= 16 * NRM || c < 16 * NRM) {
+          sm[l * KP + c] = e[2 * q];
+          sm[(LT + l) * KP + c] = e[2 * q + 1];
+        }
+      }
+    } else {
+      double *o = sm + ((NP == 2 ? lane >> 5 : 0) * LT + (lane & 31)) * KP + c0;
+#pragma unroll
+      for (int q = 0; q < NE; q++)
+        o[cs * q] = e[q];
+    }
+  };
   __syncthreads();
-  // element q < 16 of this thread in one parity's tile (c < NPP <= 128, 32
-  // lines): lanes run along c when the lines are contiguous, along the lines
-  // (two rows c per wave) otherwise, so neighbouring lanes touch neighbouring
-  // words of one parity
-  auto tile_c = [&](int q) { return contig ? lane + 64 * (q & 1) : 2 * wave + (lane >> 5) + 8 * q; };
-  auto tile_l = [&](int q) { return contig ? wave + 4 * (q >> 1) : (lane & 31); };
-  // strided lines: one line per thread, rows c0 + 8 q, so one base address
-  // and a constant step (16 elements) serve all 16 elements
-  const int c0 = 2 * wave + (lane >> 5), ls = lane & 31;
-  auto load = [&](int p, double *vt) {
-    const double *src = in + toff[ls] + (size_t)(2 * c0 + p) * lm.es;
-    const size_t step = 16 * lm.es;
-    const int len = tlen[ls];
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int c = c0 + 8 * q;
-      vt[q] = c < NPP && 2 * c + p < len ? src[q * step] : 0.0;
-    }
-  };
-  const int NR = NPP >> 4, npair = (NR + 1) >> 1;
-  const bool active = wave < npair;
-  const int R0 = wave, R1 = NR - 1 - wave;
-  const bool two = active && R1 != R0;
-  const int nk0 = active ? (NPP - 16 * R0) >> 2 : 0, nk1 = two ? (NPP - 16 * R1) >> 2 : 0;
-  const double *Bp = sm + (lane >> 4) * LTP + (lane & 15);
-  // contiguous lines: element pair (2c, 2c+1) of a line as one 16-byte
-  // access when it is aligned and whole, else two guarded words
-  auto pair_at = [&](int q, double &e0, double &e1) {
-    const int c = tile_c(q), l = tile_l(q), len = tlen[l];
-    const size_t a = toff[l] + 2 * (size_t)c;
-    e0 = e1 = 0.0;
-    if (c >= NPP) return;
-    if (2 * c + 1 < len && !(a & 1)) {
-      const double2 t = *reinterpret_cast<const double2 *>(in + a);
-      e0 = t.x;
-      e1 = t.y;
-    } else {
-      if (2 * c < len) e0 = in[a];
-      if (2 * c + 1 < len) e1 = in[a + 1];
-    }
-  };
-  double vt[16], hold[16];
-  if (CONTIG) {
-#pragma unroll
-    for (int q = 0; q < 16; q++) pair_at(q, hold[q], vt[q]);  // hold: parity 0 for now
-  } else {
-    load(0, vt);
-  }
-  for (int p = 0; p < 2; p++) {
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int c = tile_c(q);
-      if (c < NPP) sm[c * LTP + tile_l(q)] = CONTIG && p == 0 ? hold[q] : vt[q];
-    }
+  fetch(0);
+  stage();
+  const d4 z = {0.0, 0.0, 0.0, 0.0};
+  double *const mine = sm + ((NP == 2 ? p * LT : 0) + (lane & 15)) * KP + (lane >> 4);
+  for (int slot = 0; item < nitem; item += gridDim.x) {
+    const int nslot = slot == 2 ? 0 : slot + 1;
+    const bool more = item + gridDim.x < nitem;
     __syncthreads();
-    d4 D00 = {0.0, 0.0, 0.0, 0.0}, D01 = D00, D10 = D00, D11 = D00;
-    if (active) {
-      // A fragments of row tile R from its diagonal k-step on: 64 doubles each
-      const double *K0 = K + (((size_t)p * NR + R0) * (NPP >> 2) + 4 * R0) * 64 + lane;
-      const double *K1 = K + (((size_t)p * NR + R1) * (NPP >> 2) + 4 * R1) * 64 + lane;
-      constexpr int G = kDenseKG, NG = 32 / G;  // nk0 <= 32, nk1 <= 16
-      double a0[2][G], a1[2][G];
+    if (more) fetch(nslot);
+    offsets(item + 2 * gridDim.x, nslot == 2 ? 0 : nslot + 1);
+    d4 D[2][NH];  // [row tile][16-line half]
+    auto products = [&](auto r0) {
+      constexpr int r = decltype(r0)::value;
 #pragma unroll
-      for (int kk = 0; kk < G; kk++) {
-        a0[0][kk] = kk < nk0 ? K0[64 * kk] : 0.0;
-        a1[0][kk] = kk < nk1 ? K1[64 * kk] : 0.0;
-      }
+      for (int h = 0; h < NH; h++) D[0][h] = D[1][h] = z;
 #pragma unroll
-      for (int gi = 0; gi < NG; gi++) {
-        const int cur = gi & 1;
-        if (gi + 1 < NG) {
+      for (int g = 0; g < NG; g++) {
+        constexpr int n0 = NRM - r;
+        const int col = g < n0 ? r + g : NRM - 1 - r + g - n0;
+        if (col >= NR) continue;
+        const double *b = mine + 16 * col;
 #pragma unroll
-          for (int kk = 0; kk < G; kk++) {
-            const int k = G * (gi + 1) + kk;
-            a0[cur ^ 1][kk] = k < nk0 ? K0[64 * k] : 0.0;
-            if (k < 16) a1[cur ^ 1][kk] = k < nk1 ? K1[64 * k] : 0.0;
+        for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+          for (int h = 0; h < NH; h++) {
+            d4 &d = D[g < n0 ? 0 : 1][h];
+            d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[g][kk], b[16 * h * KP + 4 * kk], d, 0, 0, 0);
           }
-        }
-#pragma unroll
-        for (int kk = 0; kk < G; kk++) {
-          const int k = G * gi + kk;
-          if (k < nk0) {
-            const double *b = Bp + (16 * R0 + 4 * k) * LTP;
-            D00 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[cur][kk], b[0], D00, 0, 0, 0);
-            D01 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[cur][kk], b[16], D01, 0, 0, 0);
-          }
-          if (k < 16 && k < nk1) {
-            const double *b = Bp + (16 * R1 + 4 * k) * LTP;
-            D10 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[cur][kk], b[0], D10, 0, 0, 0);
-            D11 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[cur][kk], b[16], D11, 0, 0, 0);
-          }
-        }
       }
-    }
-    __syncthreads();  // every wave is done with the input tile
-    if (active) {
-      double *o = sm + (16 * R0 + (lane >> 4)) * LTP + (lane & 15);
+    };
+    constexpr int top = NRM / 2 - 1;  // (waves have R0 <= top)
+    if (R0 == 0)
+      products(std::integral_constant<int, 0>{});
+    else if (R0 == 1)
+      products(std::integral_constant<int, std::min(1, top)>{});
+    else if (R0 == 2)
+      products(std::integral_constant<int, std::min(2, top)>{});
+    else
+      products(std::integral_constant<int, top>{});
+    if constexpr (CONTIG) {
+      __syncthreads();  // every wave is done with the input tile
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        o[4 * v * LTP] = D00[v];
-        o[4 * v * LTP + 16] = D01[v];
+      for (int j = 0; j < 2; j++) {
+        double *o = mine + 16 * (j ? R1 : R0);
+#pragma unroll
+        for (int h = 0; h < NH; h++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) o[16 * h * KP + 4 * v] = D[j][h][v];
       }
-      if (two) {
-        o = sm + (16 * R1 + (lane >> 4)) * LTP + (lane & 15);
+      __syncthreads();
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          o[4 * v * LTP] = D10[v];
-          o[4 * v * LTP + 16] = D11[v];
-        }
-      }
-    }
-    __syncthreads();
-    if (CONTIG) {
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int c = tile_c(q), l = tile_l(q);
-        const double v = c < NPP ? sm[c * LTP + l] : 0.0;
-        if (p == 0) {
-          hold[q] = v;  // even outputs, stored with the odd ones
-          continue;
-        }
-        const int len = tlen[l];
-        const size_t a = toff[l] + 2 * (size_t)c;
-        if (c >= NPP || 2 * c >= len) continue;
-        if (2 * c + 1 < len && !(a & 1)) {
-          *reinterpret_cast<double2 *>(out + a) = make_double2(hold[q], v);
-        } else {
-          out[a] = hold[q];
-          if (2 * c + 1 < len) out[a + 1] = v;
-        }
+      for (int q = 0; q < QL; q++) {
+        const int l = wave + NW * (q / QH), c = std::min(lane + 64 * (q % QH), 16 * NRM - 1);
+        const d2 t = {sm[l * KP + c], sm[(LT + l) * KP + c]};
+        store_pair(t, rsrc(out, slot, l), 16 * lane + 1024 * (q % QH));
       }
     } else {
-      double *dst = out + toff[ls] + (size_t)(2 * c0 + p) * lm.es;
-      const size_t step = 16 * lm.es;
-      const int len = tlen[ls];
 #pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int c = c0 + 8 * q;
-        if (c < NPP && 2 * c + p < len) dst[q * step] = sm[c * LTP + ls];
+      for (int h = 0; h < NH; h++) {
+        const int l = 16 * h + (lane & 15), len = tlen[slot * LT + l];
+        size_t step = 8 * es;
+        asm volatile("" : "+s"(step));
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          const int r0 = 2 * (16 * (j ? R1 : R0) + (lane >> 4)) + p;
+          double *dst = out + toff[slot * LT + l] + (size_t)r0 * es;
+#pragma unroll
+          for (int v = 0; v < 4; v++, dst += step)
+            if (r0 + 8 * v < len) *dst = D[j][h][v];
+        }
       }
     }
-    __syncthreads();  // the tile is free for the next parity
-    if (!CONTIG && p == 0) load(1, vt);
+    __syncthreads();  // the tile is free for the next one
+    if (more) stage();
+    slot = nslot;
   }
 }
 
-// the tile [NPP][LTP], then the lines' offsets (size_t) and lengths (int)
-static size_t dense_shared_bytes(int NPP) {
-  return 8 * (size_t)NPP * kDenseLTP + kDenseLT * (sizeof(size_t) + sizeof(int));
+// the tile [NP][LT][16 NRM + 2], then three items' offsets (size_t) and
+// lengths (int)
+static size_t dense_shared_bytes(int NRM, int LT, int NP) {
+  return 8 * (size_t)NP * LT * (16 * NRM + 2) + 3 * LT * (sizeof(size_t) + sizeof(int));
 }
 
 // Batched lines of the direct path with kDenseMaxN < N <= kGemmMaxN: the same
@@ -2993,7 +3025,7 @@ static size_t dense_shared_bytes(int NPP) {
 // 27.  Splitting a tile's columns over two or four groups of waves: 4 lines of
 // 2048 26 -> 24 us, but 1024 lines of 1024 19.4 -> 20.5 and 25.5.
 constexpr int kGemmRT = 32, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmKP = kGemmKC + 2;
-constexpr size_t kGemmFewLines = 16384;
+constexpr size_t kGemmFewLines = 4096;
 // The work of tile (bx, by) of the tiled dense product (grid (line tiles,
 // row tiles)); k_lines_gemm runs one grid of them, k_lines_gemm_multi the
 // grids of several size classes in one launch.
@@ -3243,11 +3275,12 @@ static void launch_direct(const direct_plan_s *dp, const double *d_in, double *d
 }
 
 // Whether a call of nlines lines through direct plan dp takes the tiled dense
-// product (k_lines_gemm): the one-tile kernel has the lower cost per line,
-// the tiled one far more work-groups for a given call, so above N = 32 the
-// tiled kernel takes calls of up to kGemmFewLines lines (N = 256: 600 lines
-// in 7 us against 18 us; 65,536 lines in 119 us against 90 us) unless the
-// plan's dense_tile says otherwise.
+// product (k_lines_gemm): the whole-line kernel has the lower cost per line,
+// the tiled one more work-groups for a given call, so above N = 32 the tiled
+// kernel takes calls of up to kGemmFewLines lines unless the plan's dense_tile
+// says otherwise.  Tiled / whole-line (us, contiguous): N = 256 with 1000
+// lines 6.2 / 7.3, 4096 lines 8.2 / 8.5 (strided 8.7 / 7.7), 16,384 lines 25.3
+// / 20.4; N = 128 with 4096 lines 5.1 / 5.5, 16,384 lines 11.2 / 9.7.
 bool dense_tiled(const direct_plan_s *dp, size_t dir, size_t nlines) {
   const int N = (int)dp->N;
   return dp->d_K[dir] && nlines >= 4 &&
@@ -3294,6 +3327,25 @@ static void launch_lines_gemm(Prof *prof, const double *K, int NPP, int N, const
            gemm_shared_bytes(), st, d_in, d_out, lm, nlines, N, NPP, K);
 }
 
+// The same on the kernel that holds whole lines (N <= kDenseMaxN).
+static void launch_lines_dense(Prof *prof, const double *K, int NPP, int N, const double *d_in,
+                               double *d_out, const LineMap &lm, size_t nlines, hipStream_t st) {
+  // per_cu: the work-groups that a CU's registers and LDS hold, times 256 CUs
+  auto go = [&](auto kern, int NRM, int LT, int NP, int per_cu) {
+    const size_t items = (nlines + LT - 1) / LT * (3 - NP);
+    launch_k(prof, kern, dim3((unsigned)std::min<size_t>(items, 256 * per_cu)), 32 * NRM * NP,
+             dense_shared_bytes(NRM, LT, NP), st, d_in, d_out, lm, nlines, N, NPP, K);
+  };
+  if (lm.es == 1)
+    NPP > 64   ? go(k_lines_dense<true, 8, 16, 2>, 8, 16, 2, 2)
+    : NPP > 32 ? go(k_lines_dense<true, 4, 32, 2>, 4, 32, 2, 3)
+               : go(k_lines_dense<true, 2, 16, 2>, 2, 16, 2, 8);
+  else
+    NPP > 64   ? go(k_lines_dense<false, 8, 32, 1>, 8, 32, 1, 3)
+    : NPP > 32 ? go(k_lines_dense<false, 4, 32, 2>, 4, 32, 2, 3)
+               : go(k_lines_dense<false, 2, 32, 2>, 2, 32, 2, 6);
+}
+
 // Batched lines through a direct plan: dense MFMA products when the plan has
 // them and the batch is large enough, else one row per thread.
 static int launch_direct_lines(const direct_plan_s *dp, const double *d_in, double *d_out,
@@ -3302,13 +3354,7 @@ static int launch_direct_lines(const direct_plan_s *dp, const double *d_in, doub
   if (dense_tiled(dp, dir, nlines)) {
     launch_lines_gemm(dp->prof, dp->d_K[dir], dp->NPP, N, d_in, d_out, lm, nlines, st);
   } else if (dp->d_K[dir] && nlines >= 4) {
-    const size_t nb = (nlines + kDenseLT - 1) / kDenseLT;
-    if (lm.es == 1)
-      launch_k(dp->prof, k_lines_dense<true>, dim3((unsigned)nb), kDenseNT,
-          dense_shared_bytes(dp->NPP), st, d_in, d_out, lm, nlines, N, dp->NPP, dp->d_K[dir]);
-    else
-      launch_k(dp->prof, k_lines_dense<false>, dim3((unsigned)nb), kDenseNT,
-          dense_shared_bytes(dp->NPP), st, d_in, d_out, lm, nlines, N, dp->NPP, dp->d_K[dir]);
+    launch_lines_dense(dp->prof, dp->d_K[dir], dp->NPP, N, d_in, d_out, lm, nlines, st);
   } else {
     launch_direct(dp, d_in, d_out, dir, lm, nlines, st);
   }

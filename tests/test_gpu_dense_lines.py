@@ -1,5 +1,7 @@
-"""Line calls of FMM plans of N <= 2048 as the tiled dense product on FP64 MFMA
-(k_lines_gemm).  Sampled lines against the oracle, tolerance 1e-14 log2 N per line as in the other line
+"""Line calls as dense products on FP64 MFMA: k_lines_dense (direct plans of
+N <= 256, more than 4,096 lines, or N <= 32) and k_lines_gemm (longer lines
+and smaller calls, and the line calls of FMM plans of N <= 2048).  Sampled
+lines against the oracle, tolerance 1e-14 log2 N per line as in the other line
 tests."""
 import math
 
@@ -44,6 +46,32 @@ def check(orc, x, y, direction, maxs, rows):
     op = orc.FMMPlan(N, maxs, 18, orc.BOTH)
     for r in rows:
         assert relerr(y[r], op.execute(np.ascontiguousarray(x[r]), direction)) <= tol(N), (r, direction)
+
+
+# row tiles 1, 2 | 3, 4 | 5 .. 8 of the three widths, full and partly empty,
+# odd lengths; 4,097 lines: past the tiled product's share, one line in the
+# last tile; 70 lines: fewer tiles than the GPU holds
+@pytest.mark.parametrize("N", [2, 15, 31, 32, 33, 63, 64, 65, 97, 128, 129, 191, 225, 255, 256])
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_whole_lines(amd, orc, N, strided, direction):
+    B = 70 if N <= 32 else 4097
+    announce(f"whole lines N={N} B={B} strided={strided} dir={direction}")
+    x = np.random.default_rng(N).uniform(-1, 1, (B, N))
+    plan = amd.FMMPlan(N, 64, 18, direction)
+    y = run_lines(amd, plan, x, direction, strided, pad=3)
+    check(orc, x, y, direction, 64, [0, 15, 16, 31, 32, B // 2, B - 2, B - 1])
+
+
+def test_whole_lines_many_tiles(amd, orc):
+    """60,001 lines: every work-group walks several tiles, some one more than
+    others, the last tile holds one line."""
+    for N, strided in ((256, False), (256, True), (100, False), (100, True), (40, True)):
+        announce(f"whole lines N={N} B=60001 strided={strided}")
+        x = np.random.default_rng(N).uniform(-1, 1, (60001, N))
+        plan = amd.FMMPlan(N, 64, 18, 0)
+        y = run_lines(amd, plan, x, 0, strided)
+        check(orc, x, y, 0, 64, [0, 1, 31, 32, 24575, 24576, 49151, 49152, 59999, 60000])
 
 
 @pytest.mark.parametrize("N,B", [(257, 2), (500, 33), (769, 40), (1000, 65), (1536, 17),
