@@ -3024,6 +3024,10 @@ static size_t dense_shared_bytes(int NRM, int LT, int NP) {
 // 1024 24.0 -> 19.4 us, 4096 lines of 2048 212 -> 177, 32 lines of 2048 35 ->
 // 27.  Splitting a tile's columns over two or four groups of waves: 4 lines of
 // 2048 26 -> 24 us, but 1024 lines of 1024 19.4 -> 20.5 and 25.5.
+// Chunks from the last to the diagonal's instead of upwards: a 1200 x 900 array
+// through both axes and back 111 -> 96 us (the prefetch behind the last chunk
+// falls on lines just read), 2-norm error at N = 2000 3.2-4.6e-16 ->
+// 1.7-2.8e-16 (the FMM of the same lines 2.3-7.3e-16).
 constexpr int kGemmRT = 32, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmKP = kGemmKC + 2;
 constexpr size_t kGemmFewLines = 4096;
 // The work of tile (bx, by) of the tiled dense product (grid (line tiles,
@@ -3052,9 +3056,11 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
   const bool active = R < NR;  // the last row tile may be partly past NPP
   const size_t es = CONTIG ? 1 : lm.es;
   const d4 z = {0.0, 0.0, 0.0, 0.0};
-  // sums of the two 16-line halves: each chunk's own, added to the total (one
-  // long chain over up to 1024 columns would lose a digit: 2-norm error
-  // against double-double sums at N = 2000 1.3-1.8e-15 in one chain)
+  // sums of the two 16-line halves: each chunk's own, added to the total, from
+  // the last column to the diagonal (K falls off away from it, so the large
+  // terms come last; one long chain over up to 1024 columns would lose a digit:
+  // 2-norm error against double-double sums at N = 2000 1.3-1.8e-15 in one
+  // chain)
   d4 D0 = z, D1 = z;
   const double *Bp = sm + (p * LT + (lane & 15)) * KP + (lane >> 4);
   // the fragments of row tile R (zeros past NPP, and for a row tile past it)
@@ -3105,9 +3111,10 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     }
   };
   auto fragment = [&](int c0, int ks) { return load_one(Kr, 8 * lane + 512 * (ks & 7), 128 * c0 + 512 * (ks & 8)); };
-  fetch_in(kGemmRT * rt);
+  const int cf = kGemmRT * rt, cl = cf + (NPP - 1 - cf) / KC * KC;  // first and last chunk
+  fetch_in(cl);
 #pragma unroll
-  for (int ks = 0; ks < KC / 4; ks++) a[ks] = fragment(kGemmRT * rt, ks);
+  for (int ks = 0; ks < KC / 4; ks++) a[ks] = fragment(cl, ks);
   // one k-step: its products, then the same step's fragment of chunk cn
   d4 S0, S1;
   auto step = [&](int ks, int cn) {
@@ -3118,7 +3125,7 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     // (the scheduler would gather the loads and hold both chunks' fragments)
     if (ks & 1) __builtin_amdgcn_sched_barrier(0);
   };
-  for (int c0 = kGemmRT * rt; c0 < NPP; c0 += KC) {
+  for (int c0 = cl; c0 >= cf; c0 -= KC) {
     if constexpr (CONTIG) {
 #pragma unroll
       for (int q = 0; q < QL; q++) {
@@ -3132,20 +3139,17 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     }
     __syncthreads();
     // the next chunk's inputs load during this chunk's products
-    int cn = c0 + KC;
+    int cn = std::max(c0 - KC, cf);
     fetch_in(cn);
     asm volatile("" : "+s"(cn));
     S0 = S1 = z;
+#pragma unroll
+    for (int ks = KC / 4 - 1; ks >= 4; ks--) step(ks, cn);
     // the tile's second row tile starts 16 columns on (K_p is zero before)
-    if (c0 != kGemmRT * rt || wave < 2) {
+    if (c0 != cf || wave < 2) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++) step(ks, cn);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) a[ks] = fragment(cn, ks);
+      for (int ks = 3; ks >= 0; ks--) step(ks, cn);
     }
-#pragma unroll
-    for (int ks = 4; ks < KC / 4; ks++) step(ks, cn);
     D0 += S0;
     D1 += S1;
     __syncthreads();  // the tile is free for the next chunk
