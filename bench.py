@@ -57,9 +57,11 @@ def kernel_bytes(name, info, N):
 
     k_m2l: the M2L matrices (Nc*M^2 doubles), two multipole vectors read and
     two M2L vectors written per block (Nb blocks, 2M doubles each).
-    k_down: input, output, the Lambda table the band reads (a for L2C, an for
-    C2L; the 2s-entry head is negligible) and one M2L vector per chunk slot.
-    k_up: input, one multipole vector per chunk slot.
+    k_up (with the near field): input, the band sums, the Lambda table the
+    band reads (a for L2C, an for C2L; the 2s-entry head is negligible) and
+    one multipole vector per chunk slot.
+    k_down (k_far): the band sums read, the output, one M2L vector per chunk
+    slot.
     k_direct (single transforms of N <= 8192 on an FMM plan): input, output
     and the Lambda table a (C2L reads an and dn, 1.5 N; counted as N).
     """
@@ -68,9 +70,9 @@ def kernel_bytes(name, info, N):
     if name == "k_m2l":
         return 8 * (Nc * M * M + 4 * Nb * 2 * M)
     if name == "k_down":
-        return 8 * (3 * N + slots * 2 * M)
+        return 8 * (2 * N + slots * 2 * M)
     if name == "k_up":
-        return 8 * (N + slots * 2 * M)
+        return 8 * (3 * N + slots * 2 * M)
     if name == "k_direct":
         return 8 * 3 * N
     return 8 * 2 * N
@@ -118,9 +120,9 @@ def _counter_means(csv_dir, counter, copy_kib):
                 if name.startswith("l2c::"):
                     name = name[5:]
                 # profile slots: k_m2l covers k_m2l_t and k_m2l, k_down the
-                # downward kernels (k_down8r, k_down8, k_down)
+                # downward kernels (k_far, k_down8r, k_down8, k_down)
                 for tag, slot in (("k_up", "k_up"), ("k_m2l_t", "k_m2l"), ("k_m2l", "k_m2l"),
-                                  ("k_down8r", "k_down"),
+                                  ("k_far", "k_down"), ("k_down8r", "k_down"),
                                   ("k_down8", "k_down"), ("k_down", "k_down"),
                                   ("k_direct", "k_direct")):
                     if name.startswith(tag + "<") or name.startswith(tag + "(") or name == tag:

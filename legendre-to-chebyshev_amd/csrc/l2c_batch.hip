@@ -39,7 +39,7 @@ struct BatchClass {
   std::vector<size_t> idx;  // transforms of the class, in batch order
   int method = 0;        // 0 direct, 1 FMM
   size_t s = 0, L = 0;   // FMM leaf size and depth
-  // FMM: 0 fused downward kernel, 1 k_band + k_far; direct: 0 the default
+  // FMM: 0 the band in the k_up launch, 1 a k_band launch; direct: 0 the default
   // dense kernel for the line count, 1 the one-tile kernel, 2 the tiled one
   int variant = 0;
   double ms = -1;        // tuner time of the chosen method

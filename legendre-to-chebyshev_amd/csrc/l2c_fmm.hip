@@ -38,6 +38,28 @@ constexpr double k2Pi = 0.63661977236758134307553505349;  // 2/pi
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
+// two doubles at any 8-byte boundary, moved as one 16-byte access
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+// Buffer descriptor of n doubles at p (both wave-uniform): raw buffer loads
+// check each dword against the length and return zero past it.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t line_rsrc(const double *p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 8 * n, 0x00020000);
+}
+__device__ __forceinline__ double load_one(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+}
+// The two doubles at byte voff (per lane) + soff (uniform) of the buffer.
+__device__ __forceinline__ d2 load_pair(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+  return __builtin_bit_cast(d2, v);
+}
+
+__device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int voff) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
+}
+
 struct WsLayout {
   size_t w, part, m2l, total;
 };
@@ -57,6 +79,302 @@ size_t ws_doubles(const Geo &g) { return ws_layout(g).total; }
 __host__ __device__ __forceinline__ int sk4(int c) { return c + (c >> 2); }
 __host__ __device__ __forceinline__ int sk8(int k) { return k + (k >> 3); }
 
+
+// ---------------------------------------------------------------------------
+// The near-field band (src/C/leg2cheb.c:236-535) of 16 leaf chunks, any leaf
+// size s <= 64, by the 256 threads of a work-group: rows r of parity sg take
+// the columns c = r + t, t < len (2 s - 16 gam for row group gam, shorter in
+// the last chunk), y_r = sum H(t - rho) P(2 r0 + sg + t + rho) x(r0 + t).
+// Each lane owns 16 rows of one chunk and parity: lane = chunk + 16 parity +
+// 32 del, row group gam = 2 p + del; waves split (p, columns).  All lanes of a
+// wave sit at the same t, so H is wave-uniform: scalar loads, which the
+// products take as operands; P runs through a ring of 16 registers.  Per
+// column a lane reads one x and one P from LDS for 16 terms (one multiply and
+// one FMA each), four columns ahead.
+//   x, per parity, half index h from the first chunk: h + h / s when 4
+//     divides s (one pad per chunk), else h; parity 1 at +nxs, nxs odd when
+//     s = 2 mod 4, else 16 mod 32
+//   P, entry m from the first row: m + 2 (m / 2s) for even s (every 2s
+//     entries are followed by a copy of the next two), else m
+// so that the 32 lanes of half a wave read distinct banks, and a lane's four
+// entries are always consecutive (it meets a chunk's end only between them,
+// S16: s a multiple of 16, only between trips of 16).
+// Bound by FP64 issue on large calls (4.6 M vector instructions at N = 2^20,
+// s = 64, three quarters of them the products), on one small line by the
+// work-group's own chain (window loads 2 us, its trips 1 us each, staging).
+// As k_band alone, s = 64: 2^16 10.0 us, 2^20 17.3, 64 lines of 2^18 165; with
+// 8 rows a lane, H from LDS and a Lambda window per chunk, s = 16, 32, 64 only,
+// 11.3, 18.6 and 212.
+constexpr int kBandNT = 256, kBandG = 16, kBandMaxS = 64;
+struct BandLds {
+  int nx, pad, nxs, np, pw, PS, CS, total;
+};
+__host__ __device__ inline BandLds band_lds(const Geo &g) {
+  const int s = g.s;
+  BandLds d;
+  d.nx = (kBandG + 1) * s + 32;  // half indices per parity: the last chunk's columns, a trip over
+  d.pad = (s & 3) == 0;
+  const int n = d.nx + (d.pad ? d.nx / s + 1 : 0);
+  d.nxs = (s & 3) == 2 ? n | 1 : n + (48 - n % 32) % 32;
+  d.pw = 2 * d.nxs;
+  d.pw += d.pw & 1;  // 16-byte rows
+  d.np = 2 * kBandG * s + s + 64;
+  d.np += d.np & 1;
+  d.PS = 2 * s + ((s & 1) ? 0 : 2);
+  // staging of the sums, [segment][chunk][CS], over the windows
+  d.CS = d.PS;
+  const int npair = (s + 31) / 32;
+  // (the unused prefetch behind a last trip may pass the windows' ends)
+  d.total = std::max(d.pw + d.np + ((s & 1) ? 0 : 2 * (d.np / (2 * s) + 1)) + 32,
+                     (kBandNT / 64 / npair) * kBandG * d.CS);
+  return d;
+}
+size_t band_shared_bytes(const Geo &g) { return 8 * (size_t)band_lds(g).total; }
+inline unsigned band_groups(const Geo &g) {  // work-groups of one line
+  return (unsigned)((((size_t)2 << g.L) + kBandG - 1) / kBandG);
+}
+
+typedef const __attribute__((address_space(4))) double *kdouble;  // uniform, read-only
+
+// A lane's read pointers into the windows: the next quad of x and of P, and
+// the columns to the next chunk end of each (a pad of px or pp doubles then).
+struct BandPtr {
+  const double *x, *p;
+  int lx, lp;
+};
+constexpr int kBT = 2;  // products in flight before their sums
+// One trip of 16 columns from column tb on; X, P of the trip's first quad are
+// in XA, PA, and on return those of the next trip's.  The trip's 31 values of
+// H are scalar loads (hp: the head, 16 zeros before it).  KIND 0: as it is; 1:
+// columns t >= len read x as zero; 2: that, and the terms left of the diagonal
+// (rho > t) are left out, for the trip from column 0.
+template <int KIND, bool S16>
+__device__ __forceinline__ void band_trip(BandPtr &b, int s1, int s2, kdouble hp, int tb, int len,
+                                          double (&pr)[16], double (&XA)[4], double (&PA)[4],
+                                          double (&acc)[16]) {
+  double XB[4], PB[4], hw[32];
+#pragma unroll
+  for (int k = 1; k < 32; k++) hw[k] = hp[tb - 16 + k];
+  // x of the quad after the current one, P 16 further on
+#define QUAD_FETCH(X, P, Q)                                      \
+  {                                                              \
+    if (!S16 || (Q) == 3) {                                      \
+      b.lx -= S16 ? 16 : 4;                                      \
+      b.lp -= S16 ? 16 : 4;                                      \
+      const bool ox_ = b.lx == 0, op_ = b.lp == 0;               \
+      b.x += ox_ ? 5 : 4;                                        \
+      b.p += op_ ? 6 : 4;                                        \
+      b.lx = ox_ ? s1 : b.lx;                                    \
+      b.lp = op_ ? s2 : b.lp;                                    \
+    } else {                                                     \
+      b.x += 4;                                                  \
+      b.p += 4;                                                  \
+    }                                                            \
+    _Pragma("unroll") for (int k_ = 0; k_ < 4; k_++) {           \
+      X[k_] = b.x[k_];                                           \
+      P[k_] = b.p[k_];                                           \
+    }                                                            \
+  }
+#define QUAD_STEP(X, P, Q)                                                          \
+  _Pragma("unroll") for (int j_ = 0; j_ < 4; j_++) {                                \
+    const int k_ = 4 * (Q) + j_;                                                    \
+    const double x_ = KIND != 0 ? (tb + k_ < len ? X[j_] : 0.0) : X[j_];            \
+    _Pragma("unroll") for (int q_ = 0; q_ < 16 / kBT; q_++) {                       \
+      double t_[kBT];                                                               \
+      _Pragma("unroll") for (int i_ = 0; i_ < kBT; i_++) {                          \
+        const int r_ = kBT * q_ + i_;                                               \
+        t_[i_] = KIND != 2 || r_ <= k_ ? hw[16 + k_ - r_] * pr[(k_ + r_) & 15] : 0.0; \
+      }                                                                             \
+      __builtin_amdgcn_sched_barrier(0);                                            \
+      _Pragma("unroll") for (int i_ = 0; i_ < kBT; i_++) {                          \
+        const int r_ = kBT * q_ + i_;                                               \
+        if (KIND != 2 || r_ <= k_) acc[r_] += t_[i_] * x_;                          \
+      }                                                                             \
+    }                                                                               \
+    pr[k_] = P[j_];                                                                 \
+    __builtin_amdgcn_sched_barrier(0);                                              \
+  }
+  QUAD_FETCH(XB, PB, 0)
+  QUAD_STEP(XA, PA, 0)
+  QUAD_FETCH(XA, PA, 1)
+  QUAD_STEP(XB, PB, 1)
+  QUAD_FETCH(XB, PB, 2)
+  QUAD_STEP(XA, PA, 2)
+  QUAD_FETCH(XA, PA, 3)
+  QUAD_STEP(XB, PB, 3)
+#undef QUAD_STEP
+#undef QUAD_FETCH
+}
+
+// Band group grp of the line at src / dst (element stride es, length Nl): the
+// sums are stored over the output, raw (the C2L diagonal included), or with
+// the final scaling when scale != 0.
+template <bool S16>
+__device__ __forceinline__ void band_group(const double *__restrict__ src,
+                                           double *__restrict__ dst, size_t es, int Nl,
+                                           const Geo &g, int dir, int grp, int scale,
+                                           const double *__restrict__ tab,
+                                           const double *__restrict__ head, double *sm) {
+  const int s = g.s, N = g.N;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const size_t hc0 = (size_t)grp * kBandG * s, row0 = 2 * hc0;
+  if (row0 >= (size_t)Nl) return;  // the whole work-group
+  const BandLds ly = band_lds(g);
+  double *xs = sm, *pw = sm + ly.pw;
+  const unsigned inv = ((1u << 20) + s - 1) / s;  // h / s = h inv >> 20 for h < 2200
+  auto chunk = [&](int h) { return (int)(__umul24(h, inv) >> 20); };
+  const bool even = (s & 1) == 0;
+  // ---- windows: pairs of P, pairs (2 h, 2 h + 1) of x; past the table's and
+  // the line's ends zeros
+  constexpr int QX = 5;  // ceil(nx / 256), ceil(np / 512) for s = 64
+  d2 vp[QX], vx[QX];
+  {
+    const __amdgpu_buffer_rsrc_t r =
+        line_rsrc(tab + row0, (int)std::min<size_t>((size_t)N - row0, ly.np));
+#pragma unroll
+    for (int q = 0; q < QX; q++) vp[q] = load_pair(r, 16 * tid + 4096 * q, 0);
+  }
+  if (es == 1) {
+    const __amdgpu_buffer_rsrc_t r =
+        line_rsrc(src + row0, (int)std::min<size_t>((size_t)Nl - row0, 2 * ly.nx));
+#pragma unroll
+    for (int q = 0; q < QX; q++) vx[q] = load_pair(r, 16 * tid + 4096 * q, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < QX; q++) {
+      const size_t i = row0 + 2 * (size_t)(tid + kBandNT * q);
+      vx[q].x = src[std::min(i, (size_t)Nl - 1) * es];
+      vx[q].y = src[std::min(i + 1, (size_t)Nl - 1) * es];
+      if (i >= (size_t)Nl) vx[q].x = 0.0;
+      if (i + 1 >= (size_t)Nl) vx[q].y = 0.0;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < QX; q++) {
+    const int h = tid + kBandNT * q, c = chunk(h);
+    if (2 * h < ly.np) {
+      const int a = 2 * h + (even ? 2 * c : 0);
+      *reinterpret_cast<d2 *>(pw + a) = vp[q];
+      if (even && h == c * s && c > 0) *reinterpret_cast<d2 *>(pw + a - 2) = vp[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < QX; q++) {
+    const int h = tid + kBandNT * q;
+    if (h < ly.nx) {
+      const int a = h + (ly.pad ? chunk(h) : 0);
+      double x0 = vx[q].x, x1 = vx[q].y;
+      if (dir == C2L) {  // v_i = i u_i, v_0 = u_0
+        const double i = (double)(row0 + 2 * h);
+        x0 *= i == 0.0 ? 1.0 : i;
+        x1 *= i + 1.0;
+      }
+      xs[a] = x0;
+      xs[ly.nxs + a] = x1;
+    }
+  }
+  lds_sync();
+
+  // ---- the band
+  const int ng = (s + 15) >> 4, npair = (ng + 1) >> 1;
+  const int lseg = npair == 1 ? 2 : 1, nseg = 1 << lseg;
+  const int p = npair == 1 ? 0 : wave & 1, seg = npair == 1 ? wave : wave >> 1;
+  double acc[16];
+#pragma unroll
+  for (int k = 0; k < 16; k++) acc[k] = 0.0;
+  {
+    const int gl = lane & 15, sg = (lane >> 4) & 1, gam = 2 * p + (lane >> 5);
+    const size_t beta = (size_t)grp * kBandG + gl, nLm1 = (size_t)g.nL - 1;
+    const size_t r0 = beta * s + 16 * gam, cnt = (N - sg + 1) / 2;
+    const size_t cend = beta < nLm1 ? (beta + 2) * s : cnt;
+    const int len = 16 * gam < s && r0 < cnt ? (int)(cend - r0) : 0;
+    const int T = (2 * s - 32 * p + 15) >> 4;  // trips of the pair's longer group
+    const int t0 = 16 * (T * seg >> lseg), t1 = 16 * (T * (seg + 1) >> lseg);
+    // columns that every live row of the wave has (none where the chunks'
+    // ends differ)
+    const bool last = ((size_t)grp + 1) * kBandG > nLm1;
+    const int common = last ? 0 : 2 * s - 16 * std::min(2 * p + 1, ng - 1);
+    kdouble hp = (kdouble)head;
+    double pr[16], XA[4], PA[4];
+    const int s1 = ly.pad ? s : 1 << 20, s2 = even ? 2 * s : 1 << 20;
+    const int hq = gl * s + 16 * gam + t0, cx = chunk(hq);
+    BandPtr b;
+    b.x = xs + sg * ly.nxs + hq + (ly.pad ? cx : 0);
+    b.lx = ly.pad ? s * (cx + 1) - hq : 1 << 20;
+    // entry m = 2 h0 + t + sg of P at column t; its first 16, then the quad after
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const int m = 2 * hq - t0 + 4 * q, c = chunk(m >> 1);
+      const double *pm = pw + sg + m + (even ? 2 * c : 0);
+#pragma unroll
+      for (int k = 0; k < 4; k++) (q < 4 ? pr[4 * q + k] : PA[k]) = pm[k];
+      b.p = pm;
+      b.lp = even ? 2 * s * (c + 1) - m : 1 << 20;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) XA[k] = b.x[k];
+    int tb = t0;
+    if (tb == 0 && tb < t1) {
+      band_trip<2, S16>(b, s1, s2, hp, tb, len, pr, XA, PA, acc);
+      tb = 16;
+    }
+    for (; tb < t1 && tb + 16 <= common; tb += 16)
+      band_trip<0, S16>(b, s1, s2, hp, tb, len, pr, XA, PA, acc);
+    for (; tb < t1; tb += 16) band_trip<1, S16>(b, s1, s2, hp, tb, len, pr, XA, PA, acc);
+  }
+  // the lane's rows again, from a fresh copy of its index (the empty asm hides
+  // that it is the one used above, so nothing is held through the trips)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int gl = ln & 15, sg = (ln >> 4) & 1, gam = 2 * p + (ln >> 5);
+  if (dir == C2L) {
+    // less the sum; the C2L diagonal sqrt(pi) an_i v_i (src/C/leg2cheb.c:416)
+    const int h0 = gl * s + 16 * gam;
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      const int h = h0 + k, c = chunk(h);
+      const double d = kSqrtPi * xs[sg * ly.nxs + h + (ly.pad ? c : 0)] *
+                       pw[sg + 2 * h + (even ? 2 * c : 0)];
+      acc[k] = (seg == 0 ? d : 0.0) - acc[k];
+    }
+  }
+  const bool live = ((size_t)grp * kBandG + gl) * s + 16 * gam < (size_t)(N - sg + 1) / 2;
+  lds_sync();  // windows dead: the staging takes their place
+  if (live) {
+    double *o = sm + (seg * kBandG + gl) * ly.CS + 32 * gam + sg;
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (16 * gam + k < s) o[2 * k] = acc[k];
+  }
+  lds_sync();
+  // ---- the segments' sums, stored
+  const int nr = (int)std::min<size_t>((size_t)kBandG * 2 * s, (size_t)Nl - row0);
+  auto value = [&](int e) {
+    const double *o = sm + e + (even ? 2 * chunk(e >> 1) : 0);
+    double v = o[0] + o[kBandG * ly.CS];
+    if (nseg == 4) v += o[2 * kBandG * ly.CS] + o[3 * kBandG * ly.CS];
+    if (scale) {
+      const size_t i = row0 + e;
+      if (dir == L2C) {
+        v *= k2Pi;
+        if (i == 0) v *= 0.5;
+      } else {
+        v *= (double)i + 0.5;
+      }
+    }
+    return v;
+  };
+  if (es == 1) {
+    const __amdgpu_buffer_rsrc_t r = line_rsrc(dst + row0, nr);
+    for (int e = 2 * tid; e < nr; e += 2 * kBandNT) {
+      const d2 v = {value(e), e + 1 < nr ? value(e + 1) : 0.0};
+      store_pair(v, r, 8 * e);
+    }
+  } else {
+    for (int e = tid; e < nr; e += kBandNT) dst[(row0 + e) * es] = value(e);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // k_up: grid (2^(lu+2), lines), 256 threads.  G = 2^gu <= 16 leaf chunks.
@@ -79,17 +397,15 @@ size_t up_shared_bytes(const Geo &g) {
 // LM: the subtree levels on MFMA (MT > 0; chosen for subtrees of 2^3 and
 // 2^4 leaf chunks in calls of up to 8 lines) or on VALU.
 template <int MT, bool LM>
-__global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up(
-    const double *__restrict__ in, LineMap lm, Geo g,
-                                              int dir, const double *__restrict__ T,
-                                              const double *__restrict__ U,
-                                              const double *__restrict__ P,
-                                              double *__restrict__ wsall, size_t wsstride) {
-  extern __shared__ double sm[];
+__device__ __forceinline__ void up_group(const double *__restrict__ in, const LineMap &lm,
+                                         const Geo &g, int dir, const double *__restrict__ T,
+                                         const double *__restrict__ U,
+                                         const double *__restrict__ P,
+                                         double *__restrict__ wsall, size_t wsstride, int j,
+                                         double *sm) {
   const int M = MT > 0 ? MT : g.M;
   const int s = g.s, L = g.L, M2 = 2 * M, MM = M * M;
   const int G = 1 << g.gu;
-  const int j = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const double *src = in + line_off(lm, blockIdx.y);
   const size_t Nl = (size_t)line_len(lm, blockIdx.y, g.N);  // zeros past the line's end
@@ -322,6 +638,232 @@ __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4)))
     }
     part[((size_t)lev * ((size_t)4 << g.lu) + j) * M2 + o] = acc;
   }
+}
+
+// ---------------------------------------------------------------------------
+// The upward pass of a subtree of G = 2^gu <= 16 leaf chunks, M = 18 (steps 1
+// and 2, src/C/leg2cheb.c:1379-1399), all of it on v_mfma_f64_16x16x4f64 (A
+// operand: lane l holds A[l%16][l/16]; B: lane l holds B[l/16][l%16]; D: lane
+// l, register v holds D[l/16 + 4v][l%16]):
+//   leaf moments W_par (G x M) = X_par (G x s) T_par (s x M), one wave per
+//     (parity, 16-column tile of M);
+//   parents (M x 2n) = [U0 U1] (M x 2M) times the children stacked (2M x 2n),
+//     column 2c + parity for parent c, one wave per 16-row tile;
+//   contributions of the root to its ancestors above the subtree.
+// Every operand is loaded before any is used; each level leaves through LDS as
+// whole vectors.  Bound by latency: one chain of loads, products and barriers
+// per work-group.  s = 64: 2^16 5.5 us, 2^20 10.1, 64 lines of 2^18 89; with
+// scalar loads, the moments stored a double at a time from the accumulators
+// and (more than 8 lines) VALU levels 6.0, 11.8 and 107.  LDS: input [2][16][xst] (xst = 2 mod 4: rows in distinct
+// banks), two levels' moments [16 + 8][2][M].
+__host__ __device__ inline int up18_xstride(int s) { return s + (6 - (s & 3)) % 4; }
+struct Up18Lds {
+  int xst, w0, w1, total;
+};
+__host__ __device__ inline Up18Lds up18_lds(const Geo &g) {
+  Up18Lds d;
+  d.xst = up18_xstride(g.s);
+  d.w0 = 2 * 16 * d.xst;
+  d.w1 = d.w0 + 16 * 36;
+  d.total = d.w1 + 16 * 36;  // (the levels read 16 chunks, used or not)
+  return d;
+}
+bool up18_eligible(const Geo &g) { return g.M == 18 && g.s <= 64; }
+__device__ __forceinline__ void up18_group(const double *__restrict__ in, const LineMap &lm,
+                                           const Geo &g, int dir, const double *__restrict__ T,
+                                           const double *__restrict__ U,
+                                           const double *__restrict__ P,
+                                           double *__restrict__ wsall, size_t wsstride, int j,
+                                           double *sm) {
+  constexpr int M = 18, M2 = 36, MM = M * M;
+  const int s = g.s, G = 1 << g.gu;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, kq = lane >> 4;
+  const size_t es = lm.es, base = (size_t)j * G * 2 * s;
+  const size_t Nl = (size_t)line_len(lm, blockIdx.y, g.N);  // zeros past the line's end
+  const double *src = in + line_off(lm, blockIdx.y) + base * es;
+  const int nl = base < Nl ? (int)std::min<size_t>(Nl - base, (size_t)G * 2 * s) : 0;
+  double *ws = wsall + blockIdx.y * wsstride;
+  const WsLayout lay = ws_layout(g);
+  const Up18Lds ly = up18_lds(g);
+  double *xs = sm, *w0 = sm + ly.w0, *w1 = sm + ly.w1;
+
+  // ---- loads: input pairs (2 h, 2 h + 1)
+  constexpr int QX = 4;  // 16 s / 256 for s = 64
+  d2 vx[QX];
+  if (es == 1) {
+    const __amdgpu_buffer_rsrc_t r = line_rsrc(nl ? src : in, nl);
+#pragma unroll
+    for (int q = 0; q < QX; q++) vx[q] = load_pair(r, 16 * tid + 4096 * q, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < QX; q++) {
+      const int e = 2 * (tid + 256 * q);
+      vx[q].x = e < nl ? src[(size_t)e * es] : 0.0;
+      vx[q].y = e + 1 < nl ? src[(size_t)(e + 1) * es] : 0.0;
+    }
+  }
+  // T, rows 4 q + kq, column kb of this wave's (parity, tile); columns past M
+  // lie past the descriptor's end and read zero
+  const int sg = wave >> 1, kb = (wave & 1) * 16 + n16;
+  constexpr int QT = 16;
+  double tb[QT];
+  {
+    const __amdgpu_buffer_rsrc_t r = line_rsrc(T + (size_t)sg * s * M, s * M);
+    const int off = kb < M ? 8 * (kq * M + kb) : 1 << 30;
+#pragma unroll
+    for (int q = 0; q < QT; q++) tb[q] = load_one(r, off, 4 * M * 8 * q);
+  }
+  // [U0 U1], rows 16 rt + n16 of waves rt < 2: column k = 4 kk + kq, the
+  // second operator from k = M on
+  double ua[9];
+  {
+    const __amdgpu_buffer_rsrc_t r = line_rsrc(U, 2 * MM);
+    const int ra = wave * 16 + n16;
+    const int o0 = ra < M ? 8 * (ra * M + kq) : 1 << 30, o1 = ra < M ? o0 + 8 * (MM - M) : 1 << 30;
+    const int o4 = kq < 2 ? o0 : o1;
+#pragma unroll
+    for (int kk = 0; kk < 9; kk++) ua[kk] = load_one(r, kk < 4 ? o0 : kk == 4 ? o4 : o1, 32 * kk);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const unsigned inv = ((1u << 20) + s - 1) / s;  // h / s = h inv >> 20 for h <= 1024
+#pragma unroll
+  for (int q = 0; q < QX; q++) {
+    const int h = tid + 256 * q;
+    if (h < G * s) {
+      const int c = (int)(__umul24(h, inv) >> 20);
+      double x0 = vx[q].x, x1 = vx[q].y;
+      if (dir == C2L) {  // v_i = i u_i, v_0 = u_0 (src/C/leg2cheb.c:1325-1335)
+        const double i = (double)(base + 2 * h);
+        x0 *= i == 0.0 ? 1.0 : i;
+        x1 *= i + 1.0;
+      }
+      const int a = c * ly.xst + h - c * s;
+      xs[a] = x0;
+      xs[16 * ly.xst + a] = x1;
+    }
+  }
+  lds_sync();
+
+  // ---- step 1: leaf moments (rows of X past G are not used: each row of a
+  // product depends on its own row of A alone)
+  {
+    const double *xrow = xs + (sg * 16 + n16) * ly.xst + kq;
+    d4 D0 = {0, 0, 0, 0}, D1 = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < QT; q += 2) {
+      if (4 * q >= s) continue;
+      double a0 = xrow[4 * q], a1 = xrow[4 * q + 4];
+      if (4 * q + 8 > s) {
+        a0 = 4 * q + kq < s ? a0 : 0.0;
+        a1 = 4 * q + 4 + kq < s ? a1 : 0.0;
+      }
+      D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, tb[q], D0, 0, 0, 0);
+      D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, tb[q + 1], D1, 0, 0, 0);
+    }
+    D0 += D1;
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (kb < M) w0[(kq + 4 * v) * M2 + sg * M + kb] = D0[v];
+  }
+  lds_sync();
+
+  // ---- step 2: up the subtree; each level's vectors go out as they lie in LDS
+  auto store_level = [&](const double *wl, int lev, int n) {
+    double *w = ws + lay.w + (slot_base(lev) + (size_t)j * n) * M2;
+    for (int e = tid; e < n * M; e += 256)
+      *reinterpret_cast<d2 *>(w + 2 * e) = *reinterpret_cast<const d2 *>(wl + 2 * e);
+  };
+  store_level(w0, g.L - 1, G);
+  int n = G;
+  for (int lev = g.L - 2; lev >= g.lu; lev--) {
+    n >>= 1;
+    if (wave < 2) {
+      const int cc = n16 >> 1, sgc = n16 & 1;
+      double bv[9];
+#pragma unroll
+      for (int kk = 0; kk < 9; kk++) {
+        const int k = 4 * kk + kq, pu = k < M ? 0 : 1;
+        // children of column pair cc of the 8 (past n: values not used)
+        bv[kk] = w0[((2 * cc + pu) * 2 + sgc) * M + k - pu * M];
+      }
+      d4 D0 = {0, 0, 0, 0}, D1 = {0, 0, 0, 0};
+#pragma unroll
+      for (int kk = 0; kk < 9; kk += 2) {
+        D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[kk], bv[kk], D0, 0, 0, 0);
+        if (kk + 1 < 9) D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[kk + 1], bv[kk + 1], D1, 0, 0, 0);
+      }
+      D0 += D1;
+      double *o = w1 + n16 * M + wave * 16 + kq;
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (wave * 16 + kq + 4 * v < M && n16 < 2 * n) o[4 * v] = D0[v];
+    }
+    lds_sync();
+    double *tmp = w0;
+    w0 = w1;
+    w1 = tmp;
+    store_level(w0, lev, n);
+  }
+
+  // ---- contributions of the root (level lu, chunk j) to its ancestors:
+  // part[l][j] = P(lu-l, j mod 2^(lu-l)) w_root
+  double *part = ws + lay.part;
+  for (int task = tid; task < g.lu * M2; task += 256) {
+    const int lev = task / M2, o = task - lev * M2, sgp = o >= M, i = o - sgp * M;
+    const int k = g.lu - lev;
+    const size_t d = (size_t)j & (((size_t)1 << k) - 1);
+    const d2 *prow = reinterpret_cast<const d2 *>(P + ((((size_t)1 << k) - 2) + d) * MM +
+                                                  (size_t)i * M);
+    const double *x = w0 + sgp * M;
+    double a0 = 0, a1 = 0;
+#pragma unroll
+    for (int l = 0; l < M / 2; l++) {
+      const d2 p = prow[l];
+      a0 += p.x * x[2 * l];
+      a1 += p.y * x[2 * l + 1];
+    }
+    part[((size_t)lev * ((size_t)4 << g.lu) + j) * M2 + o] = a0 + a1;
+  }
+}
+
+// The upward pass and, in the same launch, the near-field band, which needs
+// nothing of the tree: grid (work-groups, lines, 2) with the band groups at z =
+// 0, ahead of the shorter upward groups, or (.., .., 1) for the upward pass
+// alone.  The band's products fill the CUs that the upward groups' loads and
+// barriers leave idle, and a launch and its tail go: s = 64, k_band and k_up
+// apart / together 2^16 15.5 / 10.8 us, 2^20 27.4 / 22.0, 64 lines of 2^18 254 /
+// 247.  Band groups behind the upward ones of each line: 256 lines of 2^15 220
+// us a call against 188.
+struct BandArgs {
+  double *out;
+  const double *tab, *head;
+};
+template <bool S16>
+__global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up(
+    const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
+    const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
+    size_t wsstride, BandArgs ba) {
+  extern __shared__ double sm[];
+  if (blockIdx.z + 1 == gridDim.z) {
+    if ((int)blockIdx.x < 4 << g.lu)
+      up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, blockIdx.x, sm);
+  } else {
+    const size_t off = line_off(lm, blockIdx.y);
+    band_group<S16>(in + off, ba.out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
+                    blockIdx.x, 0, ba.tab, ba.head, sm);
+  }
+}
+
+// The upward pass for other ranks and leaf sizes.
+template <int MT, bool LM>
+__global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up_any(
+    const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
+    const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
+    size_t wsstride) {
+  extern __shared__ double sm[];
+  up_group<MT, LM>(in, lm, g, dir, T, U, P, wsall, wsstride, blockIdx.x, sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -1030,7 +1572,9 @@ __host__ __device__ inline DownLds down_lds(const Geo &g) {
 }
 size_t down8_shared_bytes(const Geo &g);
 size_t down_shared_bytes(const Geo &g) {
-  return g.fast ? down8_shared_bytes(g) : 8 * (size_t)down_lds(g).total;
+  return g.fast ? down8_shared_bytes(g)
+         : g.far ? std::max(far_shared_bytes(g), band_shared_bytes(g))
+                 : 8 * (size_t)down_lds(g).total;
 }
 
 // Subtree chunk slot cl (level ld + lam, position ci) of work-group Rr:
@@ -1150,24 +1694,11 @@ __device__ __forceinline__ void subtree_locals(const Geo &g, int Rr, int tid, in
         const int p = item / nrt, rt = item - p * nrt;
         const int ra = rt * 16 + j;  // A row
         d4 D = {0, 0, 0, 0};
-        if (MT > 0) {  // all operand reads first, then the MFMA chain
-          constexpr int QK = MT > 0 ? (MT + 3) / 4 : 1;
-          double av[QK], bv[QK];
-#pragma unroll
-          for (int kk = 0; kk < QK; kk++) {
-            const int k = kk * 4 + (lane >> 4);
-            av[kk] = (ra < M && k < M) ? Dl[(p * M + ra) * (M + 1) + k] : 0.0;
-            bv[kk] = (j < n && k < M) ? cres[(bp + (j >> 1)) * M2 + (j & 1) * M + k] : 0.0;
-          }
-#pragma unroll
-          for (int kk = 0; kk < QK; kk++) D = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], bv[kk], D, 0, 0, 0);
-        } else {
-          for (int kk = 0; kk < ksteps; kk++) {
-            const int k = kk * 4 + (lane >> 4);
-            const double a = (ra < M && k < M) ? Dl[(p * M + ra) * (M + 1) + k] : 0.0;
-            const double b = (j < n && k < M) ? cres[(bp + (j >> 1)) * M2 + (j & 1) * M + k] : 0.0;
-            D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, D, 0, 0, 0);
-          }
+        for (int kk = 0; kk < ksteps; kk++) {
+          const int k = kk * 4 + (lane >> 4);
+          const double a = (ra < M && k < M) ? Dl[(p * M + ra) * (M + 1) + k] : 0.0;
+          const double b = (j < n && k < M) ? cres[(bp + (j >> 1)) * M2 + (j & 1) * M + k] : 0.0;
+          D = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, D, 0, 0, 0);
         }
         const int c = 2 * (j >> 1) + p, sgc = j & 1;
         const bool valid = j < n && ((size_t)Rr << lam) + c < ((size_t)4 << lev) - 2;
@@ -1431,7 +1962,8 @@ __global__ void __launch_bounds__(kDownNT) __attribute__((amdgpu_waves_per_eu(2)
 }
 
 // ---------------------------------------------------------------------------
-// k_down8: the downward pass for leaf sizes s = 16, 32, 64.  grid
+// k_down8: the downward pass for leaf sizes s = 16, 32, 64 of plans that have
+// no k_far (M != 18).  grid
 // (2^(ld+2), lines), 64 nw threads with nw = s/16 waves, G = 2^gd <= 16 leaf
 // chunks per work-group.
 //
@@ -1563,18 +2095,14 @@ __device__ __forceinline__ void band_seg8(const double *__restrict__ xsg,
 #undef FETCH
 }
 
-// Modes: K8_FULL band and far field; K8_BAND the near field alone, scaled
-// (directM).
-enum { K8_FULL = 0, K8_BAND = 1 };
-
-template <int DIR, int PRE, int MT>
+template <int DIR, int PRE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_down8(
-    const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g, int mode,
+    const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g,
     const double *__restrict__ wsall, size_t wsstride, const double *__restrict__ Dg,
     const double *__restrict__ Qg, const double *__restrict__ Tg, const double *__restrict__ tab,
     const double *__restrict__ head) {
   extern __shared__ double sm[];
-  const int M = MT > 0 ? MT : g.M;
+  const int M = g.M;
   const int s = g.s, N = g.N, M2 = 2 * M, MM = M * M;
   // N: the plan geometry; Nl: this line's length (inputs past it read as zero)
   const int Nl = line_len(lm, blockIdx.y, N);
@@ -1585,7 +2113,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   // the wave index is wave-uniform; saying so lets the band's column offsets
   // and head loads live in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool do_band = true, do_far = mode == K8_FULL;
   const size_t row0 = (size_t)Rr * G * 2 * s;
   if (row0 >= (size_t)Nl) return;  // the whole work-group
   const int nr = (int)std::min((size_t)G * 2 * s, (size_t)Nl - row0);
@@ -1608,232 +2135,175 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   // chain row of Q, D) are needed first; the band windows (x, the Lambda span,
   // the head) stay in flight through the tree pass, whose barriers are
   // LDS-only.
-  const int nm = do_far ? (g.ld + 2 * G - 1) * M2 : 0;
+  const int nm = (g.ld + 2 * G - 1) * M2;
   constexpr int QM = 6;
   double vm[QM];
   bool okm[QM];
-  const int nq = do_far ? g.ld * M : 0;
-  double qr[MT > 0 ? MT : 1];
-  constexpr int QD = MT > 0 ? (2 * MT * MT + 63) / 64 : 1;  // D(0), D(1) for the LDS copy
-  double vd[QD];
-  if (do_far) {
 #pragma unroll
-    for (int q = 0; q < QM; q++) {
-      const int e = q * NT + tid;
-      const size_t a = m2l_elem(g, Rr, e < nm ? e : 0, M2, okm[q]);
-      okm[q] = okm[q] && e < nm;
-      vm[q] = m2l[okm[q] ? a : 0];
-    }
-    if (MT > 0 && nq > 0) {
-      const double *qrow = qrow_ptr(Qg, g, Rr, tid < nq ? tid : 0, M);
-#pragma unroll
-      for (int l = 0; l < (MT > 0 ? MT : 1); l++) qr[l] = qrow[l * M];
-    }
-#pragma unroll
-    for (int q = 0; q < QD; q++) {
-      const int e = q * NT + tid;
-      vd[q] = Dg[e < 2 * MM ? e : 0];
-    }
+  for (int q = 0; q < QM; q++) {
+    const int e = q * NT + tid;
+    const size_t a = m2l_elem(g, Rr, e < nm ? e : 0, M2, okm[q]);
+    okm[q] = okm[q] && e < nm;
+    vm[q] = m2l[okm[q] ? a : 0];
   }
   // keep the tree operands ahead of the windows in the memory pipeline: the
   // stores below then wait for them alone
   __builtin_amdgcn_sched_barrier(0);
   // x: input elements row0 + e, e < nX (both parities interleaved)
-  const int nX = do_band ? 2 * ((G + 1) * s + 8) : 0;
+  const int nX = 2 * ((G + 1) * s + 8);
   constexpr int QX = 9;  // ceil(nX / NT) for G = 16
   double vx[QX];
   // Lambda: the contiguous span 2 hc0 + e, e < 2Gs + s + 16; element e lies
   // in chunk window e / 2s and, when e mod 2s < s + 16, also in the one before
-  const int QL = 3 * s + 16, nLs = do_band ? 2 * G * s + s + 16 : 0;
+  const int QL = 3 * s + 16, nLs = 2 * G * s + s + 16;
   constexpr int QLS = 9;  // ceil(nLs / NT) for G = 16
   double vl[QLS];
   const int nhd = 2 * s + 16;  // <= NT
   double vh = 0.0;
-  if (do_band) {
 #pragma unroll
-    for (int q = 0; q < QX; q++)
-      vx[q] = src[std::min(row0 + q * NT + tid, (size_t)Nl - 1) * lm.es];
+  for (int q = 0; q < QX; q++)
+    vx[q] = src[std::min(row0 + q * NT + tid, (size_t)Nl - 1) * lm.es];
 #pragma unroll
-    for (int q = 0; q < QLS; q++)
-      vl[q] = tab[std::min(2 * hc0 + q * NT + tid, (size_t)N - 1)];
-    vh = head[tid < nhd ? tid : 0];
-  }
+  for (int q = 0; q < QLS; q++)
+    vl[q] = tab[std::min(2 * hc0 + q * NT + tid, (size_t)N - 1)];
+  vh = head[tid < nhd ? tid : 0];
   __builtin_amdgcn_sched_barrier(0);
-  if (do_far) {
 #pragma unroll
-    for (int q = 0; q < QM; q++) {
-      const int e = q * NT + tid;
-      if (e < nm) mres[e] = okm[q] ? vm[q] : 0.0;
-    }
+  for (int q = 0; q < QM; q++) {
+    const int e = q * NT + tid;
+    if (e < nm) mres[e] = okm[q] ? vm[q] : 0.0;
   }
   for (int e = QM * NT + tid; e < nm; e += NT) {
     bool ok;
     const size_t a = m2l_elem(g, Rr, e, M2, ok);
     mres[e] = ok ? m2l[a] : 0.0;
   }
-  if (do_far) {
-#pragma unroll
-    for (int q = 0; q < QD; q++) {
-      const int e = q * NT + tid;
-      if (MT > 0 && e < 2 * MM) dl[(e / M) * (M + 1) + e % M] = vd[q];
-    }
-    for (int e = (MT > 0 ? QD * NT : 0) + tid; e < 2 * MM; e += NT)
-      dl[(e / M) * (M + 1) + e % M] = Dg[e];
-  }
+  for (int e = tid; e < 2 * MM; e += NT)
+    dl[(e / M) * (M + 1) + e % M] = Dg[e];
   lds_sync();
 
   // ---- phase 2: local expansions of the subtree
-  if (do_far)
-    subtree_locals<MT, true>(g, Rr, tid, NT, mres, qp, cres, qr, nullptr, nullptr, Qg, Dg, dl,
+  subtree_locals<0, true>(g, Rr, tid, NT, mres, qp, cres, nullptr, nullptr, nullptr, Qg, Dg, dl,
                             LdsSync{});
 
-  // A operand (T) of this wave's two far-field tiles, in flight during the band
   const int ntm = s >> 4, ksteps = (M + 3) >> 2;
-  constexpr int QK = MT > 0 ? (MT + 3) / 4 : 1;
-  double ta[2][QK];
+  // ---- the band windows
+#pragma unroll
+  for (int q = 0; q < QX; q++) {
+    const int e = q * NT + tid;
+    if (e < nX) {
+      const size_t i = row0 + e;
+      const double u = i < (size_t)Nl ? vx[q] : 0.0;
+      const int h = e >> 1;
+      xs[(e & 1) * ly.nxs + h + (h >> sh)] = (DIR == 1 && i > 0) ? u * (double)i : u;  // v_i = i u_i
+    }
+  }
+  for (int e = QX * NT + tid; e < nX; e += NT) {
+    const size_t i = row0 + e;
+    double u = i < (size_t)Nl ? src[i * lm.es] : 0.0;
+    if (DIR == 1 && i > 0) u *= (double)i;
+    const int h = e >> 1;
+    xs[(e & 1) * ly.nxs + h + (h >> sh)] = u;
+  }
+  auto put_lambda = [&](int e, double v) {
+    const int c = e >> (sh + 1), q = e - (c << (sh + 1));
+    if (2 * hc0 + e >= (size_t)N) v = 0.0;
+    if (c < G) lw[c * ly.LW + q] = v;
+    if (c > 0 && q + 2 * s < QL) lw[(c - 1) * ly.LW + q + 2 * s] = v;
+  };
+#pragma unroll
+  for (int q = 0; q < QLS; q++) {
+    const int e = q * NT + tid;
+    if (e < nLs) put_lambda(e, vl[q]);
+  }
+  for (int e = QLS * NT + tid; e < nLs; e += NT)
+    put_lambda(e, tab[std::min(2 * hc0 + e, (size_t)N - 1)]);
+  if (tid < nhd) hd[tid] = vh;
+  lds_sync();
+
+  // ---- phase 3: near field.  Lane (chunk gl, parity sg, del); wave:
+  // segment A of pair wave, segment B of pair nw-1-wave
+  const int gl = lane & 15, sg = (lane >> 4) & 1, del = lane >> 5;
+  const int cnt = (N - sg + 1) / 2;  // elements of parity sg
+  const size_t beta = (size_t)Rr * G + gl;
+  const size_t nLm1 = (size_t)g.nL - 1;
+  const size_t cend = beta < nLm1 ? (beta + 2) * s : (size_t)cnt;
+  const bool ragged = (size_t)(Rr + 1) * G > nLm1;  // work-group holds the last chunk
+  const double *xsg = xs + sg * ly.nxs;
+  double accA[8], accB[8];
+  int rA = -1, rB = -1;  // first row (half index) of each segment, -1: none
+  {
+    const int p = wave, gam = 2 * p + del, ts = s - 8 * p;
+    const size_t r0 = beta * s + 8 * gam;
+    const bool live = gl < G && r0 < (size_t)cnt;
+    const int len = live ? (int)(cend - r0) : 0;
+    const int h0 = (int)(r0 - hc0);
+    const double *pw = lw + gl * ly.LW + 16 * gam + sg;
+#pragma unroll
+    for (int k = 0; k < 8; k++) accA[k] = 0.0;
+    if (live) {
+      rA = h0;
+      if (DIR == 1) {  // C2L diagonal: sqrt(pi) an_i v_i (src/C/leg2cheb.c:416)
+        const double *xr = xsg + h0 + (h0 >> sh);
+#pragma unroll
+        for (int k = 0; k < 8; k++) accA[k] = kSqrtPi * xr[k] * pw[2 * k];
+      }
+    }
+    if (ragged)
+      band_seg8<DIR, PRE, true>(xsg, pw, hd, h0, sh, 0, std::min(ts, len), len, accA);
+    else
+      band_seg8<DIR, PRE, false>(xsg, pw, hd, h0, sh, 0, ts, len, accA);
+  }
+  {
+    const int p = nw - 1 - wave, gam = 2 * p + del, ts = s - 8 * p;
+    const size_t r0 = beta * s + 8 * gam;
+    const bool live = gl < G && r0 < (size_t)cnt;
+    const int len = live ? (int)(cend - r0) : 0;
+    const int h0 = (int)(r0 - hc0);
+    const double *pw = lw + gl * ly.LW + 16 * gam + sg;
+#pragma unroll
+    for (int k = 0; k < 8; k++) accB[k] = 0.0;
+    if (live) rB = h0;
+    if (ragged)
+      band_seg8<DIR, PRE, true>(xsg, pw, hd, h0, sh, ts, len, len, accB);
+    else
+      band_seg8<DIR, PRE, false>(xsg, pw, hd, h0, sh, ts, len, len, accB);
+  }
+  lds_sync();  // windows dead: the staging takes their place
+
+  // ---- phase 4: segment A sums to ob, segment B sums to ob2 (each row
+  // once in each)
+  auto stage = [&](int rl, const double *acc, double *dstg) {
+    if (rl < 0) return;
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (hc0 + rl + k < (size_t)cnt) dstg[slot(2 * (rl + k) + sg)] = acc[k];
+  };
+  stage(rA, accA, ob);
+  stage(rB, accB, ob2);
+  lds_sync();
+  // F_par^T (G x s) = C_par^T (G x M) T_par^T (M x s), tile (parity sgf,
+  // rows 16 rt..): A[n][k] = c_k of leaf n, B[k][m] = T_par[16 rt + m][k];
+  // lane l then holds leaf l/16 + 4v, row 16 rt + l%16; added into ob.
+  const int n = lane & 15;
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int tile = wave + j * nw, sgf = tile / ntm, rt = tile - sgf * ntm;
-    const int m = rt * 16 + (lane & 15);
-#pragma unroll
-    for (int kk = 0; kk < QK; kk++) {
+    d4 D = {0, 0, 0, 0};
+    for (int kk = 0; kk < ksteps; kk++) {
       const int k = kk * 4 + (lane >> 4);
-      ta[j][kk] = (MT > 0 && do_far && k < M) ? Tg[((size_t)sgf * s + m) * M + k] : 0.0;
+      const double bv = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
+      const double av = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
+      D = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, D, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int leaf = (lane >> 4) + 4 * v, m = rt * 16 + n;
+      const int e = 2 * (leaf * s + m) + sgf;
+      if (leaf < G && e < nr) ob[slot(e)] += D[v];
     }
   }
-
-  if (do_band) {
-    // ---- the band windows
-#pragma unroll
-    for (int q = 0; q < QX; q++) {
-      const int e = q * NT + tid;
-      if (e < nX) {
-        const size_t i = row0 + e;
-        const double u = i < (size_t)Nl ? vx[q] : 0.0;
-        const int h = e >> 1;
-        xs[(e & 1) * ly.nxs + h + (h >> sh)] = (DIR == 1 && i > 0) ? u * (double)i : u;  // v_i = i u_i
-      }
-    }
-    for (int e = QX * NT + tid; e < nX; e += NT) {
-      const size_t i = row0 + e;
-      double u = i < (size_t)Nl ? src[i * lm.es] : 0.0;
-      if (DIR == 1 && i > 0) u *= (double)i;
-      const int h = e >> 1;
-      xs[(e & 1) * ly.nxs + h + (h >> sh)] = u;
-    }
-    auto put_lambda = [&](int e, double v) {
-      const int c = e >> (sh + 1), q = e - (c << (sh + 1));
-      if (2 * hc0 + e >= (size_t)N) v = 0.0;
-      if (c < G) lw[c * ly.LW + q] = v;
-      if (c > 0 && q + 2 * s < QL) lw[(c - 1) * ly.LW + q + 2 * s] = v;
-    };
-#pragma unroll
-    for (int q = 0; q < QLS; q++) {
-      const int e = q * NT + tid;
-      if (e < nLs) put_lambda(e, vl[q]);
-    }
-    for (int e = QLS * NT + tid; e < nLs; e += NT)
-      put_lambda(e, tab[std::min(2 * hc0 + e, (size_t)N - 1)]);
-    if (tid < nhd) hd[tid] = vh;
-    lds_sync();
-
-    // ---- phase 3: near field.  Lane (chunk gl, parity sg, del); wave:
-    // segment A of pair wave, segment B of pair nw-1-wave
-    const int gl = lane & 15, sg = (lane >> 4) & 1, del = lane >> 5;
-    const int cnt = (N - sg + 1) / 2;  // elements of parity sg
-    const size_t beta = (size_t)Rr * G + gl;
-    const size_t nLm1 = (size_t)g.nL - 1;
-    const size_t cend = beta < nLm1 ? (beta + 2) * s : (size_t)cnt;
-    const bool ragged = (size_t)(Rr + 1) * G > nLm1;  // work-group holds the last chunk
-    const double *xsg = xs + sg * ly.nxs;
-    double accA[8], accB[8];
-    int rA = -1, rB = -1;  // first row (half index) of each segment, -1: none
-    {
-      const int p = wave, gam = 2 * p + del, ts = s - 8 * p;
-      const size_t r0 = beta * s + 8 * gam;
-      const bool live = gl < G && r0 < (size_t)cnt;
-      const int len = live ? (int)(cend - r0) : 0;
-      const int h0 = (int)(r0 - hc0);
-      const double *pw = lw + gl * ly.LW + 16 * gam + sg;
-#pragma unroll
-      for (int k = 0; k < 8; k++) accA[k] = 0.0;
-      if (live) {
-        rA = h0;
-        if (DIR == 1) {  // C2L diagonal: sqrt(pi) an_i v_i (src/C/leg2cheb.c:416)
-          const double *xr = xsg + h0 + (h0 >> sh);
-#pragma unroll
-          for (int k = 0; k < 8; k++) accA[k] = kSqrtPi * xr[k] * pw[2 * k];
-        }
-      }
-      if (ragged)
-        band_seg8<DIR, PRE, true>(xsg, pw, hd, h0, sh, 0, std::min(ts, len), len, accA);
-      else
-        band_seg8<DIR, PRE, false>(xsg, pw, hd, h0, sh, 0, ts, len, accA);
-    }
-    {
-      const int p = nw - 1 - wave, gam = 2 * p + del, ts = s - 8 * p;
-      const size_t r0 = beta * s + 8 * gam;
-      const bool live = gl < G && r0 < (size_t)cnt;
-      const int len = live ? (int)(cend - r0) : 0;
-      const int h0 = (int)(r0 - hc0);
-      const double *pw = lw + gl * ly.LW + 16 * gam + sg;
-#pragma unroll
-      for (int k = 0; k < 8; k++) accB[k] = 0.0;
-      if (live) rB = h0;
-      if (ragged)
-        band_seg8<DIR, PRE, true>(xsg, pw, hd, h0, sh, ts, len, len, accB);
-      else
-        band_seg8<DIR, PRE, false>(xsg, pw, hd, h0, sh, ts, len, len, accB);
-    }
-    lds_sync();  // windows dead: the staging takes their place
-
-    // ---- phase 4: segment A sums to ob, segment B sums to ob2 (each row
-    // once in each)
-    auto stage = [&](int rl, const double *acc, double *dstg) {
-      if (rl < 0) return;
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        if (hc0 + rl + k < (size_t)cnt) dstg[slot(2 * (rl + k) + sg)] = acc[k];
-    };
-    stage(rA, accA, ob);
-    stage(rB, accB, ob2);
-    lds_sync();
-  }
-  if (do_far) {
-    // F_par^T (G x s) = C_par^T (G x M) T_par^T (M x s), tile (parity sgf,
-    // rows 16 rt..): A[n][k] = c_k of leaf n, B[k][m] = T_par[16 rt + m][k];
-    // lane l then holds leaf l/16 + 4v, row 16 rt + l%16; added into ob.
-    const int n = lane & 15;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int tile = wave + j * nw, sgf = tile / ntm, rt = tile - sgf * ntm;
-      d4 D = {0, 0, 0, 0};
-      if (MT > 0) {
-        double av[QK];
-#pragma unroll
-        for (int kk = 0; kk < QK; kk++) {
-          const int k = kk * 4 + (lane >> 4);
-          av[kk] = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-        }
-#pragma unroll
-        for (int kk = 0; kk < QK; kk++) D = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], ta[j][kk], D, 0, 0, 0);
-      } else {
-        for (int kk = 0; kk < ksteps; kk++) {
-          const int k = kk * 4 + (lane >> 4);
-          const double bv = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
-          const double av = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-          D = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, D, 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int leaf = (lane >> 4) + 4 * v, m = rt * 16 + n;
-        const int e = 2 * (leaf * s + m) + sgf;
-        if (leaf < G && e < nr) ob[slot(e)] += D[v];
-      }
-    }
-    lds_sync();
-  }
+  lds_sync();
   // ---- store: the scaled sum
   for (int e = tid; e < nr; e += NT) {
     const size_t i = row0 + e;
@@ -1885,14 +2355,14 @@ __host__ __device__ inline Down8rLds down8r_lds(const Geo &g) {
 }
 size_t down8r_shared_bytes(const Geo &g) { return 8 * (size_t)down8r_lds(g).total; }
 
-template <int DIR, int PRE, int MT>
+template <int DIR, int PRE>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k_down8r(
     const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g,
     const double *__restrict__ wsall, size_t wsstride, const double *__restrict__ Dg,
     const double *__restrict__ Qg, const double *__restrict__ Tg, const double *__restrict__ tab,
     const double *__restrict__ head, int shift) {
   extern __shared__ double sm[];
-  const int M = MT > 0 ? MT : g.M;
+  const int M = g.M;
   const int s = g.s, N = g.N, M2 = 2 * M, MM = M * M;
   const int Nl = line_len(lm, blockIdx.y, N);
   const int G = 1 << g.gd, sh = 31 - __builtin_clz(s);
@@ -1985,26 +2455,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     constexpr int QM = 6;
     double vm[QM];
     bool okm[QM];
-    const int nq = g.ld * M;
-    double qr[MT > 0 ? MT : 1];
-    constexpr int QD = MT > 0 ? (2 * MT * MT + 63) / 64 : 1;
-    double vd[QD];
 #pragma unroll
     for (int q = 0; q < QM; q++) {
       const int e = q * NT + tid;
       const size_t a = m2l_elem(g, Rr, e < nm ? e : 0, M2, okm[q]);
       okm[q] = okm[q] && e < nm;
       vm[q] = m2l[okm[q] ? a : 0];
-    }
-    if (MT > 0 && nq > 0) {
-      const double *qrow = qrow_ptr(Qg, g, Rr, tid < nq ? tid : 0, M);
-#pragma unroll
-      for (int l = 0; l < (MT > 0 ? MT : 1); l++) qr[l] = qrow[l * M];
-    }
-#pragma unroll
-    for (int q = 0; q < QD; q++) {
-      const int e = q * NT + tid;
-      vd[q] = Dg[e < 2 * MM ? e : 0];
     }
 #pragma unroll
     for (int q = 0; q < QM; q++) {
@@ -2016,44 +2472,26 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
       const size_t a = m2l_elem(g, Rr, e, M2, ok);
       mres[e] = ok ? m2l[a] : 0.0;
     }
-#pragma unroll
-    for (int q = 0; q < QD; q++) {
-      const int e = q * NT + tid;
-      if (MT > 0 && e < 2 * MM) dl[(e / M) * (M + 1) + e % M] = vd[q];
-    }
-    for (int e = (MT > 0 ? QD * NT : 0) + tid; e < 2 * MM; e += NT)
+    for (int e = tid; e < 2 * MM; e += NT)
       dl[(e / M) * (M + 1) + e % M] = Dg[e];
     rs();
-    subtree_locals<MT, true>(g, Rr, tid, NT, mres, qp, cres, qr, nullptr, nullptr, Qg, Dg, dl,
+    subtree_locals<0, true>(g, Rr, tid, NT, mres, qp, cres, nullptr, nullptr, nullptr, Qg, Dg, dl,
                              rs);
     // far field: F_par^T (G x s) = C_par^T (G x M) T_par^T (M x s) on
     // v_mfma_f64_16x16x4f64, two tiles (parity, 16 rows) per wave, written
     // to obf (the chain and subtree operands under it are dead: the last
     // role barrier of subtree_locals is behind every wave)
     const int ntm = s >> 4, ksteps = (M + 3) >> 2;
-    constexpr int QK = MT > 0 ? (MT + 3) / 4 : 1;
     const int n = lane & 15;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       const int tile = wave + j * nw, sgf = tile / ntm, rt = tile - sgf * ntm;
       d4 D = {0, 0, 0, 0};
-      if (MT > 0) {
-        double av[QK], bv[QK];
-#pragma unroll
-        for (int kk = 0; kk < QK; kk++) {
-          const int k = kk * 4 + (lane >> 4);
-          bv[kk] = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
-          av[kk] = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-        }
-#pragma unroll
-        for (int kk = 0; kk < QK; kk++) D = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], bv[kk], D, 0, 0, 0);
-      } else {
-        for (int kk = 0; kk < ksteps; kk++) {
-          const int k = kk * 4 + (lane >> 4);
-          const double bv = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
-          const double av = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-          D = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, D, 0, 0, 0);
-        }
+      for (int kk = 0; kk < ksteps; kk++) {
+        const int k = kk * 4 + (lane >> 4);
+        const double bv = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
+        const double av = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
+        D = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, D, 0, 0, 0);
       }
 #pragma unroll
       for (int v = 0; v < 4; v++) {
@@ -2178,313 +2616,251 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
 }
 
 // ---------------------------------------------------------------------------
-// Split downward pass: k_band (the near field) and k_far (L2L and the leaf
-// evaluation), each lean enough that several work-groups share a CU, so one
-// work-group's loads and barriers overlap another's arithmetic.  k_band has
-// no input from the tree: it runs first and writes the raw band sums (the
-// C2L diagonal included) over the output; k_far then adds the far field and
-// applies the final scaling (src/C/leg2cheb.c:1467-1483 and the band scaling
-// of :236-535).  Both use k_down8's work-group partition (2^gd leaf chunks,
-// s/16 waves), band lane layout and LDS windows.
-struct BandLds {
-  int xs, nxs, lw, LW, hd, total;
-};
-__host__ __device__ inline BandLds band_lds(const Geo &g) {
-  const Down8Lds d = down8_lds(g);
-  return {d.xs, d.nxs, d.lw, d.LW, d.hd, d.hd + 2 * g.s + 16};
-}
-size_t band_shared_bytes(const Geo &g) { return 8 * (size_t)band_lds(g).total; }
-
-// Band sums of the work-group's rows, written over the output: raw for
-// k_far, or with the final scaling when scale != 0 (the band alone,
-// directM).  2 s/16 waves: wave w < s/16 runs segment A of row pair w, wave
-// s/16 + w segment B of row pair s/16 - 1 - w (k_down8's split of each row
-// group's columns, one segment per wave), so no wave holds two sets of sums
-// and the kernel fits 128 VGPRs.
-template <int DIR, int PRE>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k_band(
-    const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g, int scale,
+// k_band: the near field by itself, for directM (scaled) and the split
+// downward pass (down_split; raw sums, the C2L diagonal included, over the
+// output; k_far adds the far field and scales, src/C/leg2cheb.c:1467-1483 and
+// the band scaling of :236-535).  Grid (band groups, lines), 256 threads.
+template <bool S16>
+__global__ void __launch_bounds__(kBandNT) __attribute__((amdgpu_waves_per_eu(4))) k_band(
+    const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g, int dir, int scale,
     const double *__restrict__ tab, const double *__restrict__ head) {
   extern __shared__ double sm[];
+  const size_t off = line_off(lm, blockIdx.y);
+  band_group<S16>(in + off, out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
+                  (int)blockIdx.x, scale, tab, head, sm);
+}
+
+// ---------------------------------------------------------------------------
+// k_far: the downward pass of a subtree of G = 2^gd leaf chunks (any leaf size
+// s <= 64, M = 18; src/C/leg2cheb.c:1437-1483): the ancestor chain in one
+// step, the subtree's levels and the leaf evaluation on MFMA, added to the raw
+// band sums in the output, scaled and stored.  Grid (2^(ld+2), lines), 256
+// threads.  Latency-bound: every operand (M2L vectors, chain rows, D and T as
+// MFMA fragments, the band sums) is loaded up front, so that the dependent
+// steps run from registers and LDS.  s = 64: 2^16 6.7 us, 2^20 12.0, 64 lines of
+// 2^18 94; with the operands read as each step needs them 7.8, 13.3 and 130.
+constexpr int kFarNT = 256;
+struct FarLds {
+  int mres, qp, ob, CS, total;
+};
+__host__ __device__ inline FarLds far_lds(const Geo &g) {
+  const int G = 1 << g.gd, s = g.s, M2 = 2 * g.M;
+  FarLds d;
+  d.mres = (2 * G - 1) * M2;  // after the local expansions [slot][parity][M]
+  d.qp = d.mres + (g.ld + 2 * G - 1) * M2;
+  d.ob = d.mres;  // far field [leaf][CS], over the dead M2L vectors
+  d.CS = 2 * s + ((s & 1) ? 0 : 2);
+  d.total = std::max(d.qp + std::max(g.ld, 1) * M2, d.ob + G * d.CS);
+  return d;
+}
+size_t far_shared_bytes(const Geo &g) { return 8 * (size_t)far_lds(g).total; }
+bool far_eligible(const Geo &g) { return g.M == 18 && g.s <= kBandMaxS; }
+
+__global__ void __launch_bounds__(kFarNT) __attribute__((amdgpu_waves_per_eu(4))) k_far(
+    double *__restrict__ out, LineMap lm, Geo g, int dir, const double *__restrict__ wsall,
+    size_t wsstride, const double *__restrict__ Dg, const double *__restrict__ Qg,
+    const double *__restrict__ Tg) {
+  extern __shared__ double sm[];
+  constexpr int M = 18, M2 = 36, MM = M * M;
   const int s = g.s, N = g.N;
   const int Nl = line_len(lm, blockIdx.y, N);
-  const int G = 1 << g.gd, sh = 31 - __builtin_clz(s);
-  const int nw = s >> 4, NT = 128 * nw;
-  const int Rr = blockIdx.x;
+  const int G = 1 << g.gd, Rr = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t row0 = (size_t)Rr * G * 2 * s;
   if (row0 >= (size_t)Nl) return;  // the whole work-group
   const int nr = (int)std::min((size_t)G * 2 * s, (size_t)Nl - row0);
-  const size_t hc0 = (size_t)Rr * G * s;
-  const size_t off = line_off(lm, blockIdx.y);
-  const double *src = in + off;
-  double *dst = out + off;
-  const BandLds ly = band_lds(g);
-  double *xs = sm + ly.xs, *lw = sm + ly.lw, *hd = sm + ly.hd;
-  double *ob = xs, *ob2 = lw;  // staging after the band (see k_down8)
-  auto slot = [&](int e) { return e + (e >> (sh + 1)); };
-
-  // ---- loads: the x window, the Lambda span, the head (one batch), at
-  // raised priority: their address arithmetic would otherwise wait behind
-  // the band FMAs of an older work-group on the same CU
-  __builtin_amdgcn_s_setprio(2);
-  const int nX = 2 * ((G + 1) * s + 8);
-  constexpr int QX = 5;  // ceil(nX / NT) for G = 16
-  double vx[QX];
-  const int QL = 3 * s + 16, nLs = 2 * G * s + s + 16;
-  constexpr int QLS = 5;
-  double vl[QLS];
-  const int nhd = 2 * s + 16;
-#pragma unroll
-  for (int q = 0; q < QX; q++) vx[q] = src[std::min(row0 + q * NT + tid, (size_t)Nl - 1) * lm.es];
-#pragma unroll
-  for (int q = 0; q < QLS; q++) vl[q] = tab[std::min(2 * hc0 + q * NT + tid, (size_t)N - 1)];
-  const double vh = head[tid < nhd ? tid : 0];
-#pragma unroll
-  for (int q = 0; q < QX; q++) {
-    const int e = q * NT + tid;
-    if (e < nX) {
-      const size_t i = row0 + e;
-      const double u = i < (size_t)Nl ? vx[q] : 0.0;
-      const int h = e >> 1;
-      xs[(e & 1) * ly.nxs + h + (h >> sh)] = (DIR == 1 && i > 0) ? u * (double)i : u;
-    }
-  }
-  for (int e = QX * NT + tid; e < nX; e += NT) {
-    const size_t i = row0 + e;
-    double u = i < (size_t)Nl ? src[i * lm.es] : 0.0;
-    if (DIR == 1 && i > 0) u *= (double)i;
-    const int h = e >> 1;
-    xs[(e & 1) * ly.nxs + h + (h >> sh)] = u;
-  }
-  auto put_lambda = [&](int e, double v) {
-    const int c = e >> (sh + 1), q = e - (c << (sh + 1));
-    if (2 * hc0 + e >= (size_t)N) v = 0.0;
-    if (c < G) lw[c * ly.LW + q] = v;
-    if (c > 0 && q + 2 * s < QL) lw[(c - 1) * ly.LW + q + 2 * s] = v;
-  };
-#pragma unroll
-  for (int q = 0; q < QLS; q++) {
-    const int e = q * NT + tid;
-    if (e < nLs) put_lambda(e, vl[q]);
-  }
-  for (int e = QLS * NT + tid; e < nLs; e += NT)
-    put_lambda(e, tab[std::min(2 * hc0 + e, (size_t)N - 1)]);
-  if (tid < nhd) hd[tid] = vh;
-  lds_sync();
-  __builtin_amdgcn_s_setprio(0);
-
-  // ---- the band: lane (chunk gl, parity sg, del), one segment per wave
-  const int gl = lane & 15, sg = (lane >> 4) & 1, del = lane >> 5;
-  const int cnt = (N - sg + 1) / 2;
-  const size_t beta = (size_t)Rr * G + gl;
-  const size_t nLm1 = (size_t)g.nL - 1;
-  const size_t cend = beta < nLm1 ? (beta + 2) * s : (size_t)cnt;
-  const bool ragged = (size_t)(Rr + 1) * G > nLm1;
-  const double *xsg = xs + sg * ly.nxs;
-  const bool segB = wave >= nw;
-  const int p = segB ? 2 * nw - 1 - wave : wave, gam = 2 * p + del, ts = s - 8 * p;
-  const size_t r0 = beta * s + 8 * gam;
-  const bool live = gl < G && r0 < (size_t)cnt;
-  const int len = live ? (int)(cend - r0) : 0;
-  const int h0 = (int)(r0 - hc0);
-  const double *pw = lw + gl * ly.LW + 16 * gam + sg;
-  double acc[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) acc[k] = 0.0;
-  if (!segB) {
-    if (DIR == 1 && live) {  // C2L diagonal: sqrt(pi) an_i v_i (src/C/leg2cheb.c:416)
-      const double *xr = xsg + h0 + (h0 >> sh);
-#pragma unroll
-      for (int k = 0; k < 8; k++) acc[k] = kSqrtPi * xr[k] * pw[2 * k];
-    }
-    if (ragged)
-      band_seg8<DIR, PRE, true, true>(xsg, pw, hd, h0, sh, 0, std::min(ts, len), len, acc);
-    else
-      band_seg8<DIR, PRE, false, true>(xsg, pw, hd, h0, sh, 0, ts, len, acc);
-  } else {
-    if (ragged)
-      band_seg8<DIR, PRE, true, true>(xsg, pw, hd, h0, sh, ts, len, len, acc);
-    else
-      band_seg8<DIR, PRE, false, true>(xsg, pw, hd, h0, sh, ts, len, len, acc);
-  }
-  lds_sync();  // windows dead: the staging takes their place
-  if (live) {
-    double *dstg = segB ? ob2 : ob;
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (hc0 + h0 + k < (size_t)cnt) dstg[slot(2 * (h0 + k) + sg)] = acc[k];
-  }
-  lds_sync();
-  for (int e = tid; e < nr; e += NT) {
-    const size_t i = row0 + e;
-    double v = ob[slot(e)] + ob2[slot(e)];
-    if (scale) {
-      if (DIR == 0) {
-        v *= k2Pi;
-        if (i == 0) v *= 0.5;
-      } else {
-        v *= (double)i + 0.5;
-      }
-    }
-    dst[i * lm.es] = v;
-  }
-}
-
-// k_far: L2L down the ancestor chain and the subtree (as k_down8), the
-// subtree's local expansions at the leaf nodes on MFMA, added to the band
-// sums k_band left in the output, scaled and stored.
-struct FarLds {
-  int dl, cres, mres, qp, ob, total;
-};
-__host__ __device__ inline FarLds far_lds(const Geo &g) {
-  const int G = 1 << g.gd, s = g.s, M2 = 2 * g.M;
-  FarLds d;
-  d.dl = 0;  // D(0), D(1) with rows padded to M + 1
-  d.cres = d.dl + g.M * M2 + M2;
-  d.mres = d.cres + (2 * G - 1) * M2;
-  d.qp = d.mres + (g.ld + 2 * G - 1) * M2;
-  d.ob = d.qp + std::max(g.ld, 1) * M2;
-  d.total = d.ob + 2 * G * s + G;  // far field, slot(e) = e + e / 2s
-  return d;
-}
-size_t far_shared_bytes(const Geo &g) { return 8 * (size_t)far_lds(g).total; }
-
-template <int DIR, int MT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_far(
-    double *__restrict__ out, LineMap lm, Geo g, const double *__restrict__ wsall,
-    size_t wsstride, const double *__restrict__ Dg, const double *__restrict__ Qg,
-    const double *__restrict__ Tg) {
-  extern __shared__ double sm[];
-  const int M = MT > 0 ? MT : g.M;
-  const int s = g.s, N = g.N, M2 = 2 * M, MM = M * M;
-  const int Nl = line_len(lm, blockIdx.y, N);
-  const int G = 1 << g.gd, sh = 31 - __builtin_clz(s);
-  const int nw = s >> 4, NT = 64 * nw;
-  const int Rr = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const size_t row0 = (size_t)Rr * G * 2 * s;
-  if (row0 >= (size_t)Nl) return;
-  const int nr = (int)std::min((size_t)G * 2 * s, (size_t)Nl - row0);
-  const size_t off = line_off(lm, blockIdx.y);
-  double *dst = out + off;
+  const size_t es = lm.es;
+  double *dst = out + line_off(lm, blockIdx.y) + row0 * es;
   const double *m2l = wsall + blockIdx.y * wsstride + ws_layout(g).m2l;
   const FarLds ly = far_lds(g);
-  double *dl = sm + ly.dl, *cres = sm + ly.cres, *mres = sm + ly.mres, *qp = sm + ly.qp;
-  double *ob = sm + ly.ob;
-  auto slot = [&](int e) { return e + (e >> (sh + 1)); };
+  double *cres = sm, *mres = sm + ly.mres, *qp = sm + ly.qp, *ob = sm + ly.ob;
 
-  // ---- loads: the tree operands (M2L vectors, the chain row of Q, D), the
-  // band sums to add to (used last), T for the leaf evaluation
-  const int nm = (g.ld + 2 * G - 1) * M2;
-  constexpr int QM = 6;
-  double vm[QM];
-  bool okm[QM];
-  const int nq = g.ld * M;
-  double qr[MT > 0 ? MT : 1];
-  constexpr int QD = MT > 0 ? (2 * MT * MT + 63) / 64 : 1;
-  double vd[QD];
+  // ---- loads.  M2L vectors: slots [chain levels 0..ld-1][subtree, level by
+  // level], three slots of 18 pairs a wave; the last two chunks of a level
+  // have no M2L block.  Slot r of level lev is chunk slot slot_base(lev) + r =
+  // (B >> k) - 4 for the chain (k = ld - lev) and (B << lam) - 4 + ci for chunk
+  // ci of subtree level lam, B = slot_base(ld) + 4 + Rr.
+  const int nslot = g.ld + 2 * G - 1, sl = lane / 18, o2 = lane - 18 * sl;
+  const unsigned B = (4u << g.ld) + Rr;
+  auto slot_of = [&](int slot, bool &valid) -> size_t {
+    const int cl = slot - g.ld;
+    const int lam = cl < 0 ? cl : 31 - __builtin_clz(cl + 1);  // < 0: up the chain
+    const int ci = cl < 0 ? 0 : cl + 1 - (1 << lam);
+    const size_t c = (lam < 0 ? (size_t)(B >> -lam) : (size_t)B << lam) + ci;
+    valid = lane < 54 && slot < nslot && c < ((size_t)8 << (g.ld + lam)) - 2;
+    return c - 4;
+  };
+  constexpr int QM = 4;
+  d2 vm[QM];
 #pragma unroll
   for (int q = 0; q < QM; q++) {
-    const int e = q * NT + tid;
-    const size_t a = m2l_elem(g, Rr, e < nm ? e : 0, M2, okm[q]);
-    okm[q] = okm[q] && e < nm;
-    vm[q] = m2l[okm[q] ? a : 0];
-  }
-  if (MT > 0 && nq > 0) {
-    const double *qrow = qrow_ptr(Qg, g, Rr, tid < nq ? tid : 0, M);
-#pragma unroll
-    for (int l = 0; l < (MT > 0 ? MT : 1); l++) qr[l] = qrow[l * M];
-  }
-#pragma unroll
-  for (int q = 0; q < QD; q++) {
-    const int e = q * NT + tid;
-    vd[q] = Dg[e < 2 * MM ? e : 0];
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  // the band sums this work-group adds to, in flight through the tree pass
-  // (nr <= 2 G s <= 8 NT)
-  constexpr int QB = 8;
-  double vb[QB];
-#pragma unroll
-  for (int q = 0; q < QB; q++) {
-    const int e = q * NT + tid;
-    vb[q] = dst[(row0 + (e < nr ? e : 0)) * lm.es];
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int q = 0; q < QM; q++) {
-    const int e = q * NT + tid;
-    if (e < nm) mres[e] = okm[q] ? vm[q] : 0.0;
-  }
-  for (int e = QM * NT + tid; e < nm; e += NT) {
     bool ok;
-    const size_t a = m2l_elem(g, Rr, e, M2, ok);
-    mres[e] = ok ? m2l[a] : 0.0;
+    const size_t c = slot_of((4 * q + wave) * 3 + sl, ok);
+    const d2 v = *reinterpret_cast<const d2 *>(m2l + (ok ? c * M2 + 2 * o2 : 0));
+    vm[q].x = ok ? v.x : 0.0;
+    vm[q].y = ok ? v.y : 0.0;
   }
+  // chain rows: task (lev, k) = (task / M, task % M), half a row per thread
+  const int nq = g.ld * M, half = tid & 1;
+  double qr[9];
+  {
+    const int task = std::min(tid >> 1, std::max(nq - 1, 0));
+    const double *qrow = qrow_ptr(Qg, g, Rr, task, M) + half * 9 * M;
 #pragma unroll
-  for (int q = 0; q < QD; q++) {
-    const int e = q * NT + tid;
-    if (MT > 0 && e < 2 * MM) dl[(e / M) * (M + 1) + e % M] = vd[q];
+    for (int l = 0; l < 9; l++) qr[l] = nq > 0 ? qrow[l * M] : 0.0;
   }
-  for (int e = (MT > 0 ? QD * NT : 0) + tid; e < 2 * MM; e += NT)
-    dl[(e / M) * (M + 1) + e % M] = Dg[e];
-  lds_sync();
-
-  subtree_locals<MT, true>(g, Rr, tid, NT, mres, qp, cres, qr, nullptr, nullptr, Qg, Dg, dl,
-                           LdsSync{});
-
-  // ---- far field: F_par^T (G x s) = C_par^T (G x M) T_par^T (M x s) on
-  // v_mfma_f64_16x16x4f64, two tiles (parity, 16 rows) per wave
-  const int ntm = s >> 4, ksteps = (M + 3) >> 2;
-  constexpr int QK = MT > 0 ? (MT + 3) / 4 : 1;
-  const int n = lane & 15;
+  // D(p), rows 16 rt .. of this wave's item (p = wave / 2, rt = wave % 2)
+  const int n16 = lane & 15, kq = lane >> 4;
+  const int dp = wave >> 1, drt = wave & 1;
+  double av[5];
+#pragma unroll
+  for (int kk = 0; kk < 5; kk++) {
+    const int ra = drt * 16 + n16, k = 4 * kk + kq;
+    av[kk] = ra < M && k < M ? Dg[dp * MM + ra * M + k] : 0.0;
+  }
+  // T, rows 16 rt .. of parity sgf, for the tiles wave and wave + 4
+  const int ntm = (s + 15) >> 4;
+  double tv[2][5];
 #pragma unroll
   for (int j = 0; j < 2; j++) {
-    const int tile = wave + j * nw, sgf = tile / ntm, rt = tile - sgf * ntm;
-    d4 D = {0, 0, 0, 0};
-    if (MT > 0) {
-      double av[QK], bv[QK];
+    const int tile = wave + 4 * j, sgf = tile >= ntm, m = (tile - sgf * ntm) * 16 + n16;
 #pragma unroll
-      for (int kk = 0; kk < QK; kk++) {
-        const int k = kk * 4 + (lane >> 4);
-        bv[kk] = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
-        av[kk] = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-      }
-#pragma unroll
-      for (int kk = 0; kk < QK; kk++) D = __builtin_amdgcn_mfma_f64_16x16x4f64(av[kk], bv[kk], D, 0, 0, 0);
-    } else {
-      for (int kk = 0; kk < ksteps; kk++) {
-        const int k = kk * 4 + (lane >> 4);
-        const double bv = k < M ? Tg[((size_t)sgf * s + rt * 16 + n) * M + k] : 0.0;
-        const double av = (n < G && k < M) ? cres[(G - 1 + n) * M2 + sgf * M + k] : 0.0;
-        D = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, D, 0, 0, 0);
-      }
+    for (int kk = 0; kk < 5; kk++) {
+      const int k = 4 * kk + kq;
+      tv[j][kk] = tile < 2 * ntm && m < s && k < M ? Tg[((size_t)sgf * s + m) * M + k] : 0.0;
     }
+  }
+  // the band sums this work-group adds to (nr <= 2 G s <= 8 NT)
+  d2 vb[4];
+  if (es == 1) {
+    const __amdgpu_buffer_rsrc_t r = line_rsrc(dst, nr);
+#pragma unroll
+    for (int q = 0; q < 4; q++) vb[q] = load_pair(r, 16 * tid + 4096 * q, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * (tid + kFarNT * q);
+      vb[q].x = dst[(size_t)std::min(e, nr - 1) * es];
+      vb[q].y = dst[(size_t)std::min(e + 1, nr - 1) * es];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < QM; q++) {
+    const int slot = (4 * q + wave) * 3 + sl;
+    if (lane < 54 && slot < nslot) *reinterpret_cast<d2 *>(mres + slot * M2 + 2 * o2) = vm[q];
+  }
+  for (int s0 = (4 * QM + wave) * 3; s0 < nslot; s0 += 12) {  // (more than 48 slots)
+    bool ok;
+    const size_t c = slot_of(s0 + sl, ok);
+    if (lane < 54 && s0 + sl < nslot) {
+      const d2 z = {0.0, 0.0};
+      *reinterpret_cast<d2 *>(mres + (s0 + sl) * M2 + 2 * o2) =
+          ok ? *reinterpret_cast<const d2 *>(m2l + c * M2 + 2 * o2) : z;
+    }
+  }
+  lds_sync();
+
+  // ---- the subtree root: m2l_ld + sum_lev Q(ld - lev, .) m2l_lev
+  for (int t0 = 0; t0 < nq; t0 += kFarNT / 2) {
+    const int task = t0 + (tid >> 1);
+    if (t0 > 0) {
+      const double *qrow = qrow_ptr(Qg, g, Rr, std::min(task, nq - 1), M) + half * 9 * M;
+#pragma unroll
+      for (int l = 0; l < 9; l++) qr[l] = qrow[l * M];
+    }
+    const int lev = std::min(task, nq - 1) / M, k = std::min(task, nq - 1) - lev * M;
+    const double *mv = mres + lev * M2 + 9 * half;
+    double o0 = 0, o1 = 0;
+#pragma unroll
+    for (int l = 0; l < 9; l++) {
+      o0 += qr[l] * mv[l];
+      o1 += qr[l] * mv[M + l];
+    }
+    o0 += __shfl_xor(o0, 1, 64);
+    o1 += __shfl_xor(o1, 1, 64);
+    if (task < nq) qp[lev * M2 + half * M + k] = half ? o1 : o0;
+  }
+  lds_sync();
+  if (tid < M2) {
+    double v = mres[g.ld * M2 + tid];
+    for (int lev = 0; lev < g.ld; lev++) v += qp[lev * M2 + tid];
+    cres[tid] = v;
+  }
+  lds_sync();
+
+  // ---- levels ld+1..ld+gd on v_mfma_f64_16x16x4f64: children of parity p are
+  // C (M x n) = D(p) (M x M) C_parents (M x n), n = 2^lam children x 2
+  // parities <= 16 columns: column j = child 2(j >> 1) + p, parity j & 1
+  for (int lam = 1; lam <= g.gd; lam++) {
+    const int n = 1 << lam, b0 = n - 1, bp = (n >> 1) - 1, j = n16;
+    double bv[5], add[4];
+#pragma unroll
+    for (int kk = 0; kk < 5; kk++) {
+      const int k = 4 * kk + kq;
+      bv[kk] = j < n && k < M ? cres[(bp + (j >> 1)) * M2 + (j & 1) * M + k] : 0.0;
+    }
+    const int c = 2 * (j >> 1) + dp, o = (b0 + c) * M2 + (j & 1) * M + drt * 16 + kq;
+    const int nv = drt == 0 ? 4 : (kq < M - 16 ? 1 : 0);  // rows drt 16 + kq + 4 v < M
+#pragma unroll
+    for (int v = 0; v < 4; v++) add[v] = j < n && v < nv ? mres[g.ld * M2 + o + 4 * v] : 0.0;
+    d4 D0 = {0, 0, 0, 0}, D1 = {0, 0, 0, 0};
+    D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0], bv[0], D0, 0, 0, 0);
+    D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1], bv[1], D1, 0, 0, 0);
+    D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[2], bv[2], D0, 0, 0, 0);
+    D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[3], bv[3], D1, 0, 0, 0);
+    D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[4], bv[4], D0, 0, 0, 0);
+    D0 += D1;
+    const bool valid = ((size_t)Rr << lam) + c < ((size_t)4 << (g.ld + lam)) - 2;
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (j < n && v < nv) cres[o + 4 * v] = valid ? D0[v] + add[v] : 0.0;
+    lds_sync();
+  }
+
+  // ---- far field F_par^T (G x s) = C_par^T (G x M) T_par^T (M x s)
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const int tile = wave + 4 * t, sgf = tile >= ntm, rt = tile - sgf * ntm;
+    if (tile >= 2 * ntm) continue;
+    double cv[5];
+#pragma unroll
+    for (int kk = 0; kk < 5; kk++) {
+      const int k = 4 * kk + kq;
+      cv[kk] = n16 < G && k < M ? cres[(G - 1 + n16) * M2 + sgf * M + k] : 0.0;
+    }
+    d4 D = {0, 0, 0, 0};
+#pragma unroll
+    for (int kk = 0; kk < 5; kk++) D = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[kk], tv[t][kk], D, 0, 0, 0);
+    const int m = rt * 16 + n16;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const int leaf = (lane >> 4) + 4 * v, m = rt * 16 + n;
-      const int e = 2 * (leaf * s + m) + sgf;
-      if (leaf < G && e < nr) ob[slot(e)] = D[v];
+      const int leaf = kq + 4 * v;
+      if (leaf < G && m < s) ob[leaf * ly.CS + 2 * m + sgf] = D[v];
     }
   }
   lds_sync();
   // ---- the band sums plus the far field, scaled
-#pragma unroll
-  for (int q = 0; q < QB; q++) {
-    const int e = q * NT + tid;
-    if (e >= nr) continue;
+  const unsigned inv = ((1u << 20) + s - 1) / s;
+  const bool even = (s & 1) == 0;
+  auto scaled = [&](double v, int e) {
     const size_t i = row0 + e;
-    double v = vb[q] + ob[slot(e)];
-    if (DIR == 0) {
-      v *= k2Pi;
-      if (i == 0) v *= 0.5;
+    if (dir == C2L) return v * ((double)i + 0.5);
+    return i == 0 ? v * k2Pi * 0.5 : v * k2Pi;
+  };
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int h = tid + kFarNT * q, e = 2 * h;
+    if (e >= nr) continue;
+    const double *o = ob + e + (even ? 2 * (int)(__umul24(h, inv) >> 20) : 0);
+    const d2 v = {scaled(vb[q].x + o[0], e), scaled(vb[q].y + o[1], e + 1)};
+    if (es == 1) {
+      store_pair(v, line_rsrc(dst, nr), 16 * h);
     } else {
-      v *= (double)i + 0.5;
+      dst[(size_t)e * es] = v.x;
+      if (e + 1 < nr) dst[(size_t)(e + 1) * es] = v.y;
     }
-    dst[i * lm.es] = v;
   }
 }
 
@@ -2757,28 +3133,6 @@ __global__ void __launch_bounds__(256) k_direct_band(const double *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// two doubles at any 8-byte boundary, moved as one 16-byte access
-typedef double d2 __attribute__((ext_vector_type(2)));
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
-typedef unsigned u4 __attribute__((ext_vector_type(4)));
-// Buffer descriptor of n doubles at p (both wave-uniform): raw buffer loads
-// check each dword against the length and return zero past it.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t line_rsrc(const double *p, int n) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 8 * n, 0x00020000);
-}
-__device__ __forceinline__ double load_one(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-}
-// The two doubles at byte voff (per lane) + soff (uniform) of the buffer.
-__device__ __forceinline__ d2 load_pair(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return __builtin_bit_cast(d2, v);
-}
-
-__device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int voff) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
-}
-
 // Batched lines of the direct path (N <= kDenseMaxN) as dense products on FP64
 // MFMA: per parity p, OUT_p (NPP x LT) = K_p (NPP x NPP) IN_p (NPP x LT) for a
 // tile of LT lines, K_p upper triangular (the direct sums of
@@ -3400,10 +3754,9 @@ static int ensure_ws(fmm_plan_s *p, size_t nlines, const Geo &g, double **w) {
   return 0;
 }
 
-// k_down8 launch in the given mode on stream st
-template <int MT>
+// k_down8r or k_down8 launch on stream st
 static void launch_down8(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out, size_t dir,
-                         const LineMap &lm, size_t nlines, hipStream_t st, int mode, double *ws) {
+                         const LineMap &lm, size_t nlines, hipStream_t st, double *ws) {
   const size_t wsstride = ws_doubles(g);
   dim3 gd((unsigned)((size_t)4 << g.ld), (unsigned)nlines);
   const size_t shm = down_shared_bytes(g);
@@ -3411,75 +3764,61 @@ static void launch_down8(fmm_plan_s *p, const Geo &g, const double *d_in, double
   const double *tab = dir == L2C ? p->t.a : p->t.an;
   const double *htab = p->t.head[dir];
   prof_begin(p->prof, K_DOWN_BAND, st);
-  if (mode == K8_FULL && p->down_roles) {
+  if (p->down_roles) {
     const size_t shr = down8r_shared_bytes(g);
     const int rsh = std::max(-g.s, std::min(p->roles_shift, 8 * (g.s >> 4))) & ~7;
     if (dir == L2C)
-      launch_k(p->prof, k_down8r<0, 0, MT>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
+      launch_k(p->prof, k_down8r<0, 0>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
           p->t.D, p->t.Q, p->t.T, tab, htab, rsh);
     else if (p->precompute)
-      launch_k(p->prof, k_down8r<1, 1, MT>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
+      launch_k(p->prof, k_down8r<1, 1>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
           p->t.D, p->t.Q, p->t.T, tab, htab, rsh);
     else
-      launch_k(p->prof, k_down8r<1, 0, MT>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
+      launch_k(p->prof, k_down8r<1, 0>, gd, 2 * nt, shr, st, d_in, d_out, lm, g, ws, wsstride,
           p->t.D, p->t.Q, p->t.T, tab, htab, rsh);
   } else if (dir == L2C)
-    launch_k(p->prof, k_down8<0, 0, MT>, gd, nt, shm, st, d_in, d_out, lm, g, mode, ws, wsstride,
+    launch_k(p->prof, k_down8<0, 0>, gd, nt, shm, st, d_in, d_out, lm, g, ws, wsstride,
         p->t.D, p->t.Q, p->t.T, tab, htab);
   else if (p->precompute)
-    launch_k(p->prof, k_down8<1, 1, MT>, gd, nt, shm, st, d_in, d_out, lm, g, mode, ws, wsstride,
+    launch_k(p->prof, k_down8<1, 1>, gd, nt, shm, st, d_in, d_out, lm, g, ws, wsstride,
         p->t.D, p->t.Q, p->t.T, tab, htab);
   else
-    launch_k(p->prof, k_down8<1, 0, MT>, gd, nt, shm, st, d_in, d_out, lm, g, mode, ws, wsstride,
+    launch_k(p->prof, k_down8<1, 0>, gd, nt, shm, st, d_in, d_out, lm, g, ws, wsstride,
         p->t.D, p->t.Q, p->t.T, tab, htab);
   prof_end(p->prof, st);
 }
 
 // The split downward pass on st: k_band (before the tree kernels, which it
 // does not need), then k_up and k_m2l, then k_far.
-template <int MT>
 static void launch_band(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out, size_t dir,
-                        const LineMap &lm, size_t nlines, hipStream_t st, int scale) {
-  dim3 gd((unsigned)((size_t)4 << g.ld), (unsigned)nlines);
-  const size_t shm = band_shared_bytes(g);
-  const int nt = 128 * (g.s >> 4);
-  const double *tab = dir == L2C ? p->t.a : p->t.an;
-  const double *htab = p->t.head[dir];
-  prof_begin(p->prof, K_BAND, st);
-  if (dir == L2C)
-    launch_k(p->prof, k_band<0, 0>, gd, nt, shm, st, d_in, d_out, lm, g, scale, tab, htab);
-  else if (p->precompute)
-    launch_k(p->prof, k_band<1, 1>, gd, nt, shm, st, d_in, d_out, lm, g, scale, tab, htab);
-  else
-    launch_k(p->prof, k_band<1, 0>, gd, nt, shm, st, d_in, d_out, lm, g, scale, tab, htab);
+                        const LineMap &lm, size_t nlines, hipStream_t st, int scale, int slot) {
+  prof_begin(p->prof, slot, st);
+  launch_k(p->prof, (g.s & 15) == 0 ? k_band<true> : k_band<false>,
+           dim3(band_groups(g), (unsigned)nlines), kBandNT, band_shared_bytes(g), st, d_in, d_out,
+           lm, g, (int)dir, scale, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
   prof_end(p->prof, st);
 }
 
-template <int MT>
 static void launch_far(fmm_plan_s *p, const Geo &g, double *d_out, size_t dir, const LineMap &lm,
-                       size_t nlines, hipStream_t st, double *ws) {
-  dim3 gd((unsigned)((size_t)4 << g.ld), (unsigned)nlines);
-  const int nt = 64 * (g.s >> 4);
-  prof_begin(p->prof, K_FAR, st);
-  if (dir == L2C)
-    launch_k(p->prof, k_far<0, MT>, gd, nt, far_shared_bytes(g), st, d_out, lm, g, ws,
-        ws_doubles(g), p->t.D, p->t.Q, p->t.T);
-  else
-    launch_k(p->prof, k_far<1, MT>, gd, nt, far_shared_bytes(g), st, d_out, lm, g, ws,
-        ws_doubles(g), p->t.D, p->t.Q, p->t.T);
+                       size_t nlines, hipStream_t st, double *ws, int slot) {
+  prof_begin(p->prof, slot, st);
+  launch_k(p->prof, k_far, dim3((unsigned)((size_t)4 << g.ld), (unsigned)nlines), kFarNT,
+           far_shared_bytes(g), st, d_out, lm, g, (int)dir, ws, ws_doubles(g), p->t.D, p->t.Q,
+           p->t.T);
   prof_end(p->prof, st);
 }
 
-// Whether this call takes the split downward pass (k_band + k_far): always
-// (down_split 1), never (0, the default), or (2) for calls of several lines
-// of deep trees (L >= 10, N >= 2^18 at s = 64).  Against k_down8 the split
-// pass wins on such line calls (8 lines of 2^20 in 293 us against 315 us,
-// 32 lines in 1017 against 1116 us) and loses on single lines (58 against
-// 56 us at 2^20); k_down8r beats both (8 lines 286 us, 32 lines 1187
-// against 1230 us for the split pass in the same run, one line 48.6 us).
+// The downward pass of a far plan (geo.far): the band inside the k_up launch,
+// then k_far; or (down_split 1, and 2 for line calls with L >= 10) a k_band
+// launch of its own before k_up.  Per call, s = 64, k_down8r / k_band apart /
+// band in the k_up launch (us): one line of 2^11 20.1 / 23.2 / 17.7, 2^16 21.8 /
+// 25.5 / 19.3, 2^20 45.1 / 49.7 / 44.2; 16 lines of 2^13 23.6 / 26.7 / 20.3;
+// 128 of 2^15 117 / 112 / 104; 64 of 2^18 423 / 387 / 372 (k_down8r: band and
+// far field in one work-group of 16 waves, now for other ranks than 18).  The
+// band apart wins only below what a call of plain lines reaches (256 lines of
+// 2^11 36.9 / 45.5); the batch tuner times both.
 static bool use_split(const fmm_plan_s *p, size_t nlines) {
-  return p->geo.fast &&
-         (p->down_split == 1 || (p->down_split == 2 && nlines > 1 && p->geo.L >= 10));
+  return p->down_split == 1 || (p->down_split == 2 && nlines > 1 && p->geo.L >= 10);
 }
 
 // One execute (or a batch of lines): upward pass, M2L, downward pass, all on st.
@@ -3488,29 +3827,33 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
                         size_t dir, const LineMap &lm, size_t nlines, hipStream_t st,
                         int band_only, double *ws) {
   const size_t wsstride = ws_doubles(g);
-  if (lm.n && !g.fast) {  // per-line lengths: k_up and k_down8 only
-    set_error("lines of uneven length need a plan with leaf size s = 16, 32 or 64");
+  if (lm.n && !g.fast && !g.far) {  // per-line lengths: not in k_down
+    set_error("lines of uneven length need a plan with leaf size s <= 64");
     return -1;
   }
-  const bool split = use_split(p, nlines);
-  if (split) {
-    launch_band<MT>(p, g, d_in, d_out, dir, lm, nlines, st, band_only);
-    if (band_only) return 0;
+  if (band_only && g.s <= kBandMaxS) {  // directM
+    launch_band(p, g, d_in, d_out, dir, lm, nlines, st, 1, K_DOWN_BAND);
+    return 0;
   }
+  const bool split = g.far && use_split(p, nlines), fuse = g.far && !split;
+  if (split) launch_band(p, g, d_in, d_out, dir, lm, nlines, st, 0, K_BAND);
   if (!band_only) {
-    dim3 gu((unsigned)((size_t)4 << g.lu), (unsigned)nlines);
+    const bool s16 = (g.s & 15) == 0;
+    dim3 gu(4u << g.lu, (unsigned)nlines);
+    if (fuse) gu = dim3(std::max(gu.x, band_groups(g)), gu.y, 2);
+    const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]};
     prof_begin(p->prof, K_UP_SUBTREE, st);
-    // subtree levels on MFMA for deep subtrees of calls of up to 8 lines
-    // (latency-bound: 2^20 47.86 -> 47.31 us per transform, 8 lines of 2^20
-    // 248.5 -> 246.0 us); at 2^2 chunks (2^16) and for calls of 32 lines and
-    // more (throughput-bound: 32 lines of 2^18 234.9 -> 236.8 us) the VALU
-    // levels are as fast or faster
-    if (MT > 0 && g.gu >= 3 && nlines <= 8)
-      launch_k(p->prof, k_up<MT, MT != 0>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g, (int)dir,
-               p->t.T, p->t.U, p->t.P, ws, wsstride);
-    else
-      launch_k(p->prof, k_up<MT, false>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g, (int)dir,
-               p->t.T, p->t.U, p->t.P, ws, wsstride);
+    if (MT == 18 && up18_eligible(g)) {
+      const size_t shu = std::max(8 * (size_t)up18_lds(g).total, fuse ? band_shared_bytes(g) : 0);
+      launch_k(p->prof, s16 ? k_up<true> : k_up<false>, gu, kUpNT, shu, st, d_in, lm, g, (int)dir,
+               p->t.T, p->t.U, p->t.P, ws, wsstride, bu);
+    } else if (MT > 0 && g.gu >= 3 && nlines <= 8) {
+      launch_k(p->prof, k_up_any<MT, MT != 0>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g,
+               (int)dir, p->t.T, p->t.U, p->t.P, ws, wsstride);
+    } else {
+      launch_k(p->prof, k_up_any<MT, false>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g,
+               (int)dir, p->t.T, p->t.U, p->t.P, ws, wsstride);
+    }
     prof_end(p->prof, st);
     const int ntop = (int)total_blocks(g.lu), ntot = (int)total_blocks(g.L);
     const int bpw = m2l_bpw(g);
@@ -3529,8 +3872,8 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
       // the same grid; the blocks below lu from At, with the LDS of one
       // staged block (the top blocks') per work-group instead of four
       launch_k(p->prof, k_m2l_t<MT == 18 ? 18 : 1>, gm, kM2lNT,
-          8 * (size_t)(m2l_wave_lds(g.M) + kM2lNT), st, g, p->t.A[dir], p->t.At[dir], ws,
-          wsstride, nlines, lpb);
+               8 * (size_t)(m2l_wave_lds(g.M) + kM2lNT), st, g, p->t.A[dir], p->t.At[dir], ws,
+               wsstride, nlines, lpb);
     } else if (!mma) {
       launch_k(p->prof, k_m2l<MT>, gm, kM2lNT, m2l_shared_bytes(g), st, g, p->t.A[dir], ws,
           wsstride, bpw, nlines, lpb, sv);
@@ -3558,12 +3901,12 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
     }
     prof_end(p->prof, st);
   }
-  if (split) {
-    launch_far<MT>(p, g, d_out, dir, lm, nlines, st, ws);
+  if (g.far) {
+    launch_far(p, g, d_out, dir, lm, nlines, st, ws, fuse ? K_DOWN_BAND : K_FAR);
     return 0;
   }
   if (g.fast) {
-    launch_down8<MT>(p, g, d_in, d_out, dir, lm, nlines, st, band_only ? K8_BAND : K8_FULL, ws);
+    launch_down8(p, g, d_in, d_out, dir, lm, nlines, st, ws);
     return 0;
   }
   dim3 gd((unsigned)((size_t)4 << g.ld), (unsigned)nlines);

@@ -154,7 +154,8 @@ struct Geo {
   int gu, lu;  // upward work-group: 2^gu leaf chunks; cut level lu = L-1-gu
   int gd, ld;  // downward work-group: 2^gd leaf chunks; cut level ld = L-1-gd
   int nodal;   // 1: Lagrange basis (lagrange=1), 0: Chebyshev basis
-  int fast;    // 1: downward pass by k_down8 (s = 16, 32 or 64)
+  int fast;    // 1: s = 16, 32 or 64: downward pass by k_down8(r) if not far
+  int far;     // 1: near field by band groups, downward pass by k_far (M = 18, s <= 64)
 };
 
 struct DevTables {
@@ -172,8 +173,10 @@ struct DevTables {
   double *P = nullptr;   // composite upward operators for the top levels
   double *Q = nullptr;   // composite downward operators for the ancestor chain
   // band head per direction: Lambda(k) (L2C) or dn(k) (C2L) for k < min(2s,
-  // table length), zero up to 2s + 16
+  // table length), zero up to 2s + 16; head points into band_head, which holds
+  // 16 zeros before it and more after
   double *head[2] = {nullptr, nullptr};
+  double *band_head[2] = {nullptr, nullptr};
   // Split form of the M2L matrices (precision form 1), per direction: every
   // block (its three M x M submatrices, 3 M^2 coefficients) is one record of
   // rec_bytes: the coefficients of storage tier FP64 (n64), then FP32 (n32),
@@ -281,11 +284,12 @@ struct fmm_plan_s {
   // 4096 transforms 14.0 -> 14.9 M/s, while 8 lines of 2^20 lose 244 -> 259
   // us); L2C_M2L_MMA sets it at plan creation
   int m2l_mma_lines = 32;
-  // downward pass of s = 16/32/64 plans: 0 (default) one fused kernel, 1
-  // k_band + k_far, 2 k_band + k_far for calls of several lines with L >= 10;
-  // L2C_DOWN_SPLIT
+  // near field of plans with M = 18 and s <= 64: 0 (default) work-groups of the
+  // k_up launch, 1 a k_band launch of its own, 2 that for calls of several
+  // lines with L >= 10; L2C_DOWN_SPLIT
   int down_split = 0;
-  // the fused downward pass with wave roles (k_down8r: tree and far field on
+  // the downward pass of other ranks at s = 16, 32, 64 with wave roles
+  // (k_down8r: tree and far field on
   // half the waves, the band on the other half; default) or without (0:
   // k_down8); L2C_DOWN_ROLES
   int down_roles = 1;
@@ -392,6 +396,7 @@ size_t down_shared_bytes(const Geo &g);  // of the downward kernel g selects
 size_t band_shared_bytes(const Geo &g);
 size_t far_shared_bytes(const Geo &g);
 bool down8_eligible(const Geo &g);
+bool far_eligible(const Geo &g);
 size_t up_shared_bytes(const Geo &g);
 size_t ws_doubles(const Geo &g);  // execute workspace per line
 size_t flops_direct(size_t N, size_t dir, size_t precompute);

@@ -538,8 +538,8 @@ static void destroy_fmm(fmm_plan_s *p) {
   dfree(p->t.D);
   dfree(p->t.P);
   dfree(p->t.Q);
-  dfree(p->t.head[0]);
-  dfree(p->t.head[1]);
+  dfree(p->t.band_head[0]);
+  dfree(p->t.band_head[1]);
   dfree(p->d_K[0]);
   dfree(p->d_K[1]);
   dfree(p->d_w);
@@ -564,28 +564,31 @@ static void destroy_fmm(fmm_plan_s *p) {
 // single: the cuts of single-line calls, else those of line calls.  Line
 // calls (their grids hold every line's work-groups) take the largest
 // subtrees; single transforms take cuts that grow with the depth, gu = gd =
-// (L - 4) / 2 within [1, 4] (gd >= 2 for k_down8r), measured best at
+// (L - 4) / 2 within [1, 4] (gd >= 2 for k_far and k_down8r), measured best at
 // L = 4 ... 12 (s = 64: 2^16 23.1 us at (2, 2) against 26.8 us at (4, 4);
 // 2^18 26.6 against 28.6 us at (3, 3); 2^20 (4, 4) best), while line calls
 // lose with them (64 lines of 2^16: 174 K against 432 K lines/s).
 static bool choose_cuts(Geo &g, bool single) {
   const int Lm1 = g.L - 1;
-  // k_down8 (s = 16, 32, 64; L2C_DOWN8=0 selects k_down): 16 leaf chunks and
-  // up to 80 KiB of LDS (two work-groups per CU); k_down: 8 and 64 KiB
+  // k_far (M = 18, s <= 64) and k_down8 (s = 16, 32, 64): 16 leaf chunks and
+  // up to 80 KiB of LDS (two work-groups per CU); k_down (other plans, and
+  // L2C_DOWN8=0): 8 and 64 KiB
   const char *e8 = getenv("L2C_DOWN8");
   g.fast = down8_eligible(g) && !(e8 && atoi(e8) == 0) ? 1 : 0;
+  g.far = far_eligible(g) && !(e8 && atoi(e8) == 0) ? 1 : 0;
+  const bool wide = g.fast || g.far;  // 16 leaf chunks per downward work-group
   const int dcut = (g.L - 4) / 2;
-  int gu = 4, gd = g.fast ? 4 : 3;
+  int gu = 4, gd = wide ? 4 : 3;
   if (single) {
     gu = std::max(1, std::min(4, dcut));
-    if (g.fast) gd = std::max(2, std::min(4, dcut));
+    if (wide) gd = std::max(2, std::min(4, dcut));
   }
   if (const char *e = getenv("L2C_GU")) gu = atoi(e);
   if (const char *e = getenv("L2C_GD")) gd = atoi(e);
   // k_up holds its composite operators in LDS (lu of them): up to 80 KiB
-  const size_t budget = 80 * 1024, dbudget = (g.fast ? 80 : 64) * 1024;
+  const size_t budget = 80 * 1024, dbudget = (wide ? 80 : 64) * 1024;
   g.gu = std::max(0, std::min(std::min(gu, 4), Lm1));  // k_up: at most 16 leaf chunks
-  g.gd = std::max(0, std::min(std::min(gd, g.fast ? 4 : Lm1), Lm1));
+  g.gd = std::max(0, std::min(std::min(gd, wide ? 4 : Lm1), Lm1));
   for (;;) {
     g.lu = Lm1 - g.gu;
     g.ld = Lm1 - g.gd;
@@ -704,12 +707,15 @@ fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, s
   // band heads, read as uniform (scalar) loads by the band loop
   for (int d = 0; d < 2; d++) {
     if ((d == 0 && !l2c) || (d == 1 && !c2l)) continue;
-    const size_t nhd = 2 * s + 16, nh = std::min(2 * s, d == 0 ? N : (N + 1) / 2);
-    if (dmalloc(&p->t.head[d], nhd, acct)) {
+    // (16 zeros before it and past 2s + 16 as well: k_band reads whole trips)
+    const size_t nhd = 16 + 2 * s + 64, nh = std::min(2 * s, d == 0 ? N : (N + 1) / 2);
+    if (dmalloc(&p->t.band_head[d], nhd, acct)) {
       destroy_fmm(p);
       return nullptr;
     }
-    L2C_HIP(hipMemsetAsync(p->t.head[d], 0, nhd * sizeof(double), st), (destroy_fmm(p), nullptr));
+    p->t.head[d] = p->t.band_head[d] + 16;
+    L2C_HIP(hipMemsetAsync(p->t.band_head[d], 0, nhd * sizeof(double), st),
+            (destroy_fmm(p), nullptr));
     L2C_HIP(hipMemcpyAsync(p->t.head[d], d == 0 ? p->t.a : p->t.dn, nh * sizeof(double),
                            hipMemcpyDeviceToDevice, st),
             (destroy_fmm(p), nullptr));
