@@ -69,13 +69,26 @@ static void prof_harvest(Prof *pf) {
 // ---------------------------------------------------------------------------
 // The reference's flop count (the return value of execute), same formulas:
 // src/C/leg2cheb.c:1383, 1398, 1415, 1435, 1447, 1463, 1469 and the band
-// counters of directM/directL (:236-535) and direct (:152-234).
+// counters of directM/directL (:236-535) and direct (:152-234), their loops
+// over rows and blocks summed (as loops they took 120 us of a host call at
+// N = 200,000).
+// sum of N - n over the even offsets n0, n0 + 2, ... < N
+static size_t even_tails(size_t n0, size_t N) {
+  if (n0 >= N) return 0;
+  const size_t c = (N - n0 + 1) / 2;
+  return c * (N - n0) - c * (c - 1);
+}
+
 size_t flops_direct(size_t N, size_t dir, size_t pre) {
-  size_t f = N;
-  const size_t per = pre ? 2 : 3;
-  for (size_t n = dir == L2C ? 0 : 2; n < N; n += 2) f += per * (N - n);
-  f += N;
-  return f;
+  const size_t per = pre ? 2 : 3, n0 = dir == L2C ? 0 : 2;
+  return 2 * N + per * even_tails(n0, N);
+}
+
+// The near-field band: every block but the last has the same rows.
+static size_t flops_blocks(size_t nL, size_t n0, size_t h, size_t per) {
+  size_t f = 0;
+  for (size_t n = n0; n < 2 * h; n += 2) f += per * (n < h ? h : 2 * h - n);
+  return nL > 1 ? (nL - 1) * f : 0;
 }
 
 size_t flops_fmm(const fmm_plan_s *p, size_t dir) {
@@ -94,15 +107,9 @@ size_t flops_fmm(const fmm_plan_s *p, size_t dir) {
   const size_t h = 2 * s, nL = N / h;
   const size_t per = p->precompute ? 2 : 3;
   if (dir == L2C) {
-    for (size_t b = 0; b + 1 < nL; b++)
-      for (size_t n = 0; n < 4 * s; n += 2) f += per * (n < h ? h : 2 * h - n);
-    const size_t i0 = (nL - 1) * h;
-    for (size_t n = 0; 2 * n + i0 < N; n++) f += per * (N - (2 * n + i0));
-    f += N;
+    f += flops_blocks(nL, 0, h, per) + per * even_tails((nL - 1) * h, N) + N;
   } else {
-    f += 3 * N;
-    for (size_t b = 0; b + 1 < nL; b++)
-      for (size_t n = 2; n < 4 * s; n += 2) f += per * (n < h ? h : 2 * h - n);
+    f += 3 * N + flops_blocks(nL, 2, h, per);
     // last block: the reference's size_t terms sum to zero modulo 2^64
     f += 2 * N;
   }
@@ -201,25 +208,105 @@ static bool dir_planned(const fmm_plan_s *p, size_t dir) {
 }
 
 // Host staging buffers (device copy and pinned host copy of N doubles each
-// way), allocated on the first call with host arrays and kept by the plan.
-static int ensure_staging(size_t N, double **din, double **dout, double **hin, double **hout) {
-  if (*din && *dout && *hin && *hout) return 0;
-  double *a = nullptr, *b = nullptr, *c = nullptr, *d = nullptr;
-  if (hipMalloc((void **)&a, N * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&b, N * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&c, N * sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void **)&d, N * sizeof(double)) != hipSuccess) {
-    if (a) (void)hipFree(a);
-    if (b) (void)hipFree(b);
-    if (c) (void)hipHostFree(c);
-    if (d) (void)hipHostFree(d);
+// way) and the events of the copy back, made on the first call with host
+// arrays and kept by the plan.  The pinned copies are coherent: kernels read
+// and write them, which must not leave old lines in the GPU's caches.
+static int ensure_staging(size_t N, HostStage &h) {
+  if (h.d_in) return 0;
+  HostStage n;
+  bool ok = hipMalloc((void **)&n.d_in, N * sizeof(double)) == hipSuccess &&
+            hipMalloc((void **)&n.d_out, N * sizeof(double)) == hipSuccess &&
+            hipHostMalloc((void **)&n.h_in, N * sizeof(double), hipHostMallocCoherent) ==
+                hipSuccess &&
+            hipHostMalloc((void **)&n.h_out, N * sizeof(double), hipHostMallocCoherent) ==
+                hipSuccess;
+  for (size_t c = 0; ok && c < host_chunks(N); c++)
+    ok = hipEventCreateWithFlags(&n.ev[c], hipEventDisableTiming | hipEventReleaseToSystem) ==
+         hipSuccess;
+  if (!ok) {
+    free_staging(n);
     set_error("host staging allocation failed");
     return -1;
   }
-  *din = a;
-  *dout = b;
-  *hin = c;
-  *hout = d;
+  h = n;
+  return 0;
+}
+
+void free_staging(HostStage &h) {
+  if (h.d_in) (void)hipFree(h.d_in);
+  if (h.d_out) (void)hipFree(h.d_out);
+  if (h.h_in) (void)hipHostFree(h.h_in);
+  if (h.h_out) (void)hipHostFree(h.h_out);
+  for (auto &e : h.ev)
+    if (e) (void)hipEventDestroy(e);
+  h = HostStage();
+}
+
+// Host arrays to the device and back, through the pinned copies in up to
+// kHostChunks chunks of 65,536 elements and more, so that the CPU copies one
+// chunk while the link carries another.  The transfers are kernels, not
+// hipMemcpyAsync: at 160 KB and more that takes the copy engine, and the
+// hand-over between it and the compute queue costs more than the kernel does.
+// Transfers both ways and a device copy between them, us: 20,000 elements 33 by
+// hipMemcpyAsync, 21 by kernels.  CPU copies and transfers, us: 200,000 elements
+// in one chunk 82 in and 87 out, in four 59 and 61 (eight 66 and 78); 1,000,000
+// in one 285 and 409, in eight 219 and 233.  Bound by the link (1.6 MB in 36
+// us) and the CPU's copies of what does not fit its caches.  A call of 200,000
+// elements 312 -> 214 us with the flop counts above in closed form.
+__global__ void __launch_bounds__(256) k_host_copy(double *__restrict__ dst,
+                                                   const double *__restrict__ src, size_t n) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  for (size_t i = t; i < n / 2; i += (size_t)gridDim.x * 256)
+    reinterpret_cast<d2 *>(dst)[i] = reinterpret_cast<const d2 *>(src)[i];
+  if (t == 0 && (n & 1)) dst[n - 1] = src[n - 1];
+}
+
+// elements per chunk, even: every chunk starts on 16 bytes
+static size_t host_chunk(size_t N) {
+  const size_t c = (N + host_chunks(N) - 1) / host_chunks(N);
+  return c + (c & 1);
+}
+
+static void launch_host_copy(double *dst, const double *src, size_t n, hipStream_t st) {
+  const unsigned grid = (unsigned)std::min<size_t>((n / 2 + 256) / 256, 256);
+  k_host_copy<<<grid, 256, 0, st>>>(dst, src, n);
+}
+
+static int stage_in(HostStage &h, const double *in, size_t stride, size_t N, hipStream_t st) {
+  const size_t c = host_chunk(N);
+  for (size_t o = 0; o < N; o += c) {
+    const size_t n = std::min(c, N - o);
+    if (stride == 1)
+      std::memcpy(h.h_in + o, in + o, n * sizeof(double));
+    else
+      for (size_t i = o; i < o + n; i++) h.h_in[i] = in[i * stride];
+    launch_host_copy(h.d_in + o, h.h_in + o, n, st);
+  }
+  L2C_HIP(hipGetLastError(), -1);
+  return 0;
+}
+
+static int stage_out(HostStage &h, double *out, size_t stride, size_t N, hipStream_t st) {
+  const size_t c = host_chunk(N);
+  size_t k = 0;
+  for (size_t o = 0; o < N; o += c, k++) {
+    launch_host_copy(h.h_out + o, h.d_out + o, std::min(c, N - o), st);
+    if (c < N) L2C_HIP(hipEventRecord(h.ev[k], st), -1);
+  }
+  L2C_HIP(hipGetLastError(), -1);
+  k = 0;
+  for (size_t o = 0; o < N; o += c, k++) {
+    const size_t n = std::min(c, N - o);
+    if (o + c < N)
+      L2C_HIP(hipEventSynchronize(h.ev[k]), -1);
+    else
+      L2C_HIP(hipStreamSynchronize(st), -1);
+    if (stride == 1)
+      std::memcpy(out + o, h.h_out + o, n * sizeof(double));
+    else
+      for (size_t i = o; i < o + n; i++) out[i * stride] = h.h_out[i];
+  }
   return 0;
 }
 
@@ -260,22 +347,11 @@ size_t execute(const double *input_array, double *output_array, fmm_plan *p, siz
     if (rc) return (size_t)-1;
     L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
   } else {
-    direct_plan_s *dq = p->dplan;
-    if (p->L == 0 ? ensure_staging(N, &dq->d_in, &dq->d_out, &dq->h_in, &dq->h_out)
-                  : ensure_staging(N, &p->d_in, &p->d_out, &p->h_in, &p->h_out))
-      return (size_t)-1;
-    double *hin = p->L == 0 ? dq->h_in : p->h_in;
-    double *hout = p->L == 0 ? dq->h_out : p->h_out;
-    double *din = p->L == 0 ? dq->d_in : p->d_in;
-    double *dout = p->L == 0 ? dq->d_out : p->d_out;
-    for (size_t i = 0; i < N; i++) hin[i] = input_array[i * stride];
-    L2C_HIP(hipMemcpyAsync(din, hin, N * sizeof(double), hipMemcpyHostToDevice, st), (size_t)-1);
-    rc = p->L == 0 ? run_direct(p->dplan, din, dout, direction, 1, st, p->precompute)
-                   : run_fmm(p, din, dout, direction, 1, st, 0);
-    if (rc) return (size_t)-1;
-    L2C_HIP(hipMemcpyAsync(hout, dout, N * sizeof(double), hipMemcpyDeviceToHost, st), (size_t)-1);
-    L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
-    for (size_t i = 0; i < N; i++) output_array[i * stride] = hout[i];
+    HostStage &h = p->L == 0 ? p->dplan->host : p->host;
+    if (ensure_staging(N, h) || stage_in(h, input_array, stride, N, st)) return (size_t)-1;
+    rc = p->L == 0 ? run_direct(p->dplan, h.d_in, h.d_out, direction, 1, st, p->precompute)
+                   : run_fmm(p, h.d_in, h.d_out, direction, 1, st, 0);
+    if (rc || stage_out(h, output_array, stride, N, st)) return (size_t)-1;
   }
   return flops_fmm(p, direction);
 }
@@ -294,22 +370,14 @@ size_t directM(const double *input_array, double *output_array, fmm_plan *p, con
     if (run_fmm(p, input_array, output_array, L2C, strides, st, 1)) return (size_t)-1;
     L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
   } else {
-    if (ensure_staging(N, &p->d_in, &p->d_out, &p->h_in, &p->h_out)) return (size_t)-1;
-    for (size_t i = 0; i < N; i++) p->h_in[i] = input_array[i * strides];
-    L2C_HIP(hipMemcpyAsync(p->d_in, p->h_in, N * 8, hipMemcpyHostToDevice, st), (size_t)-1);
-    if (run_fmm(p, p->d_in, p->d_out, L2C, 1, st, 1)) return (size_t)-1;
-    L2C_HIP(hipMemcpyAsync(p->h_out, p->d_out, N * 8, hipMemcpyDeviceToHost, st), (size_t)-1);
-    L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
-    for (size_t i = 0; i < N; i++) output_array[i * strides] = p->h_out[i];
+    HostStage &h = p->host;
+    if (ensure_staging(N, h) || stage_in(h, input_array, strides, N, st) ||
+        run_fmm(p, h.d_in, h.d_out, L2C, 1, st, 1) || stage_out(h, output_array, strides, N, st))
+      return (size_t)-1;
   }
   // band flops only (src/C/leg2cheb.c:236-376)
   const size_t s = p->s, h = 2 * s, nL = N / h, per = p->precompute ? 2 : 3;
-  size_t f = 0;
-  for (size_t b = 0; b + 1 < nL; b++)
-    for (size_t n = 0; n < 4 * s; n += 2) f += per * (n < h ? h : 2 * h - n);
-  const size_t i0 = (nL - 1) * h;
-  for (size_t n = 0; 2 * n + i0 < N; n++) f += per * (N - (2 * n + i0));
-  return f + N;
+  return flops_blocks(nL, 0, h, per) + per * even_tails((nL - 1) * h, N) + N;
 }
 
 size_t direct(const double *input_array, double *output_array, direct_plan *dp, size_t direction,
@@ -332,13 +400,11 @@ size_t direct(const double *input_array, double *output_array, direct_plan *dp, 
       return (size_t)-1;
     L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
   } else {
-    if (ensure_staging(N, &dp->d_in, &dp->d_out, &dp->h_in, &dp->h_out)) return (size_t)-1;
-    for (size_t i = 0; i < N; i++) dp->h_in[i] = input_array[i * stride];
-    L2C_HIP(hipMemcpyAsync(dp->d_in, dp->h_in, N * 8, hipMemcpyHostToDevice, st), (size_t)-1);
-    if (run_direct(dp, dp->d_in, dp->d_out, direction, 1, st, dp->precompute)) return (size_t)-1;
-    L2C_HIP(hipMemcpyAsync(dp->h_out, dp->d_out, N * 8, hipMemcpyDeviceToHost, st), (size_t)-1);
-    L2C_HIP(hipStreamSynchronize(st), (size_t)-1);
-    for (size_t i = 0; i < N; i++) output_array[i * stride] = dp->h_out[i];
+    HostStage &h = dp->host;
+    if (ensure_staging(N, h) || stage_in(h, input_array, stride, N, st) ||
+        run_direct(dp, h.d_in, h.d_out, direction, 1, st, dp->precompute) ||
+        stage_out(h, output_array, stride, N, st))
+      return (size_t)-1;
   }
   return flops_direct(N, direction, dp->precompute);
 }

@@ -206,6 +206,19 @@ constexpr int kSlices = 6;
 enum KernelId {
   K_UP_SUBTREE = 0, K_M2L = 1, K_DOWN_BAND = 2, K_DIRECT = 3, K_FAR = 4, K_BAND = 5, K_COUNT = 8
 };
+// Staging of calls with host arrays, made by a plan's first such call.
+constexpr size_t kHostChunks = 8;
+inline size_t host_chunks(size_t N) {
+  const size_t c = (N + 65535) / 65536;
+  return c < kHostChunks ? c : kHostChunks;
+}
+struct HostStage {
+  double *d_in = nullptr, *d_out = nullptr;  // device
+  double *h_in = nullptr, *h_out = nullptr;  // pinned host
+  hipEvent_t ev[kHostChunks] = {};           // the chunks of h_out are there
+};
+void free_staging(HostStage &h);
+
 struct Prof {
   int on = 0;       // timing period in calls (0: off)
   size_t calls = 0;  // calls since enabled
@@ -265,8 +278,7 @@ struct direct_plan_s {
   // single transforms of N > 3072 on k_direct_band, else k_direct_rows
   // (L2C_DIRECT_BAND=0: always k_direct_rows)
   bool direct_band = true;
-  double *d_in = nullptr, *d_out = nullptr;  // staging (device)
-  double *h_in = nullptr, *h_out = nullptr;  // staging (pinned host)
+  l2c::HostStage host;
   hipStream_t stream = nullptr;
   l2c::Prof *prof = nullptr;
 };
@@ -331,9 +343,7 @@ struct fmm_plan_s {
   // stores replaced by a larger one; a launch on another stream may still
   // use them, so they are released only when the plan is freed
   std::vector<double *> wl_retired;
-  // host staging, allocated by the first call with host arrays
-  double *d_in = nullptr, *d_out = nullptr;  // staging (device, contiguous)
-  double *h_in = nullptr, *h_out = nullptr;  // staging (pinned host)
+  l2c::HostStage host;
   size_t hbm_bytes = 0;
   hipStream_t stream = nullptr;
   l2c::Prof *prof = nullptr;

@@ -507,10 +507,7 @@ void destroy_direct(direct_plan_s *dp) {
   dfree(dp->d_dn);
   dfree(dp->d_K[0]);
   dfree(dp->d_K[1]);
-  dfree(dp->d_in);
-  dfree(dp->d_out);
-  if (dp->h_in) (void)hipHostFree(dp->h_in);
-  if (dp->h_out) (void)hipHostFree(dp->h_out);
+  free_staging(dp->host);
   if (dp->stream) (void)hipStreamDestroy(dp->stream);
   delete dp;
 }
@@ -545,10 +542,7 @@ static void destroy_fmm(fmm_plan_s *p) {
   dfree(p->d_w);
   dfree(p->d_wl);
   for (double *r : p->wl_retired) dfree(r);
-  dfree(p->d_in);
-  dfree(p->d_out);
-  if (p->h_in) (void)hipHostFree(p->h_in);
-  if (p->h_out) (void)hipHostFree(p->h_out);
+  free_staging(p->host);
   if (p->dplan) p->dplan->prof = nullptr;
   destroy_direct(p->dplan);
   if (p->prof) {
