@@ -81,57 +81,60 @@ __host__ __device__ __forceinline__ int sk8(int k) { return k + (k >> 3); }
 
 
 // ---------------------------------------------------------------------------
-// The near-field band (src/C/leg2cheb.c:236-535) of 16 leaf chunks, any leaf
-// size s <= 64, by the 256 threads of a work-group: rows r of parity sg take
+// The near-field band (src/C/leg2cheb.c:236-535) of G = 16 (or 8) leaf chunks, any
+// leaf size s <= 64, by the 256 threads of a work-group: rows r of parity sg take
 // the columns c = r + t, t < len (2 s - 16 gam for row group gam, shorter in
 // the last chunk), y_r = sum H(t - rho) P(2 r0 + sg + t + rho) x(r0 + t).
-// Each lane owns 16 rows of one chunk and parity: lane = chunk + 16 parity +
-// 32 del, row group gam = 2 p + del; waves split (p, columns).  All lanes of a
-// wave sit at the same t, so H is wave-uniform: scalar loads, which the
-// products take as operands; P runs through a ring of 16 registers.  Per
-// column a lane reads one x and one P from LDS for 16 terms (one multiply and
-// one FMA each), four columns ahead.
+// Each lane owns 16 rows of one chunk and parity: lane = chunk + G parity + 2 G
+// del, row group gam = del, or (G = 16, more than two row groups) 2 p + del; the
+// waves split (p, columns).  All lanes of a wave sit at the same t, so H is
+// wave-uniform: scalar loads, which the products take as operands; P runs
+// through a ring of 16 registers.  Per column a lane reads one x and one P from
+// LDS for 16 terms (one multiply and one FMA each), four columns ahead.
 //   x, per parity, half index h from the first chunk: h + h / s when 4
 //     divides s (one pad per chunk), else h; parity 1 at +nxs, nxs odd when
-//     s = 2 mod 4, else 16 mod 32
+//     s = 2 mod 4, else G mod 32
 //   P, entry m from the first row: m + 2 (m / 2s) for even s (every 2s
 //     entries are followed by a copy of the next two), else m
-// so that the 32 lanes of half a wave read distinct banks, and a lane's four
-// entries are always consecutive (it meets a chunk's end only between them,
-// S16: s a multiple of 16, only between trips of 16).
+// so that the 32 lanes of half a wave read distinct banks (G = 8: pairs of lanes
+// share one of P's), and a lane's four entries are always consecutive (it meets
+// a chunk's end only between them, S16: s a multiple of 16, only between trips
+// of 16).
 // Bound by FP64 issue on large calls (4.6 M vector instructions at N = 2^20,
 // s = 64, three quarters of them the products), on one small line by the
 // work-group's own chain (window loads 2 us, its trips 1 us each, staging).
 // As k_band alone, s = 64: 2^16 10.0 us, 2^20 17.3, 64 lines of 2^18 165; with
 // 8 rows a lane, H from LDS and a Lambda window per chunk, s = 16, 32, 64 only,
 // 11.3, 18.6 and 212.
-constexpr int kBandNT = 256, kBandG = 16, kBandMaxS = 64;
+constexpr int kBandNT = 256, kBandMaxS = 64;
 struct BandLds {
   int nx, pad, nxs, np, pw, PS, CS, total;
 };
-__host__ __device__ inline BandLds band_lds(const Geo &g) {
+__host__ __device__ inline BandLds band_lds(const Geo &g, int G) {
   const int s = g.s;
   BandLds d;
-  d.nx = (kBandG + 1) * s + 32;  // half indices per parity: the last chunk's columns, a trip over
+  // half indices per parity: the last chunk's columns, to the end of its trips
+  // (G = 8: a wave's trips are those of its longest row group)
+  d.nx = (G + 1) * s + (G == 8 ? 80 : 32);
   d.pad = (s & 3) == 0;
   const int n = d.nx + (d.pad ? d.nx / s + 1 : 0);
-  d.nxs = (s & 3) == 2 ? n | 1 : n + (48 - n % 32) % 32;
+  d.nxs = (s & 3) == 2 ? n | 1 : n + (32 + G - n % 32) % 32;  // G mod 32
   d.pw = 2 * d.nxs;
   d.pw += d.pw & 1;  // 16-byte rows
-  d.np = 2 * kBandG * s + s + 64;
+  d.np = 2 * G * s + (G == 8 ? std::max(s + 64, 148) : s + 64);
   d.np += d.np & 1;
   d.PS = 2 * s + ((s & 1) ? 0 : 2);
   // staging of the sums, [segment][chunk][CS], over the windows
   d.CS = d.PS;
-  const int npair = (s + 31) / 32;
+  const int npair = G == 8 ? 1 : (s + 31) / 32;
   // (the unused prefetch behind a last trip may pass the windows' ends)
   d.total = std::max(d.pw + d.np + ((s & 1) ? 0 : 2 * (d.np / (2 * s) + 1)) + 32,
-                     (kBandNT / 64 / npair) * kBandG * d.CS);
+                     (kBandNT / 64 / npair) * G * d.CS);
   return d;
 }
-size_t band_shared_bytes(const Geo &g) { return 8 * (size_t)band_lds(g).total; }
-inline unsigned band_groups(const Geo &g) {  // work-groups of one line
-  return (unsigned)((((size_t)2 << g.L) + kBandG - 1) / kBandG);
+inline size_t band_shared_bytes(const Geo &g, int G) { return 8 * (size_t)band_lds(g, G).total; }
+inline unsigned band_groups(const Geo &g, int G) {  // work-groups of one line
+  return (unsigned)((((size_t)2 << g.L) + G - 1) / G);
 }
 
 typedef const __attribute__((address_space(4))) double *kdouble;  // uniform, read-only
@@ -209,7 +212,7 @@ __device__ __forceinline__ void band_trip(BandPtr &b, int s1, int s2, kdouble hp
 // Band group grp of the line at src / dst (element stride es, length Nl): the
 // sums are stored over the output, raw (the C2L diagonal included), or with
 // the final scaling when scale != 0.
-template <bool S16>
+template <bool S16, int G>
 __device__ __forceinline__ void band_group(const double *__restrict__ src,
                                            double *__restrict__ dst, size_t es, int Nl,
                                            const Geo &g, int dir, int grp, int scale,
@@ -218,16 +221,16 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
   const int s = g.s, N = g.N;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const size_t hc0 = (size_t)grp * kBandG * s, row0 = 2 * hc0;
+  const size_t hc0 = (size_t)grp * G * s, row0 = 2 * hc0;
   if (row0 >= (size_t)Nl) return;  // the whole work-group
-  const BandLds ly = band_lds(g);
+  const BandLds ly = band_lds(g, G);
   double *xs = sm, *pw = sm + ly.pw;
   const unsigned inv = ((1u << 20) + s - 1) / s;  // h / s = h inv >> 20 for h < 2200
   auto chunk = [&](int h) { return (int)(__umul24(h, inv) >> 20); };
   const bool even = (s & 1) == 0;
   // ---- windows: pairs of P, pairs (2 h, 2 h + 1) of x; past the table's and
   // the line's ends zeros
-  constexpr int QX = 5;  // ceil(nx / 256), ceil(np / 512) for s = 64
+  constexpr int QX = G == 8 ? 3 : 5;  // ceil(nx / 256), ceil(np / 512) for s = 64
   d2 vp[QX], vx[QX];
   {
     const __amdgpu_buffer_rsrc_t r =
@@ -277,15 +280,15 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
   lds_sync();
 
   // ---- the band
-  const int ng = (s + 15) >> 4, npair = (ng + 1) >> 1;
+  const int ng = (s + 15) >> 4, npair = G == 8 ? 1 : (ng + 1) >> 1;
   const int lseg = npair == 1 ? 2 : 1, nseg = 1 << lseg;
   const int p = npair == 1 ? 0 : wave & 1, seg = npair == 1 ? wave : wave >> 1;
   double acc[16];
 #pragma unroll
   for (int k = 0; k < 16; k++) acc[k] = 0.0;
   {
-    const int gl = lane & 15, sg = (lane >> 4) & 1, gam = 2 * p + (lane >> 5);
-    const size_t beta = (size_t)grp * kBandG + gl, nLm1 = (size_t)g.nL - 1;
+    const int gl = lane & (G - 1), sg = lane / G & 1, gam = 2 * p + lane / (2 * G);
+    const size_t beta = (size_t)grp * G + gl, nLm1 = (size_t)g.nL - 1;
     const size_t r0 = beta * s + 16 * gam, cnt = (N - sg + 1) / 2;
     const size_t cend = beta < nLm1 ? (beta + 2) * s : cnt;
     const int len = 16 * gam < s && r0 < cnt ? (int)(cend - r0) : 0;
@@ -293,8 +296,8 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
     const int t0 = 16 * (T * seg >> lseg), t1 = 16 * (T * (seg + 1) >> lseg);
     // columns that every live row of the wave has (none where the chunks'
     // ends differ)
-    const bool last = ((size_t)grp + 1) * kBandG > nLm1;
-    const int common = last ? 0 : 2 * s - 16 * std::min(2 * p + 1, ng - 1);
+    const bool last = ((size_t)grp + 1) * G > nLm1;
+    const int common = last ? 0 : 2 * s - 16 * std::min(G == 8 ? 3 : 2 * p + 1, ng - 1);
     kdouble hp = (kdouble)head;
     double pr[16], XA[4], PA[4];
     const int s1 = ly.pad ? s : 1 << 20, s2 = even ? 2 * s : 1 << 20;
@@ -327,7 +330,7 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
   // that it is the one used above, so nothing is held through the trips)
   int ln = lane;
   asm volatile("" : "+v"(ln));
-  const int gl = ln & 15, sg = (ln >> 4) & 1, gam = 2 * p + (ln >> 5);
+  const int gl = ln & (G - 1), sg = ln / G & 1, gam = 2 * p + ln / (2 * G);
   if (dir == C2L) {
     // less the sum; the C2L diagonal sqrt(pi) an_i v_i (src/C/leg2cheb.c:416)
     const int h0 = gl * s + 16 * gam;
@@ -339,21 +342,21 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
       acc[k] = (seg == 0 ? d : 0.0) - acc[k];
     }
   }
-  const bool live = ((size_t)grp * kBandG + gl) * s + 16 * gam < (size_t)(N - sg + 1) / 2;
+  const bool live = ((size_t)grp * G + gl) * s + 16 * gam < (size_t)(N - sg + 1) / 2;
   lds_sync();  // windows dead: the staging takes their place
   if (live) {
-    double *o = sm + (seg * kBandG + gl) * ly.CS + 32 * gam + sg;
+    double *o = sm + (seg * G + gl) * ly.CS + 32 * gam + sg;
 #pragma unroll
     for (int k = 0; k < 16; k++)
       if (16 * gam + k < s) o[2 * k] = acc[k];
   }
   lds_sync();
   // ---- the segments' sums, stored
-  const int nr = (int)std::min<size_t>((size_t)kBandG * 2 * s, (size_t)Nl - row0);
+  const int nr = (int)std::min<size_t>((size_t)G * 2 * s, (size_t)Nl - row0);
   auto value = [&](int e) {
     const double *o = sm + e + (even ? 2 * chunk(e >> 1) : 0);
-    double v = o[0] + o[kBandG * ly.CS];
-    if (nseg == 4) v += o[2 * kBandG * ly.CS] + o[3 * kBandG * ly.CS];
+    double v = o[0] + o[G * ly.CS];
+    if (nseg == 4) v += o[2 * G * ly.CS] + o[3 * G * ly.CS];
     if (scale) {
       const size_t i = row0 + e;
       if (dir == L2C) {
@@ -840,7 +843,7 @@ struct BandArgs {
   double *out;
   const double *tab, *head;
 };
-template <bool S16>
+template <bool S16, int G>
 __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up(
     const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
     const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
@@ -851,7 +854,7 @@ __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4)))
       up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, blockIdx.x, sm);
   } else {
     const size_t off = line_off(lm, blockIdx.y);
-    band_group<S16>(in + off, ba.out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
+    band_group<S16, G>(in + off, ba.out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
                     blockIdx.x, 0, ba.tab, ba.head, sm);
   }
 }
@@ -1573,7 +1576,7 @@ __host__ __device__ inline DownLds down_lds(const Geo &g) {
 size_t down8_shared_bytes(const Geo &g);
 size_t down_shared_bytes(const Geo &g) {
   return g.fast ? down8_shared_bytes(g)
-         : g.far ? std::max(far_shared_bytes(g), band_shared_bytes(g))
+         : g.far ? std::max(far_shared_bytes(g), band_shared_bytes(g, 16))
                  : 8 * (size_t)down_lds(g).total;
 }
 
@@ -2626,7 +2629,7 @@ __global__ void __launch_bounds__(kBandNT) __attribute__((amdgpu_waves_per_eu(4)
     const double *__restrict__ tab, const double *__restrict__ head) {
   extern __shared__ double sm[];
   const size_t off = line_off(lm, blockIdx.y);
-  band_group<S16>(in + off, out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
+  band_group<S16, 16>(in + off, out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
                   (int)blockIdx.x, scale, tab, head, sm);
 }
 
@@ -3794,8 +3797,8 @@ static void launch_band(fmm_plan_s *p, const Geo &g, const double *d_in, double 
                         const LineMap &lm, size_t nlines, hipStream_t st, int scale, int slot) {
   prof_begin(p->prof, slot, st);
   launch_k(p->prof, (g.s & 15) == 0 ? k_band<true> : k_band<false>,
-           dim3(band_groups(g), (unsigned)nlines), kBandNT, band_shared_bytes(g), st, d_in, d_out,
-           lm, g, (int)dir, scale, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
+           dim3(band_groups(g, 16), (unsigned)nlines), kBandNT, band_shared_bytes(g, 16), st, d_in,
+           d_out, lm, g, (int)dir, scale, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
   prof_end(p->prof, st);
 }
 
@@ -3806,6 +3809,18 @@ static void launch_far(fmm_plan_s *p, const Geo &g, double *d_out, size_t dir, c
            far_shared_bytes(g), st, d_out, lm, g, (int)dir, ws, ws_doubles(g), p->t.D, p->t.Q,
            p->t.T);
   prof_end(p->prof, st);
+}
+
+// Groups of 8 chunks halve a small call's chain of trips (four to two at s =
+// 64) and waste a fifth of the lanes' columns: taken while the band's groups of
+// 16 leave most of the chip idle, for leaf sizes with more than two row groups.
+// us per call, 16 / 8 chunks: one line of 2^13 18.8 / 16.0, 2^16 19.8 / 17.0,
+// 200,000 (s = 49) 24.3 / 21.0, 2^18 23.8 / 21.3, 2^19 (256 groups of 16) 33.8 /
+// 32.4, 600,000 (512) 39.3 / 41.6, 2^20 44.1 / 45.7; 16 lines of 2^13 (64) 20.3 /
+// 17.9, 2 of 2^16 (64) 20.7 / 18.7, 4 of 2^16 (128) 22.0 / 22.8, 12 of 2^14 (96)
+// 21.3 / 21.8, 2 of 2^18 (256) 26.0 / 30.8.
+static bool band_by_8(const Geo &g, size_t nlines) {
+  return g.s > 32 && band_groups(g, 16) * nlines <= (nlines == 1 ? 256 : 64);
 }
 
 // The downward pass of a far plan (geo.far): the band inside the k_up launch,
@@ -3840,12 +3855,15 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
   if (!band_only) {
     const bool s16 = (g.s & 15) == 0;
     dim3 gu(4u << g.lu, (unsigned)nlines);
-    if (fuse) gu = dim3(std::max(gu.x, band_groups(g)), gu.y, 2);
+    const bool b8 = fuse && band_by_8(g, nlines);
+    if (fuse) gu = dim3(std::max(gu.x, band_groups(g, b8 ? 8 : 16)), gu.y, 2);
     const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]};
     prof_begin(p->prof, K_UP_SUBTREE, st);
     if (MT == 18 && up18_eligible(g)) {
-      const size_t shu = std::max(8 * (size_t)up18_lds(g).total, fuse ? band_shared_bytes(g) : 0);
-      launch_k(p->prof, s16 ? k_up<true> : k_up<false>, gu, kUpNT, shu, st, d_in, lm, g, (int)dir,
+      const size_t shu = std::max(8 * (size_t)up18_lds(g).total,
+                                  fuse ? band_shared_bytes(g, b8 ? 8 : 16) : 0);
+      launch_k(p->prof, b8 ? (s16 ? k_up<true, 8> : k_up<false, 8>)
+                           : (s16 ? k_up<true, 16> : k_up<false, 16>), gu, kUpNT, shu, st, d_in, lm, g, (int)dir,
                p->t.T, p->t.U, p->t.P, ws, wsstride, bu);
     } else if (MT > 0 && g.gu >= 3 && nlines <= 8) {
       launch_k(p->prof, k_up_any<MT, MT != 0>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g,

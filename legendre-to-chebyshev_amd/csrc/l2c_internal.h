@@ -403,7 +403,6 @@ int build_slices(fmm_plan_s *p, int dir);  // precision form 2 tables of one dir
 void drop_graphs(fmm_plan_s *p);  // synchronises the plan's stream first
 size_t flops_fmm(const fmm_plan_s *p, size_t dir);
 size_t down_shared_bytes(const Geo &g);  // of the downward kernel g selects
-size_t band_shared_bytes(const Geo &g);
 size_t far_shared_bytes(const Geo &g);
 bool down8_eligible(const Geo &g);
 bool far_eligible(const Geo &g);

@@ -123,3 +123,43 @@ def test_other_ranks(amd, orc, monkeypatch, N, maxs, M):
         u = np.random.default_rng(N).uniform(-1, 1, N)
         for d in (0, 1):
             assert relerr(plan.execute(u, d), op.execute(u, d)) <= tol(N), (name, value, d)
+
+
+@pytest.mark.parametrize("s", range(1, 65))
+def test_many_lines(amd, orc, s):
+    """Calls of many lines, whose band takes 8 chunks per work-group (the first
+    two) or 16 (the last) for s > 32, contiguous and strided."""
+    announce(f"many lines, leaf size {s}")
+    for L, r, B in ((1, 0, 16), (3, 5, 37), (4, 1, 70)):
+        N = 4 << L if s == 1 else s * (4 << L) - min(r, (4 << L) - 1)
+        plan = amd.FMMPlan(N, s, 18, 2)
+        assert plan.info()["s"] == s
+        op = orc.FMMPlan(N, s, 18, 2)
+        x = np.random.default_rng(64 * L + s).uniform(-1, 1, (B, N))
+        for d in (0, 1):
+            o = {l: op.execute(np.ascontiguousarray(x[l]), d) for l in (0, 7, 15, B - 1)}
+            for strided in (False, True):
+                z = lines(amd, plan, x, d, strided, pad=1)
+                for l in o:
+                    assert relerr(z[l], o[l]) <= tol(N), (N, d, strided, l)
+
+
+@pytest.mark.parametrize("N,s,B", [(4096, 64, 20), (4000, 32, 17), (9000, 36, 33), (9000, 36, 3)])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_not_finite(amd, N, s, B, direction):
+    """A NaN or Inf reaches the rows of its own line that it belongs to, at or
+    before its place and of its parity, and no other (the near field; upward
+    of it the far field spreads it to all of them)."""
+    announce(f"not finite N={N} B={B} dir={direction}")
+    plan = amd.FMMPlan(N, s, 18, direction)
+    for strided in (False, True):
+        for pos in (0, 1, N // 3, N // 2 + 1, N - 130, N - 2, N - 1):
+            for val in (np.inf, np.nan):
+                x = np.random.default_rng(B).uniform(0.5, 1, (B, N))
+                x[B // 2, pos] = val
+                z = lines(amd, plan, x, direction, strided)
+                want = np.zeros((B, N), bool)
+                want[B // 2, pos % 2:pos + 1:2] = True
+                bad = ~np.isfinite(z)
+                assert not np.any(bad & ~want), (strided, pos, val)
+                assert bad[B // 2, pos]
