@@ -151,12 +151,29 @@ __device__ __forceinline__ double2 quarter_root(const double2 *ts, int u) {
   return r;
 }
 
-// One Stockham stage of radix R on NC columns of length L held in LDS with
-// column stride L + 1.  Sub-transform size 2^LOGNS before the stage.  The
+// Layout of NC columns of length 2^LOGL in LDS: one element of padding after
+// every eight, so that the butterflies' outputs (stride R in a column's first
+// stage, pairs and fours of neighbours in the next) fall on distinct banks, and
+// a column stride that keeps neighbouring columns apart (8 / NC mod 8 elements:
+// loads and stores run the columns fastest).  Not where it would leave one
+// work-group per CU instead of two.  With columns of L + 1 and no padding, bank
+// conflicts took 1.3 of the 2.1 us that the LDS is busy in a pass of N = 2^20.
+template <int LOGL, int NC>
+struct Cols {
+  static constexpr int L = 1 << LOGL, LP = L + L / 8;
+  static constexpr bool PAD = LOGL >= 4 && (NC * (LP + 8) + L / 4) * 16 <= 80 * 1024;
+  static constexpr int STEP = NC >= 8 ? 1 : 8 / NC;
+  static constexpr int LD = PAD ? LP + (STEP + 8 - LP % 8) % 8 : L + 1;
+  __device__ static int at(int col, int i) { return col * LD + (PAD ? i + (i >> 3) : i); }
+};
+
+// One Stockham stage of radix R on NC columns of length L held in LDS (Cols).
+// Sub-transform size 2^LOGNS before the stage.  The
 // reads of every butterfly go to registers, then the stage writes in place.
 template <int LOGL, int NC, int T, int R, int LOGNS, int S>
 __device__ __forceinline__ void fft_stage(double2 *buf, const double2 *ts) {
-  constexpr int L = 1 << LOGL, LD = L + 1, Q = L / R, TOT = NC * Q;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, Q = L / R, TOT = NC * Q;
   constexpr int NB = (TOT + T - 1) / T, NS = 1 << LOGNS;
   constexpr int STEP = L / (NS * R);
   double2 v[NB][R];
@@ -165,9 +182,8 @@ __device__ __forceinline__ void fft_stage(double2 *buf, const double2 *ts) {
     const int id = threadIdx.x + b * T;
     if (TOT % T == 0 || id < TOT) {
       const int col = id / Q, j = id % Q;
-      const double2 *src = buf + col * LD + j;
 #pragma unroll
-      for (int t = 0; t < R; ++t) v[b][t] = src[t * Q];
+      for (int t = 0; t < R; ++t) v[b][t] = buf[Z::at(col, j + t * Q)];
       if constexpr (NS > 1) {
         const int k = j & (NS - 1);
 #pragma unroll
@@ -186,9 +202,8 @@ __device__ __forceinline__ void fft_stage(double2 *buf, const double2 *ts) {
     const int id = threadIdx.x + b * T;
     if (TOT % T == 0 || id < TOT) {
       const int col = id / Q, j = id % Q, k = j & (NS - 1);
-      double2 *dst = buf + col * LD + (j - k) * R + k;
 #pragma unroll
-      for (int t = 0; t < R; ++t) dst[t * NS] = v[b][t];
+      for (int t = 0; t < R; ++t) buf[Z::at(col, (j - k) * R + k + t * NS)] = v[b][t];
     }
   }
   __syncthreads();
@@ -295,7 +310,8 @@ template <int LOGM, int NV, int LAY>
 __global__ void __launch_bounds__(kElems / 8)
     k_dct2_1p(const double *__restrict__ x, double *__restrict__ y, size_t count, LineMap lm,
               Tabs tb) {
-  constexpr int M = 1 << LOGM, LD = M + 1, H = M / 2, T = kElems / 8;
+  using Z = Cols<LOGM, NV>;
+  constexpr int M = 1 << LOGM, LD = Z::LD, H = M / 2, T = kElems / 8;
   constexpr int NI = NV * M / T, NL = NV * H / T;  // items per thread: post, load
   extern __shared__ double2 z[];
   double2 *ts = z + NV * LD;
@@ -336,8 +352,8 @@ __global__ void __launch_bounds__(kElems / 8)
     int vi, m;
     item<H, NV, STRIDED>(threadIdx.x + it * T, vi, m);
     if (v0 + vi < count) {
-      z[vi * LD + m] = make_double2(p0[it].x, p1[it].x);
-      z[vi * LD + (M - 1 - m)] = make_double2(p1[it].y, p0[it].y);
+      z[Z::at(vi, m)] = make_double2(p0[it].x, p1[it].x);
+      z[Z::at(vi, M - 1 - m)] = make_double2(p1[it].y, p0[it].y);
     }
   }
   __syncthreads();
@@ -347,7 +363,7 @@ __global__ void __launch_bounds__(kElems / 8)
     int vi, k;
     item<M, NV, STRIDED>(threadIdx.x + it * T, vi, k);
     if (v0 + vi < count)
-      dct2_post(y + start(vi), k, M, z[vi * LD + k], conj2(z[vi * LD + ((M - k) & (M - 1))]),
+      dct2_post(y + start(vi), k, M, z[Z::at(vi, k)], conj2(z[Z::at(vi, (M - k) & (M - 1))]),
                 t1[it], t4[it], es);
   }
 }
@@ -356,7 +372,8 @@ __global__ void __launch_bounds__(kElems / 8)
 template <int LOGL, int NC, int PT>
 __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     k_dct2_p1(const double *__restrict__ x, double2 *__restrict__ W, int logM1, Tabs tb) {
-  constexpr int L = 1 << LOGL, LD = L + 1, C = NC / 2, T = NC * L / PT;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, LD = Z::LD, C = NC / 2, T = NC * L / PT;
   extern __shared__ double2 z[];
   double2 *ts = z + NC * LD;
   const int M1 = 1 << logM1;
@@ -384,8 +401,8 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 #pragma unroll
   for (int it = 0; it < PT / 2; ++it) {
     const int id = threadIdx.x + it * T, i = id % NC, n2 = id / NC;
-    z[i * LD + n2] = make_double2(p0[it].x, p1[it].x);
-    z[partner<C>(i) * LD + (L - 1 - n2)] = make_double2(p1[it].y, p0[it].y);
+    z[Z::at(i, n2)] = make_double2(p0[it].x, p1[it].x);
+    z[Z::at(partner<C>(i), L - 1 - n2)] = make_double2(p1[it].y, p0[it].y);
   }
   __syncthreads();
   fft_cols<LOGL, NC, T, -1, PT == 8 ? 3 : 2>(z, ts);
@@ -393,7 +410,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   for (int it = 0; it < PT; ++it) {
     const int id = threadIdx.x + it * T, i = id / L, k2 = id % L;
     const size_t n1 = size_t(col_reflect<C>(i, a, M1));
-    W[(n1 << LOGL) + k2] = cmul(z[i * LD + k2], cmul(th[it], tl[it]));
+    W[(n1 << LOGL) + k2] = cmul(z[Z::at(i, k2)], cmul(th[it], tl[it]));
   }
 }
 
@@ -401,7 +418,8 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 template <int LOGL, int NC, int PT>
 __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     k_dct2_p2(const double2 *__restrict__ W, double *__restrict__ y, int logM2, Tabs tb) {
-  constexpr int L = 1 << LOGL, LD = L + 1, C = NC / 2, T = NC * L / PT;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, LD = Z::LD, C = NC / 2, T = NC * L / PT;
   extern __shared__ double2 z[];
   double2 *ts = z + NC * LD;
   const int M2 = 1 << logM2;
@@ -427,7 +445,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   }
   load_quarter<LOGL, T>(ts, tb.tw);
 #pragma unroll
-  for (int it = 0; it < PT; ++it) z[i * LD + (threadIdx.x + it * T) / NC] = d[it];
+  for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
   fft_cols<LOGL, NC, T, -1, PT == 8 ? 3 : 2>(z, ts);
   // the partner of column k2: itself for k2 = 0 (row (L - k1) mod L) and for
@@ -437,7 +455,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   for (int it = 0; it < PT; ++it) {
     const int k1 = (threadIdx.x + it * T) / NC;
     const int row = k2 == 0 ? ((L - k1) & (L - 1)) : L - 1 - k1;
-    dct2_post(y, size_t(k1) * M2 + k2, M, z[i * LD + k1], conj2(z[ip * LD + row]),
+    dct2_post(y, size_t(k1) * M2 + k2, M, z[Z::at(i, k1)], conj2(z[Z::at(ip, row)]),
               cmul(r1[it], c1), cmul(r4[it], c4));
   }
 }
@@ -460,7 +478,8 @@ template <int LOGM, int NV, int LAY>
 __global__ void __launch_bounds__(kElems / 8)
     k_dct3_1p(const double *__restrict__ Y, double *__restrict__ x, size_t count, LineMap lm,
               Tabs tb) {
-  constexpr int M = 1 << LOGM, LD = M + 1, H = M / 2, N = 2 * M, T = kElems / 8;
+  using Z = Cols<LOGM, NV>;
+  constexpr int M = 1 << LOGM, LD = Z::LD, H = M / 2, N = 2 * M, T = kElems / 8;
   constexpr int NI = NV * M / T, NL = NV * N / T, NS = NV * H / T;
   extern __shared__ double2 z[];
   double2 *ts = z + NV * LD;
@@ -509,7 +528,7 @@ __global__ void __launch_bounds__(kElems / 8)
   for (int it = 0; it < NI; ++it) {
     int vi, k;
     item<M, NV, STRIDED>(threadIdx.x + it * T, vi, k);
-    z[vi * LD + k] = zp[it];
+    z[Z::at(vi, k)] = zp[it];
   }
   __syncthreads();
   fft_cols<LOGM, NV, T, 1>(z, ts);
@@ -518,7 +537,7 @@ __global__ void __launch_bounds__(kElems / 8)
     int vi, m;
     item<H, NV, STRIDED>(threadIdx.x + it * T, vi, m);
     if (v0 + vi < count) {
-      const double2 A = z[vi * LD + m], B = z[vi * LD + (M - 1 - m)];
+      const double2 A = z[Z::at(vi, m)], B = z[Z::at(vi, M - 1 - m)];
       double *dst = x + start(vi) + 4 * size_t(m) * es;
       if (STRIDED) {
         dst[0] = A.x;
@@ -538,7 +557,8 @@ __global__ void __launch_bounds__(kElems / 8)
 template <int LOGL, int NC, int PT>
 __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     k_dct3_p1(const double *__restrict__ Y, double2 *__restrict__ W, int logM1, Tabs tb) {
-  constexpr int L = 1 << LOGL, LD = L + 1, C = NC / 2, T = NC * L / PT;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, LD = Z::LD, C = NC / 2, T = NC * L / PT;
   extern __shared__ double2 z[];
   double2 *ts = z + NC * LD;
   double *yr = reinterpret_cast<double *>(z);
@@ -586,7 +606,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   }
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < PT; ++it) z[i * LD + (threadIdx.x + it * T) / NC] = zp[it];
+  for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = zp[it];
   __syncthreads();
   // store items: i = id / L, k2 = id % L; twiddle e^{+2 pi i n1 k2 / M}
   double2 th[PT], tl[PT];
@@ -601,7 +621,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   for (int it = 0; it < PT; ++it) {
     const int id = threadIdx.x + it * T, j = id / L, k2 = id % L;
     const size_t m1 = size_t(col_negate<C>(j, a, M1));
-    W[(m1 << LOGL) + k2] = cmul(z[j * LD + k2], conj2(cmul(th[it], tl[it])));
+    W[(m1 << LOGL) + k2] = cmul(z[Z::at(j, k2)], conj2(cmul(th[it], tl[it])));
   }
 }
 
@@ -609,7 +629,8 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 template <int LOGL, int NC, int PT>
 __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     k_dct3_p2(const double2 *__restrict__ W, double *__restrict__ x, int logM2, Tabs tb) {
-  constexpr int L = 1 << LOGL, LD = L + 1, C = NC / 2, T = NC * L / PT;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, LD = Z::LD, C = NC / 2, T = NC * L / PT;
   extern __shared__ double2 z[];
   double2 *ts = z + NC * LD;
   const int M2 = 1 << logM2;
@@ -624,7 +645,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   for (int it = 0; it < PT; ++it) d[it] = W[size_t((threadIdx.x + it * T) / NC) * M2 + k2];
   load_quarter<LOGL, T>(ts, tb.tw);
 #pragma unroll
-  for (int it = 0; it < PT; ++it) z[i * LD + (threadIdx.x + it * T) / NC] = d[it];
+  for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
   fft_cols<LOGL, NC, T, 1, PT == 8 ? 3 : 2>(z, ts);
   const int ip = partner<C>(i);
@@ -632,7 +653,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   for (int it = 0; it < PT / 2; ++it) {
     const int k1 = (threadIdx.x + it * T) / NC;  // < L/2
     const size_t m = size_t(k1) * M2 + k2;
-    const double2 A = z[i * LD + k1], B = z[ip * LD + (L - 1 - k1)];
+    const double2 A = z[Z::at(i, k1)], B = z[Z::at(ip, L - 1 - k1)];
     double *dst = x + 4 * m;
     *reinterpret_cast<double2 *>(dst) = make_double2(A.x, B.y);
     *reinterpret_cast<double2 *>(dst + 2) = make_double2(A.y, B.x);
@@ -651,7 +672,8 @@ template <int LOGL, int NC, int S, int PT>
 __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     k_fft_mid(const double2 *__restrict__ W, double2 *__restrict__ W2, int logL1, int logL3,
               Tabs tb) {
-  constexpr int L = 1 << LOGL, LD = L + 1, T = NC * L / PT;
+  using Z = Cols<LOGL, NC>;
+  constexpr int L = 1 << LOGL, LD = Z::LD, T = NC * L / PT;
   extern __shared__ double2 z[];
   double2 *ts = z + NC * LD;
   const size_t M = size_t(1) << (logL1 + LOGL + logL3);
@@ -674,7 +696,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
   }
   load_quarter<LOGL, T>(ts, tb.tw);
 #pragma unroll
-  for (int it = 0; it < PT; ++it) z[i * LD + (threadIdx.x + it * T) / NC] = d[it];
+  for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
   fft_cols<LOGL, NC, T, S, PT == 8 ? 3 : 2>(z, ts);
 #pragma unroll
@@ -682,7 +704,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     const size_t k2 = (threadIdx.x + it * T) / NC;
     double2 w = cmul(th[it], tl[it]);
     if constexpr (S > 0) w.y = -w.y;
-    W2[(((n1 << LOGL) + k2) << logL3) + k3] = cmul(z[i * LD + k2], w);
+    W2[(((n1 << LOGL) + k2) << logL3) + k3] = cmul(z[Z::at(i, k2)], w);
   }
 }
 
@@ -771,7 +793,8 @@ void launch_1p_lay(const l2c_dct_plan *p, const double *in, double *out, int kin
                    const LineMap &lm, hipStream_t st) {
   constexpr int M = 1 << LOGM, NV = kElems / M;
   const size_t shmem =
-      (size_t(NV) * (M + 1) + (LOGM > 3 ? M / 4 : 0)) * sizeof(double2) + NV * sizeof(size_t);
+      (size_t(NV) * Cols<LOGM, NV>::LD + (LOGM > 3 ? M / 4 : 0)) * sizeof(double2) +
+      NV * sizeof(size_t);
   const dim3 grid(unsigned((count + NV - 1) / NV)), blk(kElems / 8);
   if (kind == 2)
     hipLaunchKernelGGL((k_dct2_1p<LOGM, NV, LAY>), grid, blk, shmem, st, in, out, count, lm, p->tb);
@@ -801,7 +824,7 @@ template <int LOGL, int E, int PT>
 void launch_pass_e(const l2c_dct_plan *p, int pass, const double *in, double *out, int kind,
                    hipStream_t st) {
   constexpr int L = 1 << LOGL, NC = pass_nc<LOGL, E>(), T = NC * L / PT;
-  const size_t shmem = (size_t(NC) * (L + 1) + L / 4) * sizeof(double2);
+  const size_t shmem = (size_t(NC) * Cols<LOGL, NC>::LD + L / 4) * sizeof(double2);
   const int other = pass == 1 ? p->c_first : p->c_last;  // number of columns = 2^other
   const dim3 grid(unsigned((size_t(1) << other) / NC), unsigned(p->count));
   // the last pass reads the second workspace after a middle pass
@@ -820,7 +843,7 @@ void launch_pass_e(const l2c_dct_plan *p, int pass, const double *in, double *ou
 template <int LOGL, int E, int PT>
 void launch_mid_e(const l2c_dct_plan *p, int kind, hipStream_t st) {
   constexpr int L = 1 << LOGL, NC = E / L, T = E / PT;
-  const size_t shmem = (size_t(NC) * (L + 1) + L / 4) * sizeof(double2);
+  const size_t shmem = (size_t(NC) * Cols<LOGL, NC>::LD + L / 4) * sizeof(double2);
   const dim3 grid(unsigned(size_t(1) << (p->l_last + p->l_first)) / NC, unsigned(p->count));
   const double2 *w1 = p->d_work;
   double2 *w2 = p->d_work + p->count * (size_t(1) << p->logM);
