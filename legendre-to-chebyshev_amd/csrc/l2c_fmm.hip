@@ -2914,16 +2914,32 @@ __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ 
   const size_t off = line_off(lm, blockIdx.y);
   const double *u = in + off;
   const size_t es = lm.es;
-  // (four independent sums per lane, so that a trip's loads are in flight
-  // together, measured no faster: 10.3 against 9.6 us at N = 4096; the
-  // kernel is bound by its three loads per term, not by their latency)
+  // QR terms' loads in flight at once (a term past the end reads the lane's
+  // first one and adds nothing), and what the C2L diagonal needs before them
+  constexpr int QR = 4;
+  double ud = 0, pd = 0;
+  if (dir == C2L) {
+    ud = u[(size_t)i * es];
+    pd = an[i];
+  }
+  const double *Ht = dir == L2C ? a : dn, *Pt = dir == L2C ? a : an;
   double acc = 0;
-  if (dir == L2C) {
-    for (int n = 2 * lane; n + i < N; n += 128)
-      acc += a[n / 2] * k2Pi * a[n / 2 + i] * u[(size_t)(n + i) * es];
-  } else {
-    for (int n = 2 + 2 * lane; n + i < N; n += 128)
-      acc -= dn[n / 2] * an[n / 2 + i] * (u[(size_t)(n + i) * es] * (double)(n + i));
+  for (int k0 = lane + (dir == L2C ? 0 : 1); 2 * k0 + i < N; k0 += 64 * QR) {
+    double h[QR], p[QR], x[QR];
+#pragma unroll
+    for (int q = 0; q < QR; q++) {
+      const int k = 2 * (k0 + 64 * q) + i < N ? k0 + 64 * q : k0;
+      h[q] = Ht[k];
+      p[q] = Pt[k + i];
+      x[q] = u[(size_t)(2 * k + i) * es];
+    }
+#pragma unroll
+    for (int q = 0; q < QR; q++) {
+      const int n = 2 * (k0 + 64 * q);
+      const double t = dir == L2C ? h[q] * k2Pi * p[q] * x[q]
+                                  : -(h[q] * p[q] * (x[q] * (double)(n + i)));
+      if (n + i < N) acc += t;
+    }
   }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
@@ -2931,8 +2947,8 @@ __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ 
     if (dir == L2C) {
       if (i == 0) acc /= 2;
     } else {
-      const double vi = i == 0 ? u[0] : u[(size_t)i * es] * (double)i;
-      acc = (kSqrtPi * vi * an[i] + acc) * ((double)i + 0.5);
+      const double vi = i == 0 ? ud : ud * (double)i;
+      acc = (kSqrtPi * vi * pd + acc) * ((double)i + 0.5);
     }
     out[off + (size_t)i * es] = acc;
   }
@@ -2951,7 +2967,7 @@ __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ 
 // kDbChunk columns (one chunk up to N = 8192); per chunk, lane j of
 // the wave for part c of group g takes the columns t = m - r0 in
 // [(64c + j) T, (64c + j + 1) T) of the group's 8 rows, T a multiple of 8
-// with T/8 odd; the 64 lanes' sums are added across the wave, then the
+// with T/8 odd or two; the 64 lanes' sums are added across the wave, then the
 // parts through LDS.  Every window stores index e at e + e/8, so the 64
 // lanes' addresses (64 segments of T/8 padded blocks apart) fall in distinct
 // banks.  G = 1 (8 rows, four parts) while two work-groups' windows fit a
@@ -2970,6 +2986,14 @@ size_t dband_shared_bytes(int N) {
   return 8 * (size_t)(3 * w + 24);  // windows, the other parts' row sums (G = 1)
 }
 // G = 1 while two work-groups' windows fit one CU's 160 KB of LDS, else 4
+// Entries per thread and batch of the window loads: nine where that saves the
+// first work-groups a batch (N = 4096 7.0 -> 6.3 us a call, 8192 10.9 -> 10.4), else
+// eight (nine: 5000 8.6 -> 8.8, 7000 9.0 -> 9.3)
+inline int dband_batch(int N) {
+  if ((N + 1) / 2 > kDbChunk) return 8;
+  const int w = dband_win((N + 1) / 2);
+  return (w + 2303) / 2304 < (w + 2047) / 2048 ? 9 : 8;
+}
 inline int dband_groups(int N) { return dband_shared_bytes(N) <= 80 * 1024 ? 1 : 4; }
 
 // Columns [t0, t1) of the lane's 8 rows, t0 a multiple of 8; xq, pq, hq: the
@@ -3023,7 +3047,7 @@ __device__ __forceinline__ void direct_seg8(const double *__restrict__ xq,
 // Grid ((R0 + 8 G - 1) / (8 G), 2, lines) with R0 = (N + 1) / 2, 256
 // threads, dband_shared_bytes(N) of LDS; line blockIdx.z of lm (unpacked
 // maps).
-template <int DIR, int G>
+template <int DIR, int G, int QF>
 __global__ void __launch_bounds__(256) k_direct_band(const double *__restrict__ in,
                                                      double *__restrict__ out, LineMap lm, int N,
                                                      const double *__restrict__ a,
@@ -3062,7 +3086,6 @@ __global__ void __launch_bounds__(256) k_direct_band(const double *__restrict__ 
     // entry per trip: 8.6 against 8.2 us at N = 4096; QF = 16 takes 174
     // VGPRs and was slower still)
     const int tb = ch * kDbChunk;
-    constexpr int QF = 8;
     for (int e0 = tid; e0 < W; e0 += QF * 256) {
       double vx[QF], vp[QF], vh[QF];
 #pragma unroll
@@ -3087,7 +3110,9 @@ __global__ void __launch_bounds__(256) k_direct_band(const double *__restrict__ 
     __syncthreads();
     const int cw = std::min(kDbChunk, span - tb);
     int T8 = (cw + 512 * NP - 1) / (512 * NP);
-    T8 |= 1;
+    // (two: pairs of lanes share a bank, but a trip less than three: N = 4500 8.2 ->
+    // 7.7 us)
+    if (NP == 1 || T8 != 2) T8 |= 1;
     const int T = 8 * T8;
     const int t0 = tb + (64 * c + lane) * T;
     const int t1 = std::min(std::min(t0 + T, tb + kDbChunk), len);
@@ -3601,17 +3626,12 @@ static void launch_direct_one(Prof *prof, int N, size_t dir, const double *a, co
     const int G = dband_groups(N), rows = 8 * G;
     const dim3 grid((unsigned)(((N + 1) / 2 + rows - 1) / rows), 2, nlines);
     const size_t shm = dband_shared_bytes(N);
-    if (G == 1) {
-      if (dir == L2C)
-        launch_k(prof, k_direct_band<0, 1>, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
-      else
-        launch_k(prof, k_direct_band<1, 1>, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
-    } else {
-      if (dir == L2C)
-        launch_k(prof, k_direct_band<0, 4>, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
-      else
-        launch_k(prof, k_direct_band<1, 4>, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
-    }
+    const bool nine = dband_batch(N) == 9;
+    auto kernel = G == 1 ? (dir == L2C ? (nine ? k_direct_band<0, 1, 9> : k_direct_band<0, 1, 8>)
+                                       : (nine ? k_direct_band<1, 1, 9> : k_direct_band<1, 1, 8>))
+                         : (dir == L2C ? (nine ? k_direct_band<0, 4, 9> : k_direct_band<0, 4, 8>)
+                                       : (nine ? k_direct_band<1, 4, 9> : k_direct_band<1, 4, 8>));
+    launch_k(prof, kernel, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
     return;
   }
   launch_k(prof, k_direct_rows, dim3((unsigned)((N + 3) / 4), nlines), 256, 0, st, d_in, d_out,
