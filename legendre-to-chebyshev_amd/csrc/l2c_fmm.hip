@@ -3408,7 +3408,7 @@ static size_t dense_shared_bytes(int NRM, int LT, int NP) {
 // 2048 26 -> 24 us, but 1024 lines of 1024 19.4 -> 20.5 and 25.5.
 // Chunks from the last to the diagonal's instead of upwards: a 1200 x 900 array
 // through both axes and back 111 -> 96 us (the prefetch behind the last chunk
-// falls on lines just read), 2-norm error at N = 2000 3.2-4.6e-16 ->
+// falls on lines just read; 97 with the test for NaN and Inf), 2-norm error at N = 2000 3.2-4.6e-16 ->
 // 1.7-2.8e-16 (the FMM of the same lines 2.3-7.3e-16).
 constexpr int kGemmRT = 32, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmKP = kGemmKC + 2;
 constexpr size_t kGemmFewLines = 4096;
@@ -3427,7 +3427,8 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
   const int rt = (int)by, p = wave & 1;
   const size_t l0 = (size_t)bx * LT;
   size_t *toff = (size_t *)(sm + 2 * LT * KP);
-  int *tlen = (int *)(toff + LT);
+  int *tlen = (int *)(toff + LT), *flag = tlen + LT;
+  if (tid == 0) *flag = 0;
   if (tid < LT) {
     const size_t line = l0 + tid;
     toff[tid] = line < nlines ? line_off(lm, line) : 0;
@@ -3508,6 +3509,12 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     if (ks & 1) __builtin_amdgcn_sched_barrier(0);
   };
   for (int c0 = cl; c0 >= cf; c0 -= KC) {
+    if (c0 == cf) {
+      bool bad = false;
+#pragma unroll
+      for (int q = 0; q < QE; q++) bad |= !__builtin_isfinite(e[q]);
+      if (bad) *flag = 1;
+    }
     if constexpr (CONTIG) {
 #pragma unroll
       for (int q = 0; q < QL; q++) {
@@ -3525,12 +3532,35 @@ __device__ __forceinline__ void lines_gemm_tile(const double *__restrict__ in,
     fetch_in(cn);
     asm volatile("" : "+s"(cn));
     S0 = S1 = z;
+    // a NaN or Inf among the diagonal chunk's inputs: the row tile's diagonal
+    // block goes term by term, without the zeros below the diagonal
+    const bool slow = c0 == cf && __builtin_amdgcn_readfirstlane(*flag) != 0;
 #pragma unroll
-    for (int ks = KC / 4 - 1; ks >= 4; ks--) step(ks, cn);
+    for (int ks = KC / 4 - 1; ks >= 8; ks--) step(ks, cn);
+    if (!slow || wave < 2) {
+#pragma unroll
+      for (int ks = 7; ks >= 4; ks--) step(ks, cn);
+    }
     // the tile's second row tile starts 16 columns on (K_p is zero before)
-    if (c0 != cf || wave < 2) {
+    if (c0 != cf || (wave < 2 && !slow)) {
 #pragma unroll
       for (int ks = 3; ks >= 0; ks--) step(ks, cn);
+    }
+    if (slow) {
+      const int cb = 16 * (wave >> 1);
+      const double *x = sm + (p * LT + (lane & 15)) * KP + cb;
+#pragma unroll 1
+      for (int c = 15; c >= 0; c--) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int r = (lane >> 4) + 4 * v;
+          if (c >= r) {
+            const double k = load_one(Kr, 8 * (16 * (c & 3) + r), 512 * ((cf + cb + c) >> 2));
+            S0[v] += k * x[c];
+            S1[v] += k * x[16 * KP + c];
+          }
+        }
+      }
     }
     D0 += S0;
     D1 += S1;
@@ -3609,7 +3639,8 @@ __global__ void __launch_bounds__(kGemmNT) __attribute__((amdgpu_waves_per_eu(4)
 }
 
 size_t gemm_shared_bytes() {
-  return 8 * 2 * (size_t)kGemmLT * kGemmKP + kGemmLT * (sizeof(size_t) + sizeof(int));
+  return 8 * 2 * (size_t)kGemmLT * kGemmKP + kGemmLT * (sizeof(size_t) + sizeof(int)) +
+         sizeof(int);
 }
 
 // One transform by direct sums from the Lambda tables a, an, dn (those of a

@@ -98,3 +98,22 @@ def test_fmm_plan_lines(amd, orc, monkeypatch, N, B, strided):
         check(orc, x, y, d, 64, [0, B // 2, B - 1])
         z = run_lines(amd, fmm, x, d, strided, pad=1)
         assert max(relerr(y[r], z[r]) for r in range(B)) <= tol(N)
+
+
+@pytest.mark.parametrize("N,B", [(300, 40), (1000, 70), (1536, 33), (2048, 130)])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_not_finite(amd, monkeypatch, N, B, direction):
+    """A NaN or Inf on the FMM plans' dense route reaches the rows of its line
+    and parity at or before its place, all of them, and no other."""
+    announce(f"dense route, not finite N={N} B={B} dir={direction}")
+    monkeypatch.setenv("L2C_DIRECT_LINES", "0")
+    plan = amd.FMMPlan(N, 64, 18, direction)
+    for strided in (False, True):
+        for pos in (0, 1, 30, 31, 32, 33, N // 2, N // 2 + 17, N - 2, N - 1):
+            for val in (np.inf, -np.inf, np.nan):
+                x = np.random.default_rng(N).uniform(0.5, 1, (B, N))
+                x[B // 2, pos] = val
+                y = run_lines(amd, plan, x, direction, strided)
+                want = np.zeros((B, N), bool)
+                want[B // 2, pos % 2:pos + 1:2] = True
+                assert np.array_equal(~np.isfinite(y), want), (strided, pos, val)
