@@ -148,7 +148,8 @@ struct BandPtr {
 constexpr int kBT = 2;  // products in flight before their sums
 // One trip of 16 columns from column tb on; X, P of the trip's first quad are
 // in XA, PA, and on return those of the next trip's.  The trip's 31 values of
-// H are scalar loads (hp: the head, 16 zeros before it).  KIND 0: as it is; 1:
+// H are scalar loads (hp: the head, 16 zeros before it), the last eight half a trip
+// after the others: all 31 from the start on spilled scalars to scratch in k_up.  KIND 0: as it is; 1:
 // columns t >= len read x as zero; 2: that, and the terms left of the diagonal
 // (rho > t) are left out, for the trip from column 0.
 template <int KIND, bool S16>
@@ -157,7 +158,7 @@ __device__ __forceinline__ void band_trip(BandPtr &b, int s1, int s2, kdouble hp
                                           double (&acc)[16]) {
   double XB[4], PB[4], hw[32];
 #pragma unroll
-  for (int k = 1; k < 32; k++) hw[k] = hp[tb - 16 + k];
+  for (int k = 1; k < 24; k++) hw[k] = hp[tb - 16 + k];
   // x of the quad after the current one, P 16 further on
 #define QUAD_FETCH(X, P, Q)                                      \
   {                                                              \
@@ -200,6 +201,12 @@ __device__ __forceinline__ void band_trip(BandPtr &b, int s1, int s2, kdouble hp
   QUAD_FETCH(XB, PB, 0)
   QUAD_STEP(XA, PA, 0)
   QUAD_FETCH(XA, PA, 1)
+  {
+    int t8 = tb + 8;
+    asm volatile("" : "+s"(t8));
+#pragma unroll
+    for (int k = 0; k < 8; k++) hw[24 + k] = hp[t8 + k];
+  }
   QUAD_STEP(XB, PB, 1)
   QUAD_FETCH(XB, PB, 2)
   QUAD_STEP(XA, PA, 2)
