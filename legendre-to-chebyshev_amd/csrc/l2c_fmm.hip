@@ -1279,19 +1279,36 @@ __global__ void __launch_bounds__(64) k_slice_A(const double *__restrict__ A, in
   }
 }
 
+// One flat grid: tx ty work-groups for the blocks above lu (tx blocks, their
+// multipoles summed from the k_up contributions, ty shares of lpb lines) ahead of
+// mx work-groups (four blocks each) per share of the line groups.  As a launch of
+// their own (k_m2l) the top blocks took 19 us of 64 lines of 2^18, most of it
+// with the chip nearly idle.
+struct M2lGrid {
+  int tx, ty, lpb, mx;
+  SplitView sv;  // of the blocks above lu (precision form 1)
+};
 template <int FORM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_m2l_mma(Geo g, const double *__restrict__ A,
-                                                 const bf16x8 *__restrict__ Aq,
-                                                 const double *__restrict__ Asc,
-                                                 double *__restrict__ wsall, size_t wsstride,
-                                                 size_t nlines, int groups_per_wg) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_m2l_mma(
+    Geo g, const double *__restrict__ A, const bf16x8 *__restrict__ Aq,
+    const double *__restrict__ Asc, double *__restrict__ wsall, size_t wsstride, size_t nlines,
+    int groups_per_wg, M2lGrid mg) {
   extern __shared__ double sm[];
+  int bx = (int)blockIdx.x - mg.tx * mg.ty;
+  if (bx < 0) {  // a block above lu, lpb lines of it
+    const size_t line0 = (size_t)(blockIdx.x / mg.tx) * mg.lpb;
+    m2l_top<18>(g, A, wsall, wsstride, line0, (int)std::min<size_t>(mg.lpb, nlines - line0),
+                mg.sv, sm, blockIdx.x % mg.tx);
+    return;
+  }
+  const int by = bx / mg.mx;
+  bx -= by * mg.mx;
   constexpr int M = 18, M2 = 36, MM = 324, Mp = 19;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntop = (int)total_blocks(g.lu), ntot = (int)total_blocks(g.L);
-  const int B = ntop + (int)blockIdx.x * 4 + wave;
-  if (B >= ntot) return;  // no work-group barrier in this kernel
+  const int B = ntop + bx * 4 + wave;
+  if (B >= ntot) return;  // no work-group barrier below this point
   int lev = g.lu;
   while ((int)total_blocks(lev + 1) <= B) lev++;
   const int b = B - (int)total_blocks(lev);
@@ -1299,7 +1316,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   const size_t sofs = lay.w + (slot_base(lev) + 2 * (size_t)b + 2) * M2;  // S: w(2b+2), w(2b+3)
   const size_t oofs = lay.m2l + (slot_base(lev) + 2 * (size_t)b) * M2;    // out: chunks 2b, 2b+1
   const size_t ngroups = (nlines + 7) / 8;
-  const size_t gr0 = (size_t)blockIdx.y * groups_per_wg;
+  const size_t gr0 = (size_t)by * groups_per_wg;
   const size_t gr1 = std::min(ngroups, gr0 + groups_per_wg);
   const int n = lane & 15;
   if (FORM == 0) {
@@ -3954,25 +3971,24 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
       launch_k(p->prof, k_m2l<MT>, gm, kM2lNT, m2l_shared_bytes(g), st, g, p->t.A[dir], ws,
           wsstride, bpw, nlines, lpb, sv);
     } else {
-      // the blocks above lu (multipoles summed from the k_up contributions)
-      // as before; the rest on MFMA
-      if (ntop > 0)
-        launch_k(p->prof, k_m2l<MT>, dim3((unsigned)ntop, gm.y), kM2lNT, m2l_shared_bytes(g), st, g,
-            p->t.A[dir], ws, wsstride, bpw, nlines, lpb, sv);
+      // on MFMA the blocks at levels >= lu, beside them the blocks above lu
       const int nblk = ntot - ntop;
       const unsigned mx = (unsigned)((nblk + 3) / 4);
       const size_t ngroups = (nlines + 7) / 8;
       // line groups per work-group: one while the grid stays small, more so
       // that about 8192 work-groups share the lines
       const size_t gpw = std::max<size_t>(1, (mx * ngroups + 8191) / 8192);
-      const dim3 gmm(mx, (unsigned)((ngroups + gpw - 1) / gpw));
+      const M2lGrid mg{ntop, ntop ? (int)gm.y : 0, lpb, (int)mx, sv};
+      const dim3 gmm((unsigned)(mg.tx * mg.ty + mx * ((ngroups + gpw - 1) / gpw)));
+      const size_t top = 8 * (size_t)(m2l_wave_lds(18) + kM2lNT);
       if (p->precision == 2) {
         const DevTables::Slices &sl = p->t.sl[dir];
-        launch_k(p->prof, k_m2l_mma<2>, gmm, 256, 0, st, g, p->t.A[dir], (const bf16x8 *)sl.q,
-            sl.sc, ws, wsstride, nlines, (int)gpw);
+        launch_k(p->prof, k_m2l_mma<2>, gmm, 256, top, st, g, p->t.A[dir], (const bf16x8 *)sl.q,
+            sl.sc, ws, wsstride, nlines, (int)gpw, mg);
       } else {
-        launch_k(p->prof, k_m2l_mma<0>, gmm, 256, 4 * 3 * 18 * 19 * sizeof(double), st, g,
-            p->t.A[dir], nullptr, nullptr, ws, wsstride, nlines, (int)gpw);
+        launch_k(p->prof, k_m2l_mma<0>, gmm, 256,
+            std::max(top, 4 * 3 * 18 * 19 * sizeof(double)), st, g, p->t.A[dir], nullptr, nullptr,
+            ws, wsstride, nlines, (int)gpw, mg);
       }
     }
     prof_end(p->prof, st);
