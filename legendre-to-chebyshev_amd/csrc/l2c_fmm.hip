@@ -3804,8 +3804,11 @@ static int launch_direct_lines(const direct_plan_s *dp, const double *d_in, doub
 // Whether a call of nlines lines runs its M2L below lu on MFMA (precision
 // form 2, or FP64 MFMA for line calls from m2l_mma_lines lines on).
 static bool m2l_on_mfma(const fmm_plan_s *p, size_t nlines) {
-  return p->geo.M == 18 && (p->precision == 2 ||
-                            (p->m2l_mma_lines > 0 && nlines >= (size_t)p->m2l_mma_lines));
+  if (p->geo.M != 18) return false;
+  if (p->precision == 2) return true;
+  const int t = p->m2l_mma_lines;
+  const size_t lines = t >= 0 ? (size_t)t : p->geo.L >= 8 && p->geo.L <= 10 ? 8 : 32;
+  return lines > 0 && nlines >= lines;
 }
 // The work-group geometry of a call: single-line calls take geo1, line
 // calls geo (the MFMA M2L forms, whose form-2 tables are cut at geo's lu,

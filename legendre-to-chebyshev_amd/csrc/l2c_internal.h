@@ -291,11 +291,13 @@ struct fmm_plan_s {
   // the blocks at levels >= lu as BF16 slices on MFMA (FP32 accumulation,
   // FP64 recombination)
   int precision = 0;
-  // M2L of levels >= lu on FP64 MFMA for calls of at least this many lines
-  // (0: never; from 32 lines on the MFMA form is faster: the uneven batch of
-  // 4096 transforms 14.0 -> 14.9 M/s, while 8 lines of 2^20 lose 244 -> 259
-  // us); L2C_M2L_MMA sets it at plan creation
-  int m2l_mma_lines = 32;
+  // M2L of levels >= lu on FP64 MFMA for calls of at least this many lines (0:
+  // never; L2C_M2L_MMA sets it at plan creation).  By default (-1) 32, and 8
+  // for trees of 8 to 10 levels.  us per call, VALU / MFMA, s = 64: 8 lines of
+  // 2^13 17.2 / 18.8, 24 of 2^13 21.2 / 22.1, 8 of 2^15 21.8 / 22.9, 24 33.7 / 33.0,
+  // 8 of 2^16 25.9 / 25.8, 16 39.4 / 36.6, 8 of 2^17 42.9 / 37.0, 16 63.7 / 58.4,
+  // 8 of 2^18 61.0 / 59.3, 24 146 / 144, 8 of 2^20 204 / 210
+  int m2l_mma_lines = -1;
   // near field of plans with M = 18 and s <= 64: 0 (default) work-groups of the
   // k_up launch, 1 a k_band launch of its own, 2 that for calls of several
   // lines with L >= 10; L2C_DOWN_SPLIT
