@@ -557,11 +557,14 @@ static void destroy_fmm(fmm_plan_s *p) {
 // until the work-group's LDS fits the budget.
 // single: the cuts of single-line calls, else those of line calls.  Line
 // calls (their grids hold every line's work-groups) take the largest
-// subtrees; single transforms take cuts that grow with the depth, gu = gd =
-// (L - 4) / 2 within [1, 4] (gd >= 2 for k_far and k_down8r), measured best at
-// L = 4 ... 12 (s = 64: 2^16 23.1 us at (2, 2) against 26.8 us at (4, 4);
-// 2^18 26.6 against 28.6 us at (3, 3); 2^20 (4, 4) best), while line calls
-// lose with them (64 lines of 2^16: 174 K against 432 K lines/s).
+// subtrees; single transforms take cuts that grow with the depth: with k_far gu =
+// (L - 2) / 2 in [1, 4] and gd = (L - 3) / 2 in [2, 4], else gu = gd = (L - 4) / 2 (gd
+// >= 2 for k_down8r).  us per call (gu, gd), best of all / (L - 4) / 2 with k_far: L
+// = 8 2^16 C2L 17.3 (3, 2) / 17.6; L = 9 2^17 17.2 (3, 2), 17.3 (3, 3) / 19.9; L = 10
+// 100,000 (s = 25) 17.9 (4, 3) / 19.5, 2^18 21.0 (4, 3) / 21.4; L = 11 200,000 (s =
+// 25) 23.4 (4, 4) / 27.1, 2^19 31.2 (4, 3), 31.7 (4, 4) / 33.2; L = 12 (4, 4) both.
+// Line calls lose with the small cuts (64 lines of 2^16: 174 K against 432 K
+// lines/s).
 static bool choose_cuts(Geo &g, bool single) {
   const int Lm1 = g.L - 1;
   // k_far (M = 18, s <= 64) and k_down8 (s = 16, 32, 64): 16 leaf chunks and
@@ -574,8 +577,8 @@ static bool choose_cuts(Geo &g, bool single) {
   const int dcut = (g.L - 4) / 2;
   int gu = 4, gd = wide ? 4 : 3;
   if (single) {
-    gu = std::max(1, std::min(4, dcut));
-    if (wide) gd = std::max(2, std::min(4, dcut));
+    gu = std::max(1, std::min(4, g.far ? (g.L - 2) / 2 : dcut));
+    if (wide) gd = std::max(2, std::min(4, g.far ? (g.L - 3) / 2 : dcut));
   }
   if (const char *e = getenv("L2C_GU")) gu = atoi(e);
   if (const char *e = getenv("L2C_GD")) gd = atoi(e);
