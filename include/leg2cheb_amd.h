@@ -275,7 +275,8 @@ int l2c_batch_get_class(const l2c_batch_plan *bp, size_t i, l2c_batch_class *out
 /* Precision form of a plan.  0 = plain FP64 (default).  1 = split storage:
  * the M2L matrices are stored per coefficient as FP64, FP32, BF16 or dropped,
  * chosen against 2^-29, 2^-44 and 2^-53 of each block's largest coefficient;
- * all arithmetic stays FP64.  2 = split products (M = 18): the M2L products
+ * all arithmetic stays FP64 (M = 18: line calls of 32 lines and more read the
+ * blocks below the top levels from the FP64 matrices).  2 = split products (M = 18): the M2L products
  * of the blocks below the top levels run as BF16 slices on the matrix cores
  * (each operand scaled by powers of two and cut into 6 slices of 8 bits,
  * every anti-diagonal of slice pairs accumulated exactly in FP32,

@@ -3807,7 +3807,10 @@ static bool m2l_on_mfma(const fmm_plan_s *p, size_t nlines) {
   if (p->geo.M != 18) return false;
   if (p->precision == 2) return true;
   const int t = p->m2l_mma_lines;
-  const size_t lines = t >= 0 ? (size_t)t : p->geo.L >= 8 && p->geo.L <= 10 ? 8 : 32;
+  // (form 1 keeps to its own records up to 31 lines: the bound of 8 was timed
+  // against the FP64 matrices)
+  const bool mid = p->precision == 0 && p->geo.L >= 8 && p->geo.L <= 10;
+  const size_t lines = t >= 0 ? (size_t)t : mid ? 8 : 32;
   return lines > 0 && nlines >= lines;
 }
 // The work-group geometry of a call: single-line calls take geo1, line

@@ -119,3 +119,23 @@ def test_m2l_rows_across_lanes(amd, monkeypatch, N, lines):
             p.synchronize()
             outs.append(dout.download())
         assert np.array_equal(outs[0], outs[1]), d
+
+
+@pytest.mark.parametrize("N,lines", [(1 << 16, 8), (1 << 16, 31), (1 << 17, 9), (100000, 12)])
+def test_split_form_lines(amd, N, lines):
+    """Form 1 in calls of 8 to 31 lines of trees of 8 to 10 levels reads its own
+    records, as calls of fewer lines do: its first lines bit for bit (the M2L on
+    MFMA, from the FP64 matrices, sums in another order)."""
+    announce(f"form 1 lines N={N} lines={lines}")
+    p = amd.FMMPlan(N, 64, 18, amd.BOTH)
+    p.set_precision(1)
+    x = np.random.default_rng(N + lines).uniform(-1, 1, lines * N)
+    din, dout = amd.DeviceBuffer(x.size), amd.DeviceBuffer(x.size)
+    din.upload(x)
+    for d in (0, 1):
+        outs = []
+        for n in (lines, 5):
+            p.execute_lines_device(din.ptr, dout.ptr, d, n, n, N, 0, 1)
+            p.synchronize()
+            outs.append(dout.download(5 * N))
+        assert np.array_equal(outs[0], outs[1]), d
