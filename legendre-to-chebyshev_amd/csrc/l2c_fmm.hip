@@ -60,6 +60,22 @@ __device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int v
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
 }
 
+// The (group, line) of this work-group in a launch of grid (groups, lines[, z]).
+// In general (blockIdx.x, blockIdx.y).  ACROSS, lines that lie side by side: an HBM or L2 line holds one element of each of 8 or 16 of them, so
+// the work-groups of one group of all lines run one after the other on one XCD
+// (work-groups go to the eight XCDs in turn), each fetching and writing what its
+// neighbours' elements share with its own while that is in the XCD's L2.
+struct Place {
+  unsigned grp, line;
+};
+template <bool ACROSS>
+__device__ __forceinline__ Place place() {
+  if (!ACROSS) return {blockIdx.x, blockIdx.y};
+  const unsigned nl = gridDim.y, n = gridDim.x * nl, id = blockIdx.x + gridDim.x * blockIdx.y;
+  const unsigned t = (id & 7) * (n >> 3) + std::min(id & 7, n & 7) + (id >> 3);
+  return {t / nl, t % nl};
+}
+
 struct WsLayout {
   size_t w, part, m2l, total;
 };
@@ -684,17 +700,17 @@ __device__ __forceinline__ void up18_group(const double *__restrict__ in, const 
                                            const double *__restrict__ U,
                                            const double *__restrict__ P,
                                            double *__restrict__ wsall, size_t wsstride, int j,
-                                           double *sm) {
+                                           unsigned line, double *sm) {
   constexpr int M = 18, M2 = 36, MM = M * M;
   const int s = g.s, G = 1 << g.gu;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, kq = lane >> 4;
   const size_t es = lm.es, base = (size_t)j * G * 2 * s;
-  const size_t Nl = (size_t)line_len(lm, blockIdx.y, g.N);  // zeros past the line's end
-  const double *src = in + line_off(lm, blockIdx.y) + base * es;
+  const size_t Nl = (size_t)line_len(lm, line, g.N);  // zeros past the line's end
+  const double *src = in + line_off(lm, line) + base * es;
   const int nl = base < Nl ? (int)std::min<size_t>(Nl - base, (size_t)G * 2 * s) : 0;
-  double *ws = wsall + blockIdx.y * wsstride;
+  double *ws = wsall + line * wsstride;
   const WsLayout lay = ws_layout(g);
   const Up18Lds ly = up18_lds(g);
   double *xs = sm, *w0 = sm + ly.w0, *w1 = sm + ly.w1;
@@ -850,19 +866,20 @@ struct BandArgs {
   double *out;
   const double *tab, *head;
 };
-template <bool S16, int G>
+template <bool S16, int G, bool ACROSS>
 __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up(
     const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
     const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
     size_t wsstride, BandArgs ba) {
   extern __shared__ double sm[];
+  const Place w = place<ACROSS>();
   if (blockIdx.z + 1 == gridDim.z) {
-    if ((int)blockIdx.x < 4 << g.lu)
-      up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, blockIdx.x, sm);
+    if ((int)w.grp < 4 << g.lu)
+      up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, w.grp, w.line, sm);
   } else {
-    const size_t off = line_off(lm, blockIdx.y);
-    band_group<S16, G>(in + off, ba.out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
-                    blockIdx.x, 0, ba.tab, ba.head, sm);
+    const size_t off = line_off(lm, w.line);
+    band_group<S16, G>(in + off, ba.out + off, lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, 0,
+                       ba.tab, ba.head, sm);
   }
 }
 
@@ -2647,14 +2664,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
 // downward pass (down_split; raw sums, the C2L diagonal included, over the
 // output; k_far adds the far field and scales, src/C/leg2cheb.c:1467-1483 and
 // the band scaling of :236-535).  Grid (band groups, lines), 256 threads.
-template <bool S16>
+template <bool S16, bool ACROSS>
 __global__ void __launch_bounds__(kBandNT) __attribute__((amdgpu_waves_per_eu(4))) k_band(
     const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g, int dir, int scale,
     const double *__restrict__ tab, const double *__restrict__ head) {
   extern __shared__ double sm[];
-  const size_t off = line_off(lm, blockIdx.y);
-  band_group<S16, 16>(in + off, out + off, lm.es, line_len(lm, blockIdx.y, g.N), g, dir,
-                  (int)blockIdx.x, scale, tab, head, sm);
+  const Place w = place<ACROSS>();
+  const size_t off = line_off(lm, w.line);
+  band_group<S16, 16>(in + off, out + off, lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, scale,
+                      tab, head, sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -2683,6 +2701,7 @@ __host__ __device__ inline FarLds far_lds(const Geo &g) {
 size_t far_shared_bytes(const Geo &g) { return 8 * (size_t)far_lds(g).total; }
 bool far_eligible(const Geo &g) { return g.M == 18 && g.s <= kBandMaxS; }
 
+template <bool ACROSS>
 __global__ void __launch_bounds__(kFarNT) __attribute__((amdgpu_waves_per_eu(4))) k_far(
     double *__restrict__ out, LineMap lm, Geo g, int dir, const double *__restrict__ wsall,
     size_t wsstride, const double *__restrict__ Dg, const double *__restrict__ Qg,
@@ -2690,16 +2709,17 @@ __global__ void __launch_bounds__(kFarNT) __attribute__((amdgpu_waves_per_eu(4))
   extern __shared__ double sm[];
   constexpr int M = 18, M2 = 36, MM = M * M;
   const int s = g.s, N = g.N;
-  const int Nl = line_len(lm, blockIdx.y, N);
-  const int G = 1 << g.gd, Rr = blockIdx.x;
+  const Place w = place<ACROSS>();
+  const int Nl = line_len(lm, w.line, N);
+  const int G = 1 << g.gd, Rr = w.grp;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t row0 = (size_t)Rr * G * 2 * s;
   if (row0 >= (size_t)Nl) return;  // the whole work-group
   const int nr = (int)std::min((size_t)G * 2 * s, (size_t)Nl - row0);
   const size_t es = lm.es;
-  double *dst = out + line_off(lm, blockIdx.y) + row0 * es;
-  const double *m2l = wsall + blockIdx.y * wsstride + ws_layout(g).m2l;
+  double *dst = out + line_off(lm, w.line) + row0 * es;
+  const double *m2l = wsall + w.line * wsstride + ws_layout(g).m2l;
   const FarLds ly = far_lds(g);
   double *cres = sm, *mres = sm + ly.mres, *qp = sm + ly.qp, *ob = sm + ly.ob;
 
@@ -3877,7 +3897,9 @@ static void launch_down8(fmm_plan_s *p, const Geo &g, const double *d_in, double
 static void launch_band(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out, size_t dir,
                         const LineMap &lm, size_t nlines, hipStream_t st, int scale, int slot) {
   prof_begin(p->prof, slot, st);
-  launch_k(p->prof, (g.s & 15) == 0 ? k_band<true> : k_band<false>,
+  const bool s16 = (g.s & 15) == 0;
+  launch_k(p->prof, lm.across ? (s16 ? k_band<true, true> : k_band<false, true>)
+                              : (s16 ? k_band<true, false> : k_band<false, false>),
            dim3(band_groups(g, 16), (unsigned)nlines), kBandNT, band_shared_bytes(g, 16), st, d_in,
            d_out, lm, g, (int)dir, scale, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
   prof_end(p->prof, st);
@@ -3886,7 +3908,7 @@ static void launch_band(fmm_plan_s *p, const Geo &g, const double *d_in, double 
 static void launch_far(fmm_plan_s *p, const Geo &g, double *d_out, size_t dir, const LineMap &lm,
                        size_t nlines, hipStream_t st, double *ws, int slot) {
   prof_begin(p->prof, slot, st);
-  launch_k(p->prof, k_far, dim3((unsigned)((size_t)4 << g.ld), (unsigned)nlines), kFarNT,
+  launch_k(p->prof, lm.across ? k_far<true> : k_far<false>, dim3((unsigned)((size_t)4 << g.ld), (unsigned)nlines), kFarNT,
            far_shared_bytes(g), st, d_out, lm, g, (int)dir, ws, ws_doubles(g), p->t.D, p->t.Q,
            p->t.T);
   prof_end(p->prof, st);
@@ -3936,16 +3958,19 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
   if (!band_only) {
     const bool s16 = (g.s & 15) == 0;
     dim3 gu(4u << g.lu, (unsigned)nlines);
-    const bool b8 = fuse && band_by_8(g, nlines);
+    const bool b8 = fuse && !lm.across && band_by_8(g, nlines);
     if (fuse) gu = dim3(std::max(gu.x, band_groups(g, b8 ? 8 : 16)), gu.y, 2);
     const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]};
     prof_begin(p->prof, K_UP_SUBTREE, st);
     if (MT == 18 && up18_eligible(g)) {
       const size_t shu = std::max(8 * (size_t)up18_lds(g).total,
                                   fuse ? band_shared_bytes(g, b8 ? 8 : 16) : 0);
-      launch_k(p->prof, b8 ? (s16 ? k_up<true, 8> : k_up<false, 8>)
-                           : (s16 ? k_up<true, 16> : k_up<false, 16>), gu, kUpNT, shu, st, d_in, lm, g, (int)dir,
-               p->t.T, p->t.U, p->t.P, ws, wsstride, bu);
+      // (calls with lines in turn are past band_by_8's bounds)
+      auto kernel = lm.across ? (s16 ? k_up<true, 16, true> : k_up<false, 16, true>)
+                    : b8      ? (s16 ? k_up<true, 8, false> : k_up<false, 8, false>)
+                              : (s16 ? k_up<true, 16, false> : k_up<false, 16, false>);
+      launch_k(p->prof, kernel, gu, kUpNT, shu, st, d_in, lm, g, (int)dir, p->t.T, p->t.U, p->t.P,
+               ws, wsstride, bu);
     } else if (MT > 0 && g.gu >= 3 && nlines <= 8) {
       launch_k(p->prof, k_up_any<MT, MT != 0>, gu, kUpNT, up_shared_bytes(g), st, d_in, lm, g,
                (int)dir, p->t.T, p->t.U, p->t.P, ws, wsstride);
@@ -4139,6 +4164,20 @@ static bool dense_lines(const fmm_plan_s *p, size_t dir, size_t nlines) {
   return p->d_K[dir] && p->precision == 0 && nlines >= (p->N <= 1536 ? 2 : 128);
 }
 
+// Whether the FMM kernels of a line call of N elements a line take neighbouring
+// lines in turn (place): where a line's neighbour lies nearer than its own next
+// element and the call is too large for the caches to keep what the lines share
+// from one line's work-groups to the next's.  Lines side by side, group by group /
+// line by line, s = 64 unless stated (us): 40 lines of 2^18 307 / 563, 100 807 /
+// 1530, 8 of 2^20 245 / 512, 24 of 140,000 (s = 35) 143 / 204, 500 of 33,000 (s =
+// 33) 712 / 777, 8 of 2^18 72 / 79; even at 8 of 140,000 57.4 / 57.3 and 24 of
+// 70,000 83 / 84; below, the division costs 1 to 2 %: 8 of 2500 18.1 / 17.6, 24 of
+// 16,384 31.3 / 31.0.  (With the band inside the downward kernel, whose passes over
+// a strided array are two fewer: 400, 1037, 338, 246, 923 and 83.)
+static bool lines_across(const LineMap &lm, size_t N, size_t nlines) {
+  return nlines > 1 && (lm.n0 > 1 ? lm.ls0 : lm.ls1) < lm.es && N * nlines >= (size_t)1 << 20;
+}
+
 int run_lines(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size_t nlines,
               size_t n0, size_t ls0, size_t ls1, size_t es, hipStream_t st) {
   prof_step(p->prof);
@@ -4169,6 +4208,7 @@ int run_lines(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size
   }
   // lines go in grid.y: at most 65535 per launch, each chunk reusing the
   // front of the plan's line workspace
+  lm.across = lines_across(lm, p->N, nlines);
   for (size_t l0 = 0; l0 < nlines; l0 += 65535) {
     lm.l0 = l0;
     if (launch_fmm(p, d_in, d_out, dir, lm, std::min<size_t>(65535, nlines - l0), st, 0))
@@ -4240,6 +4280,7 @@ static int run_lines_scratch(fmm_plan_s *p, double *scr, const double *d_in, dou
               std::to_string(kScratchDoubles * sizeof(double)) + "-byte scratch");
     return -1;
   }
+  lm.across = lines_across(lm, p->N, nlines);
   for (size_t l0 = 0; l0 < nlines; l0 += per) {
     lm.l0 = l0;
     const size_t nl = std::min(per, nlines - l0);

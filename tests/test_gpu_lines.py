@@ -229,3 +229,32 @@ def test_field_256_cube_with_vectors(amd, orc):
     for t in (0, nv - 1):
         ref = ov.execute(uv[t * nvec:(t + 1) * nvec], 0)
         assert relerr(gv[t * nvec:(t + 1) * nvec], ref) <= tol(nvec), t
+
+
+@pytest.mark.parametrize("split", [0, 1])
+@pytest.mark.parametrize("N,lines,inner", [(2500, 421, 421), (3000, 360, 24), (33001, 33, 11),
+                                           (140001, 9, 9), (1 << 17, 8, 8), (1 << 16, 17, 1)])
+def test_side_by_side_lines(amd, monkeypatch, split, N, lines, inner):
+    """Large calls of FMM plans whose lines lie side by side run group by group
+    over the lines (line and group counts that are no multiples of eight among
+    them): every line as from the call on the same lines back to back, bit for bit,
+    with the band in the upward launch and apart, from both entry points."""
+    announce(f"side by side N={N} lines={lines} inner={inner} split={split}")
+    assert N * lines >= 1 << 20
+    if split:
+        monkeypatch.setenv("L2C_DOWN_SPLIT", "1")
+    p = amd.FMMPlan(N, 64, 18, amd.BOTH)
+    x = np.random.default_rng(N + lines).uniform(-1, 1, (lines // inner, inner, N))
+    din, dout = amd.DeviceBuffer(x.size), amd.DeviceBuffer(x.size)
+    for d in (0, 1):
+        din.upload(x.ravel())
+        p.execute_lines_device(din.ptr, dout.ptr, d, lines, lines, N, 0, 1)
+        p.synchronize()
+        ref = dout.download().reshape(x.shape)
+        din.upload(np.ascontiguousarray(np.swapaxes(x, 1, 2)).ravel())
+        for fn in (amd.lib().l2c_execute_lines_device, amd.lib().l2c_execute_lines_device_noalloc):
+            dout.upload(np.full(x.size, 7.0))
+            assert fn(p.plan, din.ptr, dout.ptr, d, lines, inner, 1, inner * N, inner, None) == 0
+            p.synchronize()
+            g = np.swapaxes(dout.download().reshape(lines // inner, N, inner), 1, 2)
+            assert np.array_equal(g, ref), d
