@@ -60,20 +60,27 @@ __device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int v
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
 }
 
-// The (group, line) of this work-group in a launch of grid (groups, lines[, z]).
-// In general (blockIdx.x, blockIdx.y).  ACROSS, lines that lie side by side: an HBM or L2 line holds one element of each of 8 or 16 of them, so
-// the work-groups of one group of all lines run one after the other on one XCD
-// (work-groups go to the eight XCDs in turn), each fetching and writing what its
-// neighbours' elements share with its own while that is in the XCD's L2.
+// The (group, line) of work-group id of n groups of each of nl lines.  In general
+// the groups of a line follow each other.  ACROSS, lines that lie side by side: an HBM
+// or L2 line holds one element of each of 8 or 16 of them, so the work-groups of one
+// group of all lines run one after the other on one XCD (work-groups go to the eight
+// XCDs in turn), each fetching and writing what its neighbours' elements share with
+// its own while that is in the XCD's L2.
 struct Place {
   unsigned grp, line;
 };
 template <bool ACROSS>
-__device__ __forceinline__ Place place() {
-  if (!ACROSS) return {blockIdx.x, blockIdx.y};
-  const unsigned nl = gridDim.y, n = gridDim.x * nl, id = blockIdx.x + gridDim.x * blockIdx.y;
+__device__ __forceinline__ Place place_of(unsigned id, unsigned n, unsigned nl) {
+  if (!ACROSS) return {id % n, id / n};
+  n *= nl;
   const unsigned t = (id & 7) * (n >> 3) + std::min(id & 7, n & 7) + (id >> 3);
   return {t / nl, t % nl};
+}
+// that of this work-group in a launch of grid (groups, lines)
+template <bool ACROSS>
+__device__ __forceinline__ Place place() {
+  if (!ACROSS) return {blockIdx.x, blockIdx.y};
+  return place_of<true>(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x, gridDim.y);
 }
 
 struct WsLayout {
@@ -862,18 +869,35 @@ __device__ __forceinline__ void up18_group(const double *__restrict__ in, const 
 // apart / together 2^16 15.5 / 10.8 us, 2^20 27.4 / 22.0, 64 lines of 2^18 254 /
 // 247.  Band groups behind the upward ones of each line: 256 lines of 2^15 220
 // us a call against 188.
+//
+// Shallow trees (L <= 4) have fewer band groups (nb) than upward ones, and work-groups
+// go to the eight XCDs in turn: padded to the upward groups' number, two of four on
+// a line of 3300, all of the band would fall to four XCDs.  Their line calls (UP_FLAT)
+// take a grid (nb + upward groups, lines) with the nb groups of every line first and
+// none empty: 3000 lines of 3300 (s = 52) 310 -> 211 us (of it 128 the band's and 92 the
+// upward groups' in launches of their own), the call 407 -> 301.  So do calls whose
+// lines lie side by side (UP_ACROSS).  UP_FLAT for all of them costs 0.3 % (the
+// division by the group count).
+enum { UP_PLAIN = 0, UP_FLAT = 1, UP_ACROSS = 2 };
 struct BandArgs {
   double *out;
   const double *tab, *head;
+  int nb;  // band groups of a line (0: the upward pass alone)
 };
-template <bool S16, int G, bool ACROSS>
+template <bool S16, int G, int ORDER>
 __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up(
     const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
     const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
     size_t wsstride, BandArgs ba) {
   extern __shared__ double sm[];
-  const Place w = place<ACROSS>();
-  if (blockIdx.z + 1 == gridDim.z) {
+  Place w{blockIdx.x, blockIdx.y};
+  bool band = blockIdx.z + 1 != gridDim.z;
+  if (ORDER != UP_PLAIN) {
+    const unsigned nl = gridDim.y, bands = ba.nb * nl, id = blockIdx.x + gridDim.x * blockIdx.y;
+    band = id < bands;
+    w = place_of<ORDER == UP_ACROSS>(band ? id : id - bands, band ? ba.nb : 4u << g.lu, nl);
+  }
+  if (!band) {
     if ((int)w.grp < 4 << g.lu)
       up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, w.grp, w.line, sm);
   } else {
@@ -3959,16 +3983,24 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
     const bool s16 = (g.s & 15) == 0;
     dim3 gu(4u << g.lu, (unsigned)nlines);
     const bool b8 = fuse && !lm.across && band_by_8(g, nlines);
-    if (fuse) gu = dim3(std::max(gu.x, band_groups(g, b8 ? 8 : 16)), gu.y, 2);
-    const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]};
+    const int nb = fuse ? (int)band_groups(g, b8 ? 8 : 16) : 0;
+    const int order = lm.across ? UP_ACROSS
+                      : fuse && !b8 && nlines > 1 && (unsigned)nb < gu.x ? UP_FLAT : UP_PLAIN;
+    if (order != UP_PLAIN)
+      gu.x += nb;
+    else if (fuse)
+      gu = dim3(std::max(gu.x, (unsigned)nb), gu.y, 2);
+    const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir], nb};
     prof_begin(p->prof, K_UP_SUBTREE, st);
     if (MT == 18 && up18_eligible(g)) {
       const size_t shu = std::max(8 * (size_t)up18_lds(g).total,
                                   fuse ? band_shared_bytes(g, b8 ? 8 : 16) : 0);
       // (calls with lines in turn are past band_by_8's bounds)
-      auto kernel = lm.across ? (s16 ? k_up<true, 16, true> : k_up<false, 16, true>)
-                    : b8      ? (s16 ? k_up<true, 8, false> : k_up<false, 8, false>)
-                              : (s16 ? k_up<true, 16, false> : k_up<false, 16, false>);
+      auto kernel =
+          order == UP_ACROSS ? (s16 ? k_up<true, 16, UP_ACROSS> : k_up<false, 16, UP_ACROSS>)
+          : order == UP_FLAT ? (s16 ? k_up<true, 16, UP_FLAT> : k_up<false, 16, UP_FLAT>)
+          : b8               ? (s16 ? k_up<true, 8, UP_PLAIN> : k_up<false, 8, UP_PLAIN>)
+                             : (s16 ? k_up<true, 16, UP_PLAIN> : k_up<false, 16, UP_PLAIN>);
       launch_k(p->prof, kernel, gu, kUpNT, shu, st, d_in, lm, g, (int)dir, p->t.T, p->t.U, p->t.P,
                ws, wsstride, bu);
     } else if (MT > 0 && g.gu >= 3 && nlines <= 8) {

@@ -258,3 +258,31 @@ def test_side_by_side_lines(amd, monkeypatch, split, N, lines, inner):
             p.synchronize()
             g = np.swapaxes(dout.download().reshape(lines // inner, N, inner), 1, 2)
             assert np.array_equal(g, ref), d
+
+
+@pytest.mark.parametrize("N,maxs,lines", [(260, 64, 200), (130, 16, 33), (600, 64, 131), (700, 32, 3),
+                                          (1100, 50, 90), (3300, 64, 40), (4096, 64, 77),
+                                          (2100, 33, 64)])
+def test_shallow_tree_lines(amd, orc, monkeypatch, N, maxs, lines):
+    """Line calls of trees of up to four levels, whose upward launch holds the band
+    groups of all lines first and then the upward groups: as with the band in a launch
+    of its own, bit for bit, and the first and last line against the oracle."""
+    announce(f"shallow tree N={N} maxs={maxs} lines={lines}")
+    p0 = amd.FMMPlan(N, maxs, 18, amd.BOTH)
+    monkeypatch.setenv("L2C_DOWN_SPLIT", "1")
+    p1 = amd.FMMPlan(N, maxs, 18, amd.BOTH)
+    op = orc.FMMPlan(N, maxs, 18, orc.BOTH)
+    x = np.random.default_rng(N + lines).uniform(-1, 1, lines * N)
+    din, dout = amd.DeviceBuffer(x.size), amd.DeviceBuffer(x.size)
+    din.upload(x)
+    for d in (0, 1):
+        outs = []
+        for p in (p0, p1):
+            dout.upload(np.full(x.size, 7.0))
+            p.execute_lines_device(din.ptr, dout.ptr, d, lines, lines, N, 0, 1)
+            p.synchronize()
+            outs.append(dout.download())
+        assert np.array_equal(*outs), d
+        for k in (0, lines - 1):
+            ref = op.execute(np.ascontiguousarray(x[k * N:(k + 1) * N]), d)
+            assert relerr(outs[0][k * N:(k + 1) * N], ref) <= tol(N)
