@@ -2972,6 +2972,7 @@ __global__ void __launch_bounds__(256) k_direct(const double *__restrict__ in,
 // term order per lane, and add their partial sums across the wave.  Grid
 // ((N + 3) / 4, lines): four rows per work-group, line blockIdx.y of lm
 // (unpacked maps).
+template <int QR>
 __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ in,
                                                      double *__restrict__ out, LineMap lm, int N,
                                                      int dir, const double *__restrict__ a,
@@ -2983,8 +2984,12 @@ __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ 
   const double *u = in + off;
   const size_t es = lm.es;
   // QR terms' loads in flight at once (a term past the end reads the lane's
-  // first one and adds nothing), and what the C2L diagonal needs before them
-  constexpr int QR = 4;
+  // first one and adds nothing), and what the C2L diagonal needs before them.
+  // One line (three, a few waves on each SIMD: latency): 1500 4.0 us against 4.25 with
+  // one at a time, 2200 5.0 / 5.2, 3072 6.6 / 6.8; four waste more of a row's last
+  // batch (2200 5.45, 1000 3.65 / 3.55, though 2500 5.55 / 5.65).  Several lines (one:
+  // issue): 30 of 300 4.4 us against 5.8 with four, 2 of 1800 5.7 / 6.6, 8 of 1000 side
+  // by side 11.9 / 12.9.
   double ud = 0, pd = 0;
   if (dir == C2L) {
     ud = u[(size_t)i * es];
@@ -3733,8 +3738,9 @@ static void launch_direct_one(Prof *prof, int N, size_t dir, const double *a, co
     launch_k(prof, kernel, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
     return;
   }
-  launch_k(prof, k_direct_rows, dim3((unsigned)((N + 3) / 4), nlines), 256, 0, st, d_in, d_out,
-           lm, N, (int)dir, a, an, dn);
+  launch_k(prof, nlines > 1 ? k_direct_rows<1> : k_direct_rows<3>,
+           dim3((unsigned)((N + 3) / 4), nlines), 256, 0, st, d_in, d_out, lm, N, (int)dir, a, an,
+           dn);
 }
 
 // k_direct over nlines lines of map lm (one launch for any number of lines);
