@@ -117,3 +117,19 @@ def test_not_finite(amd, monkeypatch, N, B, direction):
                 want = np.zeros((B, N), bool)
                 want[B // 2, pos % 2:pos + 1:2] = True
                 assert np.array_equal(~np.isfinite(y), want), (strided, pos, val)
+
+
+@pytest.mark.parametrize("N,maxs", [(200, 64), (1000, 64), (1201, 36)])
+def test_blocks_of_planned_directions(amd, monkeypatch, N, maxs):
+    """The parity blocks of a plan of one direction and of both, direct plans and FMM
+    plans: the same results bit for bit, and no results in a direction not planned."""
+    announce(f"dense blocks by direction N={N} maxs={maxs}")
+    monkeypatch.delenv("L2C_DIRECT_MAXN", raising=False)
+    monkeypatch.setenv("L2C_DIRECT_LINES", "0")
+    x = np.random.default_rng(N).uniform(-1, 1, (50, N))
+    both = amd.FMMPlan(N, maxs, 18, amd.BOTH)
+    for d in (0, 1):
+        one = amd.FMMPlan(N, maxs, 18, d)
+        assert np.array_equal(run_lines(amd, one, x, d, False), run_lines(amd, both, x, d, False))
+        with pytest.raises(amd.L2CError):
+            run_lines(amd, one, x, 1 - d, False)
