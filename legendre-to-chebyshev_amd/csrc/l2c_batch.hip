@@ -138,7 +138,8 @@ static int make_candidate(l2c_batch_plan_s *bp, BatchClass &c, int method, size_
     if (c.dp) c.dp->dense_tile = variant;
     return c.dp ? 0 : -1;
   }
-  c.fp = create_fmm_impl(c.n_max, s, bp->M, bp->direction, 0, 0, 0);
+  // (run_packed never takes the dense blocks of an FMM plan)
+  c.fp = create_fmm_impl(c.n_max, s, bp->M, bp->direction, 0, 0, 0, false);
   if (!c.fp) return -1;
   if (c.fp->L < 1 || c.fp->s != s || !c.fp->geo.fast || reserve_lines(c.fp, c.idx.size())) {
     destroy_class_plans(c);

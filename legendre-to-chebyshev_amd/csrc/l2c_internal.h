@@ -416,7 +416,8 @@ size_t ws_doubles(const Geo &g);  // execute workspace per line
 size_t flops_direct(size_t N, size_t dir, size_t precompute);
 // implemented in l2c_plan.hip
 direct_plan_s *make_direct(size_t N, size_t direction, size_t precompute);
+// dense: the parity blocks of line calls for plans of N <= dense_max_n
 fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, size_t lagrange,
-                            size_t precompute, size_t v);
+                            size_t precompute, size_t v, bool dense = true);
 void destroy_direct(direct_plan_s *dp);
 }  // namespace l2c

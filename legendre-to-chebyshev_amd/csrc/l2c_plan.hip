@@ -617,7 +617,7 @@ static bool choose_cuts(Geo &g, bool single) {
 }
 
 fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, size_t lagrange,
-                            size_t precompute, size_t v) {
+                            size_t precompute, size_t v, bool dense) {
   clear_error();
   if (N == 0 || maxs == 0 || direction > 2) {
     set_error("create_fmm: need N > 0, maxs > 0, direction in {0,1,2}");
@@ -710,7 +710,7 @@ fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, s
     destroy_fmm(p);
     return nullptr;
   }
-  if (N <= (size_t)p->dense_max_n && N <= (size_t)p->direct_max_n &&
+  if (dense && N <= (size_t)p->dense_max_n && N <= (size_t)p->direct_max_n &&
       build_dense(N, direction, p->t.a, p->t.an, p->t.dn, p->d_K, &p->NPP, st, acct)) {
     destroy_fmm(p);
     return nullptr;
