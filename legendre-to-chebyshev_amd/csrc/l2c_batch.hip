@@ -192,20 +192,25 @@ static double time_class(l2c_batch_plan_s *bp, const BatchClass &c, size_t dir) 
   return best;
 }
 
-// Candidates of size class k: the direct sum up to 2^13 (for 32 < 2^k <= 256
-// with each dense kernel: one tile of all rows, or row tiles), the FMM with
+// Candidates of a size class k of count lines: the direct sum up to 2^13, the FMM with
 // s = 16, 32, 64 where the depth L = k - log2(s) - 2 is at least 1, each with
-// the fused and the split downward pass.
+// the fused and the split downward pass.  Classes of 32 < 2^k <= 256 have two dense
+// kernels.  The tiled one runs in one launch with the batch's other dense classes, the
+// whole-line one in a launch of its own, so it is a candidate only past the lines that
+// the tiled one takes by itself (dense_tiled); below, the two come out even alone and a
+// batch that takes the whole-line one is slower: 889 lines of 20 to 1018 62 to 69 us a
+// replay against 44, 838 of 106 to 1075 71 to 75 against 52, 932 of 251 to 2772 73 to 76
+// against 62.
 struct Cand {
   int method;
   size_t s;
   int variant;
 };
-static std::vector<Cand> candidates(int k) {
+static std::vector<Cand> candidates(int k, size_t count) {
   std::vector<Cand> v;
   if (k <= 13) {
     if (k > 5 && k <= 8) {
-      v.push_back({0, 0, 1});
+      if (count > kGemmFewLines) v.push_back({0, 0, 1});
       v.push_back({0, 0, 2});
     } else {
       v.push_back({0, 0, 0});
@@ -476,7 +481,7 @@ static l2c_batch_plan_s *create_batch_impl(const size_t *n, size_t count, size_t
     }
     double best = -1, second = -1;
     Cand pick{-1, 0, 0}, alt{-1, 0, 0};
-    for (const auto &m : candidates(c.k)) {
+    for (const auto &m : candidates(c.k, c.idx.size())) {
       if (make_candidate(bp, c, m.method, m.s, m.variant)) {
         clear_error();
         continue;

@@ -3484,7 +3484,6 @@ static size_t dense_shared_bytes(int NRM, int LT, int NP) {
 // falls on lines just read; 97 with the test for NaN and Inf), 2-norm error at N = 2000 3.2-4.6e-16 ->
 // 1.7-2.8e-16 (the FMM of the same lines 2.3-7.3e-16).
 constexpr int kGemmRT = 32, kGemmLT = 32, kGemmKC = 64, kGemmNT = 256, kGemmKP = kGemmKC + 2;
-constexpr size_t kGemmFewLines = 4096;
 // The work of tile (bx, by) of the tiled dense product (grid (line tiles,
 // row tiles)); k_lines_gemm runs one grid of them, k_lines_gemm_multi the
 // grids of several size classes in one launch.

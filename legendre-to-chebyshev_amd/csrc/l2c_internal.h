@@ -381,6 +381,8 @@ constexpr int kDenseMaxN = 256;
 // direct plans up to this length build the dense parity blocks; batched lines
 // with kDenseMaxN < N <= kGemmMaxN run them as a tiled product
 constexpr int kGemmMaxN = 4096;
+// calls of up to this many lines with N <= kDenseMaxN take the tiled product as well
+constexpr size_t kGemmFewLines = 4096;
 // implemented in l2c_exec.hip
 int run_fmm(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size_t stride,
             hipStream_t st, int band_only);

@@ -117,3 +117,14 @@ def test_tune_cache_round_trip(amd, orc, tmp_path):
         assert relerr(g1[:lengths[0]], o) <= 1e-14 * 13
     finally:
         amd.tune_cache(None)
+
+
+@pytest.mark.parametrize("count", [40, 900])
+def test_tuned_dense_classes_run_together(amd, count):
+    """The tuner leaves the dense classes of a batch on the kernel that runs them all in
+    one launch while none has more lines than that kernel takes by itself."""
+    announce(f"tuned dense classes, {count} lines")
+    lengths = np.random.default_rng(count).integers(33, 257, count)
+    for _ in range(6):
+        for c in amd.BatchPlan(lengths, 18, amd.L2C, tune=True).classes():
+            assert c["method"] != "direct" or c["variant"] == 2, c
