@@ -251,8 +251,8 @@ int l2c_batch_synchronize(l2c_batch_plan *bp);
 /* One size class of a batch plan: its padded length, the number of transforms
  * in it, the method chosen (0 direct, 1 FMM), the FMM leaf size s and depth
  * L, the tuner's time for the class in milliseconds (-1 if untuned), the
- * kernel variant (FMM: 0 fused downward pass, 1 split into band and far
- * field; direct: 0 dense kernel by line count, 1 one tile of all rows, 2 row
+ * kernel variant (FMM: 0 the near field in the upward launch, 1 in a launch of
+ * its own, for M = 18; direct: 0 dense kernel by line count, 1 whole lines, 2 row
  * tiles) and whether the choice came from the tuning cache. */
 typedef struct {
   size_t n_max, count;

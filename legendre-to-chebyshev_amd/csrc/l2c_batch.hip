@@ -141,7 +141,9 @@ static int make_candidate(l2c_batch_plan_s *bp, BatchClass &c, int method, size_
   // (run_packed never takes the dense blocks of an FMM plan)
   c.fp = create_fmm_impl(c.n_max, s, bp->M, bp->direction, 0, 0, 0, false);
   if (!c.fp) return -1;
-  if (c.fp->L < 1 || c.fp->s != s || !c.fp->geo.fast || reserve_lines(c.fp, c.idx.size())) {
+  // (variant 1, the band apart, only where there are band groups)
+  if (c.fp->L < 1 || c.fp->s != s || !c.fp->geo.fast || (variant && !c.fp->geo.far) ||
+      reserve_lines(c.fp, c.idx.size())) {
     destroy_class_plans(c);
     return -1;
   }
@@ -193,8 +195,8 @@ static double time_class(l2c_batch_plan_s *bp, const BatchClass &c, size_t dir) 
 }
 
 // Candidates of a size class k of count lines: the direct sum up to 2^13, the FMM with
-// s = 16, 32, 64 where the depth L = k - log2(s) - 2 is at least 1, each with
-// the fused and the split downward pass.  Classes of 32 < 2^k <= 256 have two dense
+// s = 16, 32, 64 where the depth L = k - log2(s) - 2 is at least 1, at the rank that
+// has band groups (18) with the band in the k_up launch and apart.  Classes of 32 < 2^k <= 256 have two dense
 // kernels.  The tiled one runs in one launch with the batch's other dense classes, the
 // whole-line one in a launch of its own, so it is a candidate only past the lines that
 // the tiled one takes by itself (dense_tiled); below, the two come out even alone and a
@@ -206,7 +208,7 @@ struct Cand {
   size_t s;
   int variant;
 };
-static std::vector<Cand> candidates(int k, size_t count) {
+static std::vector<Cand> candidates(int k, size_t count, size_t M) {
   std::vector<Cand> v;
   if (k <= 13) {
     if (k > 5 && k <= 8) {
@@ -219,7 +221,7 @@ static std::vector<Cand> candidates(int k, size_t count) {
   for (int ls = 4; ls <= 6; ls++)
     if (k - ls - 2 >= 1) {
       v.push_back({1, (size_t)1 << ls, 0});
-      v.push_back({1, (size_t)1 << ls, 1});
+      if (M == 18) v.push_back({1, (size_t)1 << ls, 1});
     }
   return v;
 }
@@ -481,7 +483,7 @@ static l2c_batch_plan_s *create_batch_impl(const size_t *n, size_t count, size_t
     }
     double best = -1, second = -1;
     Cand pick{-1, 0, 0}, alt{-1, 0, 0};
-    for (const auto &m : candidates(c.k, c.idx.size())) {
+    for (const auto &m : candidates(c.k, c.idx.size(), bp->M)) {
       if (make_candidate(bp, c, m.method, m.s, m.variant)) {
         clear_error();
         continue;

@@ -128,3 +128,19 @@ def test_tuned_dense_classes_run_together(amd, count):
     for _ in range(6):
         for c in amd.BatchPlan(lengths, 18, amd.L2C, tune=True).classes():
             assert c["method"] != "direct" or c["variant"] == 2, c
+
+
+@pytest.mark.parametrize("M", [12, 18, 24])
+def test_tuned_variants_by_rank(amd, orc, M):
+    """The near field in a launch of its own is a choice at rank 18 alone: other ranks
+    have one downward path, which the tuner times once."""
+    announce(f"tuned variants M={M}")
+    lengths = [9000, 12000, 16000] * 3
+    for _ in range(8):
+        bp = amd.BatchPlan(lengths, M, amd.L2C, tune=True)
+        for c in bp.classes():
+            assert c["method"] == "fmm" and c["variant"] in ((0, 1) if M == 18 else (0,)), c
+    u = amd.packed_coefficients(bp.lengths, seed=M)
+    g = bp.execute(u, 0)
+    if M >= 18:
+        check(amd, orc, bp, u, g, 0, which=[0, 5, 8])
