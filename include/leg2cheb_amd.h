@@ -263,7 +263,8 @@ typedef struct {
   int cached;
 } l2c_batch_class;
 /* Tuning cache for l2c_create_batch(..., tune = 1): a text file holding the
- * tuner's choice per (device, size class, population, direction, M); classes
+ * tuner's choice per (device, size class, population, direction, M, version of
+ * the kernels); classes
  * found there skip the timing, new choices are appended.  path = NULL turns
  * it off.  The environment variable L2C_TUNE_CACHE gives the default path.
  * No counterpart in the reference (its CLI keeps FFTW wisdom, src/bin/l2c.c:

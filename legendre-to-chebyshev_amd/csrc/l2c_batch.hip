@@ -296,7 +296,11 @@ static int refine_close_calls(l2c_batch_plan_s *bp, size_t dir) {
 // direction, rank), kept in a text file (l2c_tune_cache or L2C_TUNE_CACHE),
 // one "key method s variant ms" line per choice, so that later batch plans
 // of the same shapes skip the timing (the reference keeps FFTW wisdom for the
-// same purpose, src/bin/l2c.c:417-454).
+// same purpose, src/bin/l2c.c:417-454).  The key ends in kTuneKernels: raise it
+// whenever the candidates change or what a variant runs, so that choices and times of
+// other kernels are not taken (lines of other versions stay in the file, unused; the
+// first files had none).
+constexpr int kTuneKernels = 2;
 static std::mutex g_tc_mu;
 static std::string g_tc_path;
 static bool g_tc_path_set = false, g_tc_loaded = false;
@@ -327,7 +331,7 @@ static std::string tune_key(const l2c_batch_plan_s *bp, const BatchClass &c, siz
   size_t pop = 1;
   while (pop < c.idx.size()) pop <<= 1;
   return dev + "/n" + std::to_string(c.n_max) + "/count" + std::to_string(pop) + "/dir" +
-         std::to_string(dir) + "/M" + std::to_string(bp->M);
+         std::to_string(dir) + "/M" + std::to_string(bp->M) + "/k" + std::to_string(kTuneKernels);
 }
 
 static void tune_cache_load() {  // under g_tc_mu

@@ -144,3 +144,27 @@ def test_tuned_variants_by_rank(amd, orc, M):
     g = bp.execute(u, 0)
     if M >= 18:
         check(amd, orc, bp, u, g, 0, which=[0, 5, 8])
+
+
+def test_tune_cache_of_other_kernels(amd, tmp_path):
+    """Lines of a cache file whose key names another version of the kernels, or none
+    (as the first files had it), are not taken: the classes are timed again and their
+    choices appended under this version's key."""
+    announce("tune cache of other kernels")
+    lengths = [100, 500, 3000] * 5
+    try:
+        amd.tune_cache(tmp_path / "now.txt")
+        amd.BatchPlan(lengths, 18, amd.L2C, tune=True)
+        lines = (tmp_path / "now.txt").read_text().splitlines()
+        assert len(lines) == 3
+        for other in ("", "/k1"):
+            path = tmp_path / "other.txt"
+            old = [l.replace(l.split()[0], l.split()[0].rsplit("/k", 1)[0] + other) for l in lines]
+            assert not set(old) & set(lines)
+            path.write_text("\n".join(old) + "\n")
+            amd.tune_cache(path)
+            assert not any(c["cached"] for c in amd.BatchPlan(lengths, 18, amd.L2C, tune=True).classes())
+            assert len(path.read_text().splitlines()) == 6
+            assert all(c["cached"] for c in amd.BatchPlan(lengths, 18, amd.L2C, tune=True).classes())
+    finally:
+        amd.tune_cache(None)
