@@ -238,9 +238,11 @@ void l2c_free_batch(l2c_batch_plan *bp);
  * packed arrays (overwrite semantics).  Runs on the batch's own streams and
  * returns without synchronising the host; a later call on `stream` (a
  * hipStream_t, NULL = the batch's main stream) or l2c_batch_synchronize()
- * sees the result.  With l2c_batch_graph(bp, 1) the launch sequence is
- * captured into a HIP graph on the first call for a given (d_in, d_out,
- * direction) and replayed by later calls.  Returns 0 or -1. */
+ * sees the result.  With l2c_batch_graph(bp, 1) the second call in a row with
+ * the same (d_in, d_out, direction) captures the launch sequence into a HIP
+ * graph, which later calls with them replay; calls with others run launch by
+ * launch.  A plan captures once and keeps the graph until it is freed
+ * (l2c_batch_graph(bp, 0) sets it aside).  Returns 0 or -1. */
 int l2c_execute_batch_device(l2c_batch_plan *bp, const double *d_in, double *d_out,
                              size_t direction, void *stream);
 /* Same with host arrays (staged through pinned buffers; synchronous). */

@@ -70,6 +70,7 @@ struct l2c_batch_plan_s {
   hipEvent_t fork = nullptr, join[l2c::kBatchStreams] = {};
   bool graph_on = false;
   hipGraphExec_t exec = nullptr;
+  // arrays and direction of the graph, or of the last call while there is none
   const double *g_in = nullptr;
   double *g_out = nullptr;
   size_t g_dir = 99;
@@ -226,8 +227,9 @@ static std::vector<Cand> candidates(int k, size_t count, size_t M) {
   return v;
 }
 
+struct ForkJoin;
 static int launch_batch(l2c_batch_plan_s *bp, const double *d_in, double *d_out, size_t dir,
-                        hipStream_t origin);
+                        hipStream_t origin, const ForkJoin *ev = nullptr);
 
 // The whole batch, eager, on the staging buffers (min of 3 after one warm-up),
 // milliseconds; < 0 on failure.
@@ -559,14 +561,22 @@ static l2c_batch_plan_s *create_batch_impl(const size_t *n, size_t count, size_t
   return bp;
 }
 
-// Fork from `origin`, run every class on its stream, join back to `origin`.
+// Events of a fork from and a join to a stream.
+struct ForkJoin {
+  hipEvent_t fork = nullptr, join[kBatchStreams] = {};
+};
+
+// Fork from `origin`, run every class on its stream, join back to `origin`,
+// with the plan's events or those given.
 // The classes that take the tiled dense product run as one launch (on the
 // stream of the first of them) when fuse_dense is set.
 static int launch_batch(l2c_batch_plan_s *bp, const double *d_in, double *d_out, size_t dir,
-                        hipStream_t origin) {
-  L2C_HIP(hipEventRecord(bp->fork, origin), -1);
+                        hipStream_t origin, const ForkJoin *ev) {
+  const hipEvent_t fork = ev ? ev->fork : bp->fork;
+  const hipEvent_t *join = ev ? ev->join : bp->join;
+  L2C_HIP(hipEventRecord(fork, origin), -1);
   for (int i = 0; i < kBatchStreams; i++)
-    if (bp->st[i] != origin) L2C_HIP(hipStreamWaitEvent(bp->st[i], bp->fork, 0), -1);
+    if (bp->st[i] != origin) L2C_HIP(hipStreamWaitEvent(bp->st[i], fork, 0), -1);
   std::vector<DenseItem> fused;
   int fused_stream = -1;
   for (const auto &c : bp->cls) {
@@ -582,12 +592,47 @@ static int launch_batch(l2c_batch_plan_s *bp, const double *d_in, double *d_out,
     return -1;
   for (int i = 0; i < kBatchStreams; i++) {
     if (bp->st[i] == origin) continue;
-    L2C_HIP(hipEventRecord(bp->join[i], bp->st[i]), -1);
-    L2C_HIP(hipStreamWaitEvent(origin, bp->join[i], 0), -1);
+    L2C_HIP(hipEventRecord(join[i], bp->st[i]), -1);
+    L2C_HIP(hipStreamWaitEvent(origin, join[i], 0), -1);
   }
   return 0;
 }
 
+// The plan's graph for these arguments, recorded on a stream of its own with events that
+// nothing else uses.
+static int record_graph(l2c_batch_plan_s *bp, const double *d_in, double *d_out, size_t dir) {
+  ForkJoin ev;
+  bool ok = hipEventCreateWithFlags(&ev.fork, hipEventDisableTiming) == hipSuccess;
+  for (auto &e : ev.join) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  hipStream_t cap = bp->st[0];
+  hipError_t e = ok ? hipStreamSynchronize(cap) : hipErrorOutOfMemory;
+  hipGraph_t g = nullptr;
+  int rc = 0;
+  if (e == hipSuccess) e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+  if (e == hipSuccess) {
+    rc = launch_batch(bp, d_in, d_out, dir, cap, &ev);
+    e = hipStreamEndCapture(cap, &g);
+  }
+  if (!rc && e == hipSuccess && g) e = hipGraphInstantiate(&bp->exec, g, nullptr, nullptr, 0);
+  if (!rc && (e != hipSuccess || !g))
+    set_error(std::string("l2c_execute_batch_device: recording the graph: ") + hipGetErrorString(e));
+  if (rc || e != hipSuccess || !g) {
+    bp->exec = nullptr;
+    rc = -1;
+  }
+  if (g) (void)hipGraphDestroy(g);
+  if (ev.fork) (void)hipEventDestroy(ev.fork);
+  for (auto &j : ev.join)
+    if (j) (void)hipEventDestroy(j);
+  return rc;
+}
+
+// With the graph on, the second call in a row with the same arrays and direction
+// records it; calls with others run launch by launch.  A plan records once and keeps the
+// graph until it is freed: a process that released it and recorded again for each of two
+// pairs of arrays in turn ended in a segmentation fault whose cause is not known, and it
+// cost 700 us and more per call, where launch by launch takes 250 (4096 lengths up to
+// 8192; a replay 215).
 static int execute_batch_impl(l2c_batch_plan_s *bp, const double *d_in, double *d_out,
                               size_t dir, hipStream_t user) {
   if (!bp || !d_in || !d_out) {
@@ -599,37 +644,22 @@ static int execute_batch_impl(l2c_batch_plan_s *bp, const double *d_in, double *
     return -1;
   }
   const hipStream_t origin = user ? user : bp->st[0];
-  if (!bp->graph_on) return launch_batch(bp, d_in, d_out, dir, origin);
-  if (!bp->exec || bp->g_in != d_in || bp->g_out != d_out || bp->g_dir != dir) {
-    if (bp->exec) {
-      L2C_HIP(hipStreamSynchronize(origin), -1);
-      (void)hipGraphExecDestroy(bp->exec);
-      bp->exec = nullptr;
+  if (bp->graph_on) {
+    const bool same = bp->g_in == d_in && bp->g_out == d_out && bp->g_dir == dir;
+    if (!bp->exec) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (same) L2C_HIP(hipStreamIsCapturing(origin, &cs), -1);  // the caller's own graph
+      if (same && cs == hipStreamCaptureStatusNone && record_graph(bp, d_in, d_out, dir)) return -1;
+      bp->g_in = d_in;
+      bp->g_out = d_out;
+      bp->g_dir = dir;
     }
-    hipStream_t cap = bp->st[0];
-    L2C_HIP(hipStreamSynchronize(cap), -1);
-    L2C_HIP(hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal), -1);
-    const int rc = launch_batch(bp, d_in, d_out, dir, cap);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(cap, &g);
-    if (rc || e != hipSuccess || !g) {
-      if (g) (void)hipGraphDestroy(g);
-      if (!rc) set_error(std::string("graph capture failed: ") + hipGetErrorString(e));
-      return -1;
+    if (bp->exec && same) {
+      L2C_HIP(hipGraphLaunch(bp->exec, origin), -1);
+      return 0;
     }
-    const hipError_t ei = hipGraphInstantiate(&bp->exec, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (ei != hipSuccess) {
-      bp->exec = nullptr;
-      set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
-      return -1;
-    }
-    bp->g_in = d_in;
-    bp->g_out = d_out;
-    bp->g_dir = dir;
   }
-  L2C_HIP(hipGraphLaunch(bp->exec, origin), -1);
-  return 0;
+  return launch_batch(bp, d_in, d_out, dir, origin);
 }
 
 }  // namespace l2c
@@ -702,11 +732,6 @@ int l2c_batch_graph(l2c_batch_plan *bp, int enable) {
     return -1;
   }
   bp->graph_on = enable != 0;
-  if (!bp->graph_on && bp->exec) {
-    (void)hipStreamSynchronize(bp->st[0]);
-    (void)hipGraphExecDestroy(bp->exec);
-    bp->exec = nullptr;
-  }
   return 0;
 }
 
