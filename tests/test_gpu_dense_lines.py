@@ -133,3 +133,27 @@ def test_blocks_of_planned_directions(amd, monkeypatch, N, maxs):
         assert np.array_equal(run_lines(amd, one, x, d, False), run_lines(amd, both, x, d, False))
         with pytest.raises(amd.L2CError):
             run_lines(amd, one, x, 1 - d, False)
+
+
+@pytest.mark.parametrize("N,B", [(40, 9), (200, 50), (256, 70), (300, 40), (1000, 70), (1536, 33),
+                                 (2048, 130)])
+@pytest.mark.parametrize("direction", [0, 1])
+def test_tiled_product_not_finite(amd, monkeypatch, N, B, direction):
+    """A NaN or Inf in a line that runs on the tiled dense product (direct plans and the
+    FMM plans' dense route, the small-N routes on) reaches the rows of its line and
+    parity at or before its place, all of them, and no other."""
+    announce(f"tiled product, not finite N={N} B={B} dir={direction}")
+    monkeypatch.delenv("L2C_DIRECT_MAXN", raising=False)
+    monkeypatch.setenv("L2C_DIRECT_LINES", "0")
+    plan = amd.FMMPlan(N, 64, 18, direction)
+    plan.profile(True)
+    for strided in (False, True):
+        for pos in (0, 1, 15, 16, 30, 31, 32, 33, N // 2, N // 2 + 17, N - 2, N - 1):
+            for val in (np.inf, -np.inf, np.nan):
+                x = np.random.default_rng(N).uniform(0.5, 1, (B, N))
+                x[B // 2, pos] = val
+                y = run_lines(amd, plan, x, direction, strided)
+                want = np.zeros((B, N), bool)
+                want[B // 2, pos % 2:pos + 1:2] = True
+                assert np.array_equal(~np.isfinite(y), want), (strided, pos, val)
+    assert set(plan.profile_read()) == {"k_direct"}

@@ -77,3 +77,26 @@ def test_noalloc_refuses_oversized_line(amd):
     buf = amd.DeviceBuffer(8)
     rc = L.l2c_execute_lines_device_noalloc(plan.plan, buf.ptr, buf.ptr, 0, 1, 1, N, 0, 1, None)
     assert rc == -1 and "scratch" in amd.last_error()
+
+
+@pytest.mark.parametrize("N,nl", [(300, 60), (1536, 11), (1537, 130), (2048, 128)])
+def test_noalloc_dense_route(amd, orc, monkeypatch, N, nl):
+    """Line calls of FMM plans that run as the dense product (past 16,384 elements)
+    take it in both entry points: only the dense kernel runs, identical outputs."""
+    monkeypatch.delenv("L2C_DIRECT_MAXN", raising=False)
+    assert N * nl > 16384
+    L = amd.lib()
+    plan = amd.FMMPlan(N, 64, 18, amd.BOTH)
+    op = orc.FMMPlan(N, 64, 18, orc.BOTH)
+    for d in (0, 1):
+        announce(f"noalloc dense route N={N} lines={nl} dir={d}")
+        x = np.random.default_rng(N + nl + d).uniform(-1, 1, nl * N)
+        a = _lines(amd, L.l2c_execute_lines_device_noalloc, plan, x, d, nl, N)
+        plan.profile(True)
+        b = _lines(amd, L.l2c_execute_lines_device, plan, x, d, nl, N)
+        assert set(plan.profile_read()) == {"k_direct"}
+        plan.profile(False)
+        assert np.array_equal(a, b)
+        for line in (0, nl - 1):
+            ref = op.execute(np.ascontiguousarray(x[line * N:(line + 1) * N]), d)
+            assert relerr(a[line * N:(line + 1) * N], ref) <= tol(N)
