@@ -410,7 +410,8 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
 }
 
 // ---------------------------------------------------------------------------
-// k_up: grid (2^(lu+2), lines), 256 threads.  G = 2^gu <= 16 leaf chunks.
+// k_up_any: the upward pass for ranks other than 18 and leaf sizes above 64.  Grid
+// (2^(lu+2), lines), 256 threads.  G = 2^gu <= 16 leaf chunks.
 //
 // Leaf moments W_par (G x M) = X_par (G x s) T_par (s x M) run on
 // v_mfma_f64_16x16x4f64 (A operand: lane l holds A[l%16][l/16]; B: lane l
@@ -428,17 +429,20 @@ size_t up_shared_bytes(const Geo &g) {
 }
 
 // LM: the subtree levels on MFMA (MT > 0; chosen for subtrees of 2^3 and
-// 2^4 leaf chunks in calls of up to 8 lines) or on VALU.
+// 2^4 leaf chunks in calls of up to 8 lines) or on VALU: 2 lines of 70,000 (s = 137)
+// 71.3 us against 72.5, 4 of 2^20 (s = 128) 288 against 291, single ones even.  (Its body
+// in a function of its own that the kernel calls: four registers spilled to a scratch
+// frame, 700,000 (s = 86) 69.2 us against 68.2.)
 template <int MT, bool LM>
-__device__ __forceinline__ void up_group(const double *__restrict__ in, const LineMap &lm,
-                                         const Geo &g, int dir, const double *__restrict__ T,
-                                         const double *__restrict__ U,
-                                         const double *__restrict__ P,
-                                         double *__restrict__ wsall, size_t wsstride, int j,
-                                         double *sm) {
+__global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up_any(
+    const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
+    const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
+    size_t wsstride) {
+  extern __shared__ double sm[];
   const int M = MT > 0 ? MT : g.M;
   const int s = g.s, L = g.L, M2 = 2 * M, MM = M * M;
   const int G = 1 << g.gu;
+  const int j = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const double *src = in + line_off(lm, blockIdx.y);
   const size_t Nl = (size_t)line_len(lm, blockIdx.y, g.N);  // zeros past the line's end
@@ -905,16 +909,6 @@ __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4)))
     band_group<S16, G>(in + off, ba.out + off, lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, 0,
                        ba.tab, ba.head, sm);
   }
-}
-
-// The upward pass for other ranks and leaf sizes.
-template <int MT, bool LM>
-__global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4))) k_up_any(
-    const double *__restrict__ in, LineMap lm, Geo g, int dir, const double *__restrict__ T,
-    const double *__restrict__ U, const double *__restrict__ P, double *__restrict__ wsall,
-    size_t wsstride) {
-  extern __shared__ double sm[];
-  up_group<MT, LM>(in, lm, g, dir, T, U, P, wsall, wsstride, blockIdx.x, sm);
 }
 
 // ---------------------------------------------------------------------------
