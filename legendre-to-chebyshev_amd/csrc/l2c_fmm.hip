@@ -3374,6 +3374,10 @@ __global__ void __launch_bounds__(32 * NRM * NP)
     if (more) fetch(nslot);
     offsets(item + 2 * gridDim.x, nslot == 2 ? 0 : nslot + 1);
     d4 D[2][NH];  // [row tile][16-line half]
+    // (the empty asm keeps the compiler from holding the tests of all four row tile
+    // pairs through the item loop: 22 scalars and two vector registers spilled)
+    int nr = NR;
+    asm volatile("" : "+s"(nr));
     auto products = [&](auto r0) {
       constexpr int r = decltype(r0)::value;
 #pragma unroll
@@ -3382,7 +3386,7 @@ __global__ void __launch_bounds__(32 * NRM * NP)
       for (int g = 0; g < NG; g++) {
         constexpr int n0 = NRM - r;
         const int col = g < n0 ? r + g : NRM - 1 - r + g - n0;
-        if (col >= NR) continue;
+        if (col >= nr) continue;
         const double *b = mine + 16 * col;
 #pragma unroll
         for (int kk = 0; kk < 4; kk++)
