@@ -2966,10 +2966,10 @@ __global__ void __launch_bounds__(256) k_direct(const double *__restrict__ in,
 // term order per lane, and add their partial sums across the wave.  Grid
 // ((N + 3) / 4, lines): four rows per work-group, line blockIdx.y of lm
 // (unpacked maps).
-template <int QR>
+template <int dir, int QR>
 __global__ void __launch_bounds__(256) k_direct_rows(const double *__restrict__ in,
                                                      double *__restrict__ out, LineMap lm, int N,
-                                                     int dir, const double *__restrict__ a,
+                                                     const double *__restrict__ a,
                                                      const double *__restrict__ an,
                                                      const double *__restrict__ dn) {
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -3735,9 +3735,10 @@ static void launch_direct_one(Prof *prof, int N, size_t dir, const double *a, co
     launch_k(prof, kernel, grid, 256, shm, st, d_in, d_out, lm, N, a, an, dn);
     return;
   }
-  launch_k(prof, nlines > 1 ? k_direct_rows<1> : k_direct_rows<3>,
-           dim3((unsigned)((N + 3) / 4), nlines), 256, 0, st, d_in, d_out, lm, N, (int)dir, a, an,
-           dn);
+  auto kernel = nlines > 1 ? (dir == L2C ? k_direct_rows<L2C, 1> : k_direct_rows<C2L, 1>)
+                           : (dir == L2C ? k_direct_rows<L2C, 3> : k_direct_rows<C2L, 3>);
+  launch_k(prof, kernel, dim3((unsigned)((N + 3) / 4), nlines), 256, 0, st, d_in, d_out, lm, N, a,
+           an, dn);
 }
 
 // k_direct over nlines lines of map lm (one launch for any number of lines);
