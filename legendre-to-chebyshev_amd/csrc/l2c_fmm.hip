@@ -60,6 +60,12 @@ __device__ __forceinline__ void store_pair(d2 v, __amdgpu_buffer_rsrc_t r, int v
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, 0, 0);
 }
 
+// How a call's work-groups take its lines, and where the band sums wait for the far
+// field: LINES_PLAIN line by line, over the output; LINES_FLAT the same without empty
+// groups (k_up); LINES_ACROSS group by group over lines that lie side by side (place);
+// LINES_RAW line by line, back to back in the workspace (raw_sums).
+enum { LINES_PLAIN = 0, LINES_FLAT = 1, LINES_ACROSS = 2, LINES_RAW = 3 };
+
 // The (group, line) of work-group id of n groups of each of nl lines.  In general
 // the groups of a line follow each other.  ACROSS, lines that lie side by side: an HBM
 // or L2 line holds one element of each of 8 or 16 of them, so the work-groups of one
@@ -239,12 +245,12 @@ __device__ __forceinline__ void band_trip(BandPtr &b, int s1, int s2, kdouble hp
 #undef QUAD_FETCH
 }
 
-// Band group grp of the line at src / dst (element stride es, length Nl): the
-// sums are stored over the output, raw (the C2L diagonal included), or with
+// Band group grp of the line at src (element stride es, length Nl): the sums
+// go to dst (element stride ds), raw (the C2L diagonal included), or with
 // the final scaling when scale != 0.
 template <bool S16, int G>
-__device__ __forceinline__ void band_group(const double *__restrict__ src,
-                                           double *__restrict__ dst, size_t es, int Nl,
+__device__ __forceinline__ void band_group(const double *__restrict__ src, size_t es,
+                                           double *__restrict__ dst, size_t ds, int Nl,
                                            const Geo &g, int dir, int grp, int scale,
                                            const double *__restrict__ tab,
                                            const double *__restrict__ head, double *sm) {
@@ -398,14 +404,14 @@ __device__ __forceinline__ void band_group(const double *__restrict__ src,
     }
     return v;
   };
-  if (es == 1) {
+  if (ds == 1) {
     const __amdgpu_buffer_rsrc_t r = line_rsrc(dst + row0, nr);
     for (int e = 2 * tid; e < nr; e += 2 * kBandNT) {
       const d2 v = {value(e), e + 1 < nr ? value(e + 1) : 0.0};
       store_pair(v, r, 8 * e);
     }
   } else {
-    for (int e = tid; e < nr; e += kBandNT) dst[(row0 + e) * es] = value(e);
+    for (int e = tid; e < nr; e += kBandNT) dst[(row0 + e) * ds] = value(e);
   }
 }
 
@@ -876,15 +882,20 @@ __device__ __forceinline__ void up18_group(const double *__restrict__ in, const 
 //
 // Shallow trees (L <= 4) have fewer band groups (nb) than upward ones, and work-groups
 // go to the eight XCDs in turn: padded to the upward groups' number, two of four on
-// a line of 3300, all of the band would fall to four XCDs.  Their line calls (UP_FLAT)
+// a line of 3300, all of the band would fall to four XCDs.  Their line calls (LINES_FLAT)
 // take a grid (nb + upward groups, lines) with the nb groups of every line first and
 // none empty: 3000 lines of 3300 (s = 52) 310 -> 211 us (of it 128 the band's and 92 the
 // upward groups' in launches of their own), the call 407 -> 301.  So do calls whose
-// lines lie side by side (UP_ACROSS).  UP_FLAT for all of them costs 0.3 % (the
+// lines lie side by side (LINES_ACROSS).  LINES_FLAT for all of them costs 0.3 % (the
 // division by the group count).
-enum { UP_PLAIN = 0, UP_FLAT = 1, UP_ACROSS = 2 };
+//
+// LINES_RAW calls read the strided input twice, for the band and for the moments.  From a
+// stride of 8 on (a cache line per element or two) the grid is (.., lines): eight band
+// groups, then the upward groups of the same leaf chunks, on the same XCDs, which find
+// most of it in their L2.  2^20 at stride 16 k_up 50.8 -> 40.8 us, the call 94 -> 78; at
+// stride 2 one after the other is as fast or faster (64 lines of 2^16 113 / 125).
 struct BandArgs {
-  double *out;
+  double *out;  // LINES_RAW: N sums a line
   const double *tab, *head;
   int nb;  // band groups of a line (0: the upward pass alone)
 };
@@ -896,18 +907,27 @@ __global__ void __launch_bounds__(kUpNT) __attribute__((amdgpu_waves_per_eu(4)))
   extern __shared__ double sm[];
   Place w{blockIdx.x, blockIdx.y};
   bool band = blockIdx.z + 1 != gridDim.z;
-  if (ORDER != UP_PLAIN) {
+  if (ORDER == LINES_RAW && ba.nb && gridDim.z == 1) {  // (LINES_RAW, in turn)
+    const unsigned r = (4u << g.lu) / ba.nb, per = 8 + 8 * r;
+    const unsigned j = blockIdx.x % per, i = blockIdx.x / per * 8 + (j & 7);
+    if (i >= (unsigned)ba.nb) return;
+    band = j < 8;
+    w.grp = band ? i : i * r + (j >> 3) - 1;
+  }
+  if (ORDER == LINES_FLAT || ORDER == LINES_ACROSS) {
     const unsigned nl = gridDim.y, bands = ba.nb * nl, id = blockIdx.x + gridDim.x * blockIdx.y;
     band = id < bands;
-    w = place_of<ORDER == UP_ACROSS>(band ? id : id - bands, band ? ba.nb : 4u << g.lu, nl);
+    w = place_of<ORDER == LINES_ACROSS>(band ? id : id - bands, band ? ba.nb : 4u << g.lu, nl);
   }
   if (!band) {
     if ((int)w.grp < 4 << g.lu)
       up18_group(in, lm, g, dir, T, U, P, wsall, wsstride, w.grp, w.line, sm);
   } else {
     const size_t off = line_off(lm, w.line);
-    band_group<S16, G>(in + off, ba.out + off, lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, 0,
-                       ba.tab, ba.head, sm);
+    constexpr bool raw = ORDER == LINES_RAW;
+    band_group<S16, G>(in + off, lm.es, ba.out + (raw ? (size_t)w.line * g.N : off),
+                       raw ? 1 : lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, 0, ba.tab,
+                       ba.head, sm);
   }
 }
 
@@ -2682,15 +2702,16 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
 // downward pass (down_split; raw sums, the C2L diagonal included, over the
 // output; k_far adds the far field and scales, src/C/leg2cheb.c:1467-1483 and
 // the band scaling of :236-535).  Grid (band groups, lines), 256 threads.
-template <bool S16, bool ACROSS>
+template <bool S16, int ORDER>
 __global__ void __launch_bounds__(kBandNT) __attribute__((amdgpu_waves_per_eu(4))) k_band(
     const double *__restrict__ in, double *__restrict__ out, LineMap lm, Geo g, int dir, int scale,
     const double *__restrict__ tab, const double *__restrict__ head) {
   extern __shared__ double sm[];
-  const Place w = place<ACROSS>();
+  const Place w = place<ORDER == LINES_ACROSS>();
+  constexpr bool raw = ORDER == LINES_RAW;
   const size_t off = line_off(lm, w.line);
-  band_group<S16, 16>(in + off, out + off, lm.es, line_len(lm, w.line, g.N), g, dir, w.grp, scale,
-                      tab, head, sm);
+  band_group<S16, 16>(in + off, lm.es, out + (raw ? (size_t)w.line * g.N : off), raw ? 1 : lm.es,
+                      line_len(lm, w.line, g.N), g, dir, w.grp, scale, tab, head, sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -2719,15 +2740,15 @@ __host__ __device__ inline FarLds far_lds(const Geo &g) {
 size_t far_shared_bytes(const Geo &g) { return 8 * (size_t)far_lds(g).total; }
 bool far_eligible(const Geo &g) { return g.M == 18 && g.s <= kBandMaxS; }
 
-template <bool ACROSS>
+template <int ORDER>
 __global__ void __launch_bounds__(kFarNT) __attribute__((amdgpu_waves_per_eu(4))) k_far(
-    double *__restrict__ out, LineMap lm, Geo g, int dir, const double *__restrict__ wsall,
-    size_t wsstride, const double *__restrict__ Dg, const double *__restrict__ Qg,
+    double *__restrict__ out, const double *__restrict__ raw, LineMap lm, Geo g,
+    int dir, const double *__restrict__ wsall, size_t wsstride, const double *__restrict__ Dg, const double *__restrict__ Qg,
     const double *__restrict__ Tg) {
   extern __shared__ double sm[];
   constexpr int M = 18, M2 = 36, MM = M * M;
   const int s = g.s, N = g.N;
-  const Place w = place<ACROSS>();
+  const Place w = place<ORDER == LINES_ACROSS>();
   const int Nl = line_len(lm, w.line, N);
   const int G = 1 << g.gd, Rr = w.grp;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -2798,8 +2819,9 @@ __global__ void __launch_bounds__(kFarNT) __attribute__((amdgpu_waves_per_eu(4))
   }
   // the band sums this work-group adds to (nr <= 2 G s <= 8 NT)
   d2 vb[4];
-  if (es == 1) {
-    const __amdgpu_buffer_rsrc_t r = line_rsrc(dst, nr);
+  if (ORDER == LINES_RAW || es == 1) {
+    const __amdgpu_buffer_rsrc_t r =
+        line_rsrc(ORDER == LINES_RAW ? raw + (size_t)w.line * N + row0 : dst, nr);
 #pragma unroll
     for (int q = 0; q < 4; q++) vb[q] = load_pair(r, 16 * tid + 4096 * q, 0);
   } else {
@@ -3868,12 +3890,27 @@ static const Geo &call_geo(const fmm_plan_s *p, size_t nlines) {
   return nlines == 1 && !m2l_on_mfma(p, nlines) ? p->geo1 : p->geo;
 }
 
+// Whether a call's band sums wait for the far field in the workspace, back to back,
+// and not in the output (LINES_RAW): where the output's elements lie apart with nothing
+// of the call between them (single strided transforms, lines far apart), so that every
+// touch of one fetches or writes a cache line.  One transform, s = 64, workspace / output
+// (us): 2^20 at stride 16 78 / 123, at 8 62 / 77, at 2 49.5 / 51, 2^18 at 16 33 / 39,
+// 2^16 at 16 19 / 22, 20,000 at 8 17.3 / 17.9; 4 lines of 2^20 at 8 245 / 372, 64 of 2^16 at
+// 2 113 / 118.  (With the band inside the downward kernel, whose passes over the array are
+// two fewer, 2^20 at 16 87, at 8 68, 4 lines at 8 267.)  Lines that lie side by side share
+// their cache lines instead (place).
+static bool raw_sums(const Geo &g, const LineMap &lm, size_t nlines) {
+  return g.far && lm.es > 1 && !lm.across &&
+         (nlines == 1 || band_groups(g, 16) >= 4u << g.lu);  // (else LINES_FLAT)
+}
+
 // Workspace for a batch of lines: grown on demand (at least doubling), owned
 // by the plan.  Earlier calls may still be running on a caller's stream, so
 // the store being replaced is retired, not freed: the plan releases it when
 // it is itself freed, and nothing waits here on work of other streams.
-static int ensure_ws(fmm_plan_s *p, size_t nlines, const Geo &g, double **w) {
-  const size_t need = std::max<size_t>(nlines, 1) * ws_doubles(g);
+// raw: with room for the band sums of every line behind it.
+static int ensure_ws(fmm_plan_s *p, size_t nlines, const Geo &g, double **w, bool raw = false) {
+  const size_t need = std::max<size_t>(nlines, 1) * (ws_doubles(g) + (raw ? p->N : 0));
   if (p->wl_cap < need) {
     const size_t cap = std::max(need, 2 * p->wl_cap);
     double *nw = nullptr;
@@ -3923,22 +3960,30 @@ static void launch_down8(fmm_plan_s *p, const Geo &g, const double *d_in, double
 // The split downward pass on st: k_band (before the tree kernels, which it
 // does not need), then k_up and k_m2l, then k_far.
 static void launch_band(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out, size_t dir,
-                        const LineMap &lm, size_t nlines, hipStream_t st, int scale, int slot) {
+                        const LineMap &lm, size_t nlines, hipStream_t st, int order, int scale,
+                        int slot) {
   prof_begin(p->prof, slot, st);
   const bool s16 = (g.s & 15) == 0;
-  launch_k(p->prof, lm.across ? (s16 ? k_band<true, true> : k_band<false, true>)
-                              : (s16 ? k_band<true, false> : k_band<false, false>),
-           dim3(band_groups(g, 16), (unsigned)nlines), kBandNT, band_shared_bytes(g, 16), st, d_in,
-           d_out, lm, g, (int)dir, scale, dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
+  auto kernel =
+      order == LINES_ACROSS ? (s16 ? k_band<true, LINES_ACROSS> : k_band<false, LINES_ACROSS>)
+      : order == LINES_RAW  ? (s16 ? k_band<true, LINES_RAW> : k_band<false, LINES_RAW>)
+                            : (s16 ? k_band<true, LINES_PLAIN> : k_band<false, LINES_PLAIN>);
+  launch_k(p->prof, kernel, dim3(band_groups(g, 16), (unsigned)nlines), kBandNT,
+           band_shared_bytes(g, 16), st, d_in, d_out, lm, g, (int)dir, scale,
+           dir == L2C ? p->t.a : p->t.an, p->t.head[dir]);
   prof_end(p->prof, st);
 }
 
-static void launch_far(fmm_plan_s *p, const Geo &g, double *d_out, size_t dir, const LineMap &lm,
-                       size_t nlines, hipStream_t st, double *ws, int slot) {
+static void launch_far(fmm_plan_s *p, const Geo &g, double *d_out, const double *raw, size_t dir,
+                       const LineMap &lm, size_t nlines, hipStream_t st, int order, double *ws,
+                       int slot) {
   prof_begin(p->prof, slot, st);
-  launch_k(p->prof, lm.across ? k_far<true> : k_far<false>, dim3((unsigned)((size_t)4 << g.ld), (unsigned)nlines), kFarNT,
-           far_shared_bytes(g), st, d_out, lm, g, (int)dir, ws, ws_doubles(g), p->t.D, p->t.Q,
-           p->t.T);
+  launch_k(p->prof,
+           order == LINES_ACROSS ? k_far<LINES_ACROSS>
+           : order == LINES_RAW  ? k_far<LINES_RAW>
+                                 : k_far<LINES_PLAIN>,
+           dim3((unsigned)((size_t)4 << g.ld), (unsigned)nlines), kFarNT, far_shared_bytes(g), st,
+           d_out, raw, lm, g, (int)dir, ws, ws_doubles(g), p->t.D, p->t.Q, p->t.T);
   prof_end(p->prof, st);
 }
 
@@ -3971,40 +4016,47 @@ static bool use_split(const fmm_plan_s *p, size_t nlines) {
 template <int MT>
 static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out,
                         size_t dir, const LineMap &lm, size_t nlines, hipStream_t st,
-                        int band_only, double *ws) {
+                        int band_only, double *ws, double *raw = nullptr) {
   const size_t wsstride = ws_doubles(g);
   if (lm.n && !g.fast && !g.far) {  // per-line lengths: not in k_down
     set_error("lines of uneven length need a plan with leaf size s <= 64");
     return -1;
   }
   if (band_only && g.s <= kBandMaxS) {  // directM
-    launch_band(p, g, d_in, d_out, dir, lm, nlines, st, 1, K_DOWN_BAND);
+    launch_band(p, g, d_in, d_out, dir, lm, nlines, st, LINES_PLAIN, 1, K_DOWN_BAND);
     return 0;
   }
   const bool split = g.far && use_split(p, nlines), fuse = g.far && !split;
-  if (split) launch_band(p, g, d_in, d_out, dir, lm, nlines, st, 0, K_BAND);
+  int order = lm.across ? LINES_ACROSS : raw ? LINES_RAW : LINES_PLAIN;
+  double *sums = raw ? raw : d_out;  // where the band sums go
+  if (split) launch_band(p, g, d_in, sums, dir, lm, nlines, st, order, 0, K_BAND);
   if (!band_only) {
     const bool s16 = (g.s & 15) == 0;
     dim3 gu(4u << g.lu, (unsigned)nlines);
     const bool b8 = fuse && !lm.across && band_by_8(g, nlines);
     const int nb = fuse ? (int)band_groups(g, b8 ? 8 : 16) : 0;
-    const int order = lm.across ? UP_ACROSS
-                      : fuse && !b8 && nlines > 1 && (unsigned)nb < gu.x ? UP_FLAT : UP_PLAIN;
-    if (order != UP_PLAIN)
+    if (order == LINES_PLAIN && fuse && !b8 && nlines > 1 && (unsigned)nb < gu.x)
+      order = LINES_FLAT;
+    if (order == LINES_FLAT || order == LINES_ACROSS)
       gu.x += nb;
+    else if (fuse && order == LINES_RAW && !b8 && lm.es >= 8)  // in turn
+      gu.x = (nb + 7) / 8 * (8 + 8 * (gu.x / nb));
     else if (fuse)
       gu = dim3(std::max(gu.x, (unsigned)nb), gu.y, 2);
-    const BandArgs bu{d_out, dir == L2C ? p->t.a : p->t.an, p->t.head[dir], nb};
+    const BandArgs bu{sums, dir == L2C ? p->t.a : p->t.an, p->t.head[dir], nb};
     prof_begin(p->prof, K_UP_SUBTREE, st);
     if (MT == 18 && up18_eligible(g)) {
       const size_t shu = std::max(8 * (size_t)up18_lds(g).total,
                                   fuse ? band_shared_bytes(g, b8 ? 8 : 16) : 0);
       // (calls with lines in turn are past band_by_8's bounds)
       auto kernel =
-          order == UP_ACROSS ? (s16 ? k_up<true, 16, UP_ACROSS> : k_up<false, 16, UP_ACROSS>)
-          : order == UP_FLAT ? (s16 ? k_up<true, 16, UP_FLAT> : k_up<false, 16, UP_FLAT>)
-          : b8               ? (s16 ? k_up<true, 8, UP_PLAIN> : k_up<false, 8, UP_PLAIN>)
-                             : (s16 ? k_up<true, 16, UP_PLAIN> : k_up<false, 16, UP_PLAIN>);
+          order == LINES_ACROSS ? (s16 ? k_up<true, 16, LINES_ACROSS> : k_up<false, 16, LINES_ACROSS>)
+          : order == LINES_FLAT ? (s16 ? k_up<true, 16, LINES_FLAT> : k_up<false, 16, LINES_FLAT>)
+          : order == LINES_RAW
+              ? (b8 ? (s16 ? k_up<true, 8, LINES_RAW> : k_up<false, 8, LINES_RAW>)
+                    : (s16 ? k_up<true, 16, LINES_RAW> : k_up<false, 16, LINES_RAW>))
+          : b8 ? (s16 ? k_up<true, 8, LINES_PLAIN> : k_up<false, 8, LINES_PLAIN>)
+               : (s16 ? k_up<true, 16, LINES_PLAIN> : k_up<false, 16, LINES_PLAIN>);
       launch_k(p->prof, kernel, gu, kUpNT, shu, st, d_in, lm, g, (int)dir, p->t.T, p->t.U, p->t.P,
                ws, wsstride, bu);
     } else if (MT > 0 && g.gu >= 3 && nlines <= 8) {
@@ -4061,7 +4113,7 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
     prof_end(p->prof, st);
   }
   if (g.far) {
-    launch_far(p, g, d_out, dir, lm, nlines, st, ws, fuse ? K_DOWN_BAND : K_FAR);
+    launch_far(p, g, d_out, raw, dir, lm, nlines, st, order, ws, fuse ? K_DOWN_BAND : K_FAR);
     return 0;
   }
   if (g.fast) {
@@ -4090,9 +4142,18 @@ static int launch_fmm(fmm_plan_s *p, const double *d_in, double *d_out, size_t d
                       const LineMap &lm, size_t nlines, hipStream_t st, int band_only) {
   double *ws = nullptr;
   const Geo &g = call_geo(p, nlines);
-  if (ensure_ws(p, nlines, g, &ws)) return -1;
-  const int rc = g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws)
-                           : launch_fmm_m<0>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws);
+  bool raw = !band_only && raw_sums(g, lm, nlines);
+  if (raw && p->wl_cap < nlines * (ws_doubles(g) + p->N)) {
+    // nothing is allocated for them in a call that is being captured
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    L2C_HIP(hipStreamIsCapturing(st, &cs), -1);
+    raw = cs == hipStreamCaptureStatusNone;
+  }
+  if (ensure_ws(p, nlines, g, &ws, raw)) return -1;
+  double *rw = raw ? ws + nlines * ws_doubles(g) : nullptr;
+  const int rc =
+      g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws, rw)
+                : launch_fmm_m<0>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws);
   if (rc) return rc;
   L2C_HIP(hipGetLastError(), -1);
   return 0;
@@ -4309,19 +4370,21 @@ static int run_lines_scratch(fmm_plan_s *p, double *scr, const double *d_in, dou
     return 0;
   }
   const size_t wsd = std::max(ws_doubles(p->geo), ws_doubles(p->geo1));
-  const size_t per = std::min<size_t>(65535, kScratchDoubles / wsd);
+  lm.across = lines_across(lm, p->N, nlines);
+  const bool raw = raw_sums(p->geo, lm, nlines) && wsd + p->N <= kScratchDoubles;
+  const size_t per = std::min<size_t>(65535, kScratchDoubles / (wsd + (raw ? p->N : 0)));
   if (per == 0) {
     set_error("l2c_execute_lines_device_noalloc: one line of this plan needs " +
               std::to_string(wsd * sizeof(double)) + " bytes of workspace, more than the " +
               std::to_string(kScratchDoubles * sizeof(double)) + "-byte scratch");
     return -1;
   }
-  lm.across = lines_across(lm, p->N, nlines);
   for (size_t l0 = 0; l0 < nlines; l0 += per) {
     lm.l0 = l0;
     const size_t nl = std::min(per, nlines - l0);
     const Geo &g = call_geo(p, nl);
-    const int rc = g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr)
+    double *rw = raw ? scr + nl * wsd : nullptr;
+    const int rc = g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr, rw)
                              : launch_fmm_m<0>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr);
     if (rc) return rc;
     L2C_HIP(hipGetLastError(), -1);

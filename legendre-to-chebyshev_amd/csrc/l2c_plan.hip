@@ -898,7 +898,8 @@ fmm_plan_s *create_fmm_impl(size_t N, size_t maxs, size_t M, size_t direction, s
   // multipole store and staging
   const size_t slots = slot_base(L);
   (void)slots;
-  p->wl_cap = std::max(ws_doubles(g), ws_doubles(p->geo1));
+  // (a far plan's with room for the band sums of one strided transform)
+  p->wl_cap = std::max(ws_doubles(g), ws_doubles(p->geo1)) + (g.far ? N : 0);
   // (host staging buffers are allocated by the first call with host arrays)
   if (dmalloc(&p->d_wl, p->wl_cap, acct)) {
     destroy_fmm(p);

@@ -168,38 +168,3 @@ def test_tune_cache_of_other_kernels(amd, tmp_path):
             assert all(c["cached"] for c in amd.BatchPlan(lengths, 18, amd.L2C, tune=True).classes())
     finally:
         amd.tune_cache(None)
-
-
-def test_batch_graph_other_arrays(amd):
-    """With the graph on: the first arrays that two calls in a row share are recorded and
-    replayed; other arrays, the other direction and calls after l2c_batch_graph(0) run
-    launch by launch, in turn with the replays, on the plan's and on a caller's stream;
-    every result as without the graph, bit for bit."""
-    import torch
-    announce("batch graph, other arrays")
-    lengths = amd.log_uniform_lengths(300, seed=7)
-    bp = amd.BatchPlan(lengths, 18, amd.BOTH, tune=False)
-    u = [amd.packed_coefficients(lengths, seed=s) for s in (1, 2)]
-    din = [amd.DeviceBuffer(bp.total) for _ in u]
-    dout = [amd.DeviceBuffer(bp.total) for _ in u]
-    for b, x in zip(din, u):
-        b.upload(x)
-    sp = torch.cuda.Stream().cuda_stream
-
-    def call(k, d, stream=None):
-        dout[k].upload(np.full(bp.total, 7.0))
-        bp.execute_device(din[k].ptr, dout[k].ptr, d, stream=stream)
-        torch.cuda.synchronize()
-        return dout[k].download()
-
-    ref = [[call(k, d) for d in (0, 1)] for k in (0, 1)]
-    bp.graph(True)
-    turns = [(0, 0)] * 3 + [(1, 0)] * 3 + [(0, 0), (1, 0)] * 3 + [(0, 1), (0, 0), (1, 1), (0, 0)]
-    for stream in (None, sp):
-        for n, (k, d) in enumerate(turns):
-            print(f"  call {n}: arrays {k} dir {d} caller's stream {stream is not None}", flush=True)
-            assert np.array_equal(call(k, d, stream), ref[k][d]), (n, k, d)
-    bp.graph(False)
-    assert np.array_equal(call(0, 0, sp), ref[0][0])
-    bp.graph(True)
-    assert np.array_equal(call(0, 0, sp), ref[0][0])

@@ -286,3 +286,35 @@ def test_shallow_tree_lines(amd, orc, monkeypatch, N, maxs, lines):
         for k in (0, lines - 1):
             ref = op.execute(np.ascontiguousarray(x[k * N:(k + 1) * N]), d)
             assert relerr(outs[0][k * N:(k + 1) * N], ref) <= tol(N)
+
+
+@pytest.mark.parametrize("split", [0, 1])
+@pytest.mark.parametrize("N,maxs,stride", [(20000, 64, 8), (1 << 16, 64, 3), (100001, 36, 16),
+                                           (1 << 18, 64, 9), (70000, 50, 2), (9000, 128, 5)])
+def test_strided_single(amd, monkeypatch, split, N, maxs, stride):
+    """A single transform whose elements lie apart, the band sums in the workspace until
+    the far field is added: as on contiguous arrays, bit for bit; what lies between the
+    output's elements stays, and a plan graph replays it."""
+    announce(f"strided single N={N} maxs={maxs} stride={stride} split={split}")
+    if split:
+        monkeypatch.setenv("L2C_DOWN_SPLIT", "1")
+    p = amd.FMMPlan(N, maxs, 18, amd.BOTH)
+    x = np.random.default_rng(N + stride).uniform(-1, 1, N)
+    gap = np.full((N, stride), 3.0)
+    gap[:, 0] = x
+    din, dout = amd.DeviceBuffer(N * stride), amd.DeviceBuffer(N * stride)
+    for d in (0, 1):
+        din.upload(x)
+        p.execute_device(din.ptr, dout.ptr, d)
+        p.synchronize()
+        ref = dout.download(N)
+        din.upload(gap.ravel())
+        for graph in (False, True, True):
+            p.graph(graph)
+            dout.upload(np.full(N * stride, 7.0))
+            p.execute_device(din.ptr, dout.ptr, d, stride=stride)
+            p.synchronize()
+            g = dout.download().reshape(N, stride)
+            assert np.array_equal(g[:, 0], ref), (d, graph)
+            assert np.all(g[:, 1:] == 7.0)
+        p.graph(False)
