@@ -3899,8 +3899,8 @@ static const Geo &call_geo(const fmm_plan_s *p, size_t nlines) {
 // 2 113 / 118.  (With the band inside the downward kernel, whose passes over the array are
 // two fewer, 2^20 at 16 87, at 8 68, 4 lines at 8 267.)  Lines that lie side by side share
 // their cache lines instead (place).
-static bool raw_sums(const Geo &g, const LineMap &lm, size_t nlines) {
-  return g.far && lm.es > 1 && !lm.across &&
+static bool raw_sums(const Geo &g, const LineMap &lm, size_t nlines, bool across) {
+  return g.far && lm.es > 1 && !across &&
          (nlines == 1 || band_groups(g, 16) >= 4u << g.lu);  // (else LINES_FLAT)
 }
 
@@ -4016,7 +4016,7 @@ static bool use_split(const fmm_plan_s *p, size_t nlines) {
 template <int MT>
 static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double *d_out,
                         size_t dir, const LineMap &lm, size_t nlines, hipStream_t st,
-                        int band_only, double *ws, double *raw = nullptr) {
+                        int band_only, double *ws, double *raw = nullptr, bool across = false) {
   const size_t wsstride = ws_doubles(g);
   if (lm.n && !g.fast && !g.far) {  // per-line lengths: not in k_down
     set_error("lines of uneven length need a plan with leaf size s <= 64");
@@ -4027,13 +4027,13 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
     return 0;
   }
   const bool split = g.far && use_split(p, nlines), fuse = g.far && !split;
-  int order = lm.across ? LINES_ACROSS : raw ? LINES_RAW : LINES_PLAIN;
+  int order = across ? LINES_ACROSS : raw ? LINES_RAW : LINES_PLAIN;
   double *sums = raw ? raw : d_out;  // where the band sums go
   if (split) launch_band(p, g, d_in, sums, dir, lm, nlines, st, order, 0, K_BAND);
   if (!band_only) {
     const bool s16 = (g.s & 15) == 0;
     dim3 gu(4u << g.lu, (unsigned)nlines);
-    const bool b8 = fuse && !lm.across && band_by_8(g, nlines);
+    const bool b8 = fuse && !across && band_by_8(g, nlines);
     const int nb = fuse ? (int)band_groups(g, b8 ? 8 : 16) : 0;
     if (order == LINES_PLAIN && fuse && !b8 && nlines > 1 && (unsigned)nb < gu.x)
       order = LINES_FLAT;
@@ -4139,10 +4139,11 @@ static int launch_fmm_m(fmm_plan_s *p, const Geo &g, const double *d_in, double 
 }
 
 static int launch_fmm(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir,
-                      const LineMap &lm, size_t nlines, hipStream_t st, int band_only) {
+                      const LineMap &lm, size_t nlines, hipStream_t st, int band_only,
+                      bool across = false) {
   double *ws = nullptr;
   const Geo &g = call_geo(p, nlines);
-  bool raw = !band_only && raw_sums(g, lm, nlines);
+  bool raw = !band_only && raw_sums(g, lm, nlines, across);
   if (raw && p->wl_cap < nlines * (ws_doubles(g) + p->N)) {
     // nothing is allocated for them in a call that is being captured
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -4152,7 +4153,7 @@ static int launch_fmm(fmm_plan_s *p, const double *d_in, double *d_out, size_t d
   if (ensure_ws(p, nlines, g, &ws, raw)) return -1;
   double *rw = raw ? ws + nlines * ws_doubles(g) : nullptr;
   const int rc =
-      g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws, rw)
+      g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws, rw, across)
                 : launch_fmm_m<0>(p, g, d_in, d_out, dir, lm, nlines, st, band_only, ws);
   if (rc) return rc;
   L2C_HIP(hipGetLastError(), -1);
@@ -4305,10 +4306,10 @@ int run_lines(fmm_plan_s *p, const double *d_in, double *d_out, size_t dir, size
   }
   // lines go in grid.y: at most 65535 per launch, each chunk reusing the
   // front of the plan's line workspace
-  lm.across = lines_across(lm, p->N, nlines);
+  const bool across = lines_across(lm, p->N, nlines);
   for (size_t l0 = 0; l0 < nlines; l0 += 65535) {
     lm.l0 = l0;
-    if (launch_fmm(p, d_in, d_out, dir, lm, std::min<size_t>(65535, nlines - l0), st, 0))
+    if (launch_fmm(p, d_in, d_out, dir, lm, std::min<size_t>(65535, nlines - l0), st, 0, across))
       return -1;
   }
   return 0;
@@ -4370,8 +4371,8 @@ static int run_lines_scratch(fmm_plan_s *p, double *scr, const double *d_in, dou
     return 0;
   }
   const size_t wsd = std::max(ws_doubles(p->geo), ws_doubles(p->geo1));
-  lm.across = lines_across(lm, p->N, nlines);
-  const bool raw = raw_sums(p->geo, lm, nlines) && wsd + p->N <= kScratchDoubles;
+  const bool across = lines_across(lm, p->N, nlines);
+  const bool raw = raw_sums(p->geo, lm, nlines, across) && wsd + p->N <= kScratchDoubles;
   const size_t per = std::min<size_t>(65535, kScratchDoubles / (wsd + (raw ? p->N : 0)));
   if (per == 0) {
     set_error("l2c_execute_lines_device_noalloc: one line of this plan needs " +
@@ -4384,7 +4385,7 @@ static int run_lines_scratch(fmm_plan_s *p, double *scr, const double *d_in, dou
     const size_t nl = std::min(per, nlines - l0);
     const Geo &g = call_geo(p, nl);
     double *rw = raw ? scr + nl * wsd : nullptr;
-    const int rc = g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr, rw)
+    const int rc = g.M == 18 ? launch_fmm_m<18>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr, rw, across)
                              : launch_fmm_m<0>(p, g, d_in, d_out, dir, lm, nl, st, 0, scr);
     if (rc) return rc;
     L2C_HIP(hipGetLastError(), -1);

@@ -140,9 +140,6 @@ struct LineMap {
   // first line of this launch in the (n0, ls0, ls1) numbering, for batches
   // split over several launches (packed tables are offset by pointer instead)
   size_t l0 = 0;
-  // launches of grid (groups, lines): the kernels whose work-groups take the same
-  // elements of neighbouring lines in turn (see place)
-  int across = 0;
 };
 __host__ __device__ inline size_t line_off(const LineMap &m, size_t l) {
   return m.off ? m.off[l] : ((m.l0 + l) / m.n0) * m.ls1 + ((m.l0 + l) % m.n0) * m.ls0;
