@@ -157,13 +157,20 @@ __device__ __forceinline__ double2 quarter_root(const double2 *ts, int u) {
 // a column stride that keeps neighbouring columns apart (8 / NC mod 8 elements:
 // loads and stores run the columns fastest).  Not where it would leave one
 // work-group per CU instead of two.  With columns of L + 1 and no padding, bank
-// conflicts took 1.3 of the 2.1 us that the LDS is busy in a pass of N = 2^20.
-template <int LOGL, int NC>
+// conflicts took 1.3 of the 2.1 us that the LDS is busy in a pass of N = 2^20.  The
+// one-pass kernels (ONE) lose more by three work-groups to a CU instead of four than they
+// gain by the column stride: where the wide stride costs one, the columns follow each
+// other at the next odd stride after their last element (131072 DCT-II lines of 32 17.2 ->
+// 14.7 us, 65536 of 64 17.3 -> 15.0; without padding 14.9 and 16.0).
+template <int LOGL_, int NC_, bool ONE = false, bool PADDED = true>
 struct Cols {
-  static constexpr int L = 1 << LOGL, LP = L + L / 8;
-  static constexpr bool PAD = LOGL >= 4 && (NC * (LP + 8) + L / 4) * 16 <= 80 * 1024;
+  static constexpr int LOGL = LOGL_, NC = NC_, L = 1 << LOGL, LP = L + L / 8;
   static constexpr int STEP = NC >= 8 ? 1 : 8 / NC;
-  static constexpr int LD = PAD ? LP + (STEP + 8 - LP % 8) % 8 : L + 1;
+  static constexpr bool PAD = PADDED && LOGL >= 4 && (NC * (LP + 8) + L / 4) * 16 <= 80 * 1024;
+  static constexpr int WIDE = LP + (STEP + 8 - LP % 8) % 8, ODD = (LP - 1) | 1;
+  // work-groups per CU with columns of ld elements, the quarter table and the line starts
+  static constexpr int per_cu(int ld) { return 160 * 1024 / ((NC * ld + L / 4) * 16 + NC * 8); }
+  static constexpr int LD = !PAD ? L + 1 : ONE && per_cu(WIDE) < per_cu(ODD) ? ODD : WIDE;
   __device__ static int at(int col, int i) { return col * LD + (PAD ? i + (i >> 3) : i); }
   // at(col, i + n) - at(col, i) where i mod 8 + n mod 8 < 8, as for all accesses of a
   // butterfly, which then share one address; with one each, k_dct2_p1 for columns of
@@ -175,10 +182,9 @@ struct Cols {
 // One Stockham stage of radix R on NC columns of length L held in LDS (Cols).
 // Sub-transform size 2^LOGNS before the stage.  The
 // reads of every butterfly go to registers, then the stage writes in place.
-template <int LOGL, int NC, int T, int R, int LOGNS, int S>
+template <class Z, int T, int R, int LOGNS, int S>
 __device__ __forceinline__ void fft_stage(double2 *buf, const double2 *ts) {
-  using Z = Cols<LOGL, NC>;
-  constexpr int L = 1 << LOGL, Q = L / R, TOT = NC * Q;
+  constexpr int LOGL = Z::LOGL, L = 1 << LOGL, Q = L / R, TOT = Z::NC * Q;
   constexpr int NB = (TOT + T - 1) / T, NS = 1 << LOGNS;
   constexpr int STEP = L / (NS * R);
   double2 v[NB][R];
@@ -220,12 +226,13 @@ __device__ __forceinline__ void fft_stage(double2 *buf, const double2 *ts) {
 // length 2^LOGL in stages of radix 2^LOGRM (8 or 4), a smaller stage first
 // when LOGL is not a multiple of LOGRM.  The caller synchronises before the
 // call.
-template <int LOGL, int NC, int T, int S, int LOGRM = 3, int LOGNS = 0>
+template <class Z, int T, int S, int LOGRM = 3, int LOGNS = 0>
 __device__ __forceinline__ void fft_cols(double2 *buf, const double2 *ts) {
+  constexpr int LOGL = Z::LOGL;
   if constexpr (LOGNS < LOGL) {
     constexpr int LOGR = (LOGNS == 0 && LOGL % LOGRM) ? LOGL % LOGRM : LOGRM;
-    fft_stage<LOGL, NC, T, 1 << LOGR, LOGNS, S>(buf, ts);
-    fft_cols<LOGL, NC, T, S, LOGRM, LOGNS + LOGR>(buf, ts);
+    fft_stage<Z, T, 1 << LOGR, LOGNS, S>(buf, ts);
+    fft_cols<Z, T, S, LOGRM, LOGNS + LOGR>(buf, ts);
   }
 }
 
@@ -310,6 +317,13 @@ __device__ __forceinline__ void line_starts(size_t *loff, const LineMap &lm, siz
 // lines with unit element stride at even offsets, and strided lines.
 enum { kVecs = 0, kLinesUnit = 1, kLinesStrided = 2 };
 
+// The columns of a one-pass kernel.  k_dct2_1p for columns of 1024 and for strided ones of
+// 32 takes 130 and 136 registers with padding, 122 and 125 without, and more than 128 cost
+// the fourth work-group too.
+template <int KIND, int LOGM, int LAY>
+using Cols1 = Cols<LOGM, (kElems >> LOGM), true,
+                   !(KIND == 2 && (LOGM == 10 || (LOGM == 5 && LAY == kLinesStrided)))>;
+
 // One pass for M = 2^LOGM <= 2048: NV = 2048 / M vectors per work-group.
 // Vector v (v < count) starts at v N (kVecs) or line_off(lm, v) (lines), its
 // elements lm.es apart (kLinesStrided) or 1 apart.
@@ -317,7 +331,7 @@ template <int LOGM, int NV, int LAY>
 __global__ void __launch_bounds__(kElems / 8)
     k_dct2_1p(const double *__restrict__ x, double *__restrict__ y, size_t count, LineMap lm,
               Tabs tb) {
-  using Z = Cols<LOGM, NV>;
+  using Z = Cols1<2, LOGM, LAY>;
   constexpr int M = 1 << LOGM, LD = Z::LD, H = M / 2, T = kElems / 8;
   constexpr int NI = NV * M / T, NL = NV * H / T;  // items per thread: post, load
   extern __shared__ double2 z[];
@@ -364,7 +378,7 @@ __global__ void __launch_bounds__(kElems / 8)
     }
   }
   __syncthreads();
-  fft_cols<LOGM, NV, T, -1>(z, ts);
+  fft_cols<Z, T, -1>(z, ts);
 #pragma unroll
   for (int it = 0; it < NI; ++it) {
     int vi, k;
@@ -412,7 +426,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     z[Z::at(partner<C>(i), L - 1 - n2)] = make_double2(p1[it].y, p0[it].y);
   }
   __syncthreads();
-  fft_cols<LOGL, NC, T, -1, PT == 8 ? 3 : 2>(z, ts);
+  fft_cols<Z, T, -1, PT == 8 ? 3 : 2>(z, ts);
 #pragma unroll
   for (int it = 0; it < PT; ++it) {
     const int id = threadIdx.x + it * T, i = id / L, k2 = id % L;
@@ -454,7 +468,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 #pragma unroll
   for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
-  fft_cols<LOGL, NC, T, -1, PT == 8 ? 3 : 2>(z, ts);
+  fft_cols<Z, T, -1, PT == 8 ? 3 : 2>(z, ts);
   // the partner of column k2: itself for k2 = 0 (row (L - k1) mod L) and for
   // k2 = M2/2, else column partner(i); rows run backwards (L - 1 - k1)
   const int ip = (k2 == M2 / 2 || k2 == 0) ? i : partner<C>(i);
@@ -485,7 +499,7 @@ template <int LOGM, int NV, int LAY>
 __global__ void __launch_bounds__(kElems / 8)
     k_dct3_1p(const double *__restrict__ Y, double *__restrict__ x, size_t count, LineMap lm,
               Tabs tb) {
-  using Z = Cols<LOGM, NV>;
+  using Z = Cols1<3, LOGM, LAY>;
   constexpr int M = 1 << LOGM, LD = Z::LD, H = M / 2, N = 2 * M, T = kElems / 8;
   constexpr int NI = NV * M / T, NL = NV * N / T, NS = NV * H / T;
   extern __shared__ double2 z[];
@@ -538,7 +552,7 @@ __global__ void __launch_bounds__(kElems / 8)
     z[Z::at(vi, k)] = zp[it];
   }
   __syncthreads();
-  fft_cols<LOGM, NV, T, 1>(z, ts);
+  fft_cols<Z, T, 1>(z, ts);
 #pragma unroll
   for (int it = 0; it < NS; ++it) {
     int vi, m;
@@ -623,7 +637,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
     const size_t m1 = size_t(col_negate<C>(id / L, a, M1));
     pass_root_load(tb, (m1 * size_t(id % L)) & (M - 1), th[it], tl[it]);
   }
-  fft_cols<LOGL, NC, T, 1, PT == 8 ? 3 : 2>(z, ts);
+  fft_cols<Z, T, 1, PT == 8 ? 3 : 2>(z, ts);
 #pragma unroll
   for (int it = 0; it < PT; ++it) {
     const int id = threadIdx.x + it * T, j = id / L, k2 = id % L;
@@ -654,7 +668,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 #pragma unroll
   for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
-  fft_cols<LOGL, NC, T, 1, PT == 8 ? 3 : 2>(z, ts);
+  fft_cols<Z, T, 1, PT == 8 ? 3 : 2>(z, ts);
   const int ip = partner<C>(i);
 #pragma unroll
   for (int it = 0; it < PT / 2; ++it) {
@@ -705,7 +719,7 @@ __global__ void __launch_bounds__(NC * (1 << LOGL) / PT)
 #pragma unroll
   for (int it = 0; it < PT; ++it) z[Z::at(i, (threadIdx.x + it * T) / NC)] = d[it];
   __syncthreads();
-  fft_cols<LOGL, NC, T, S, PT == 8 ? 3 : 2>(z, ts);
+  fft_cols<Z, T, S, PT == 8 ? 3 : 2>(z, ts);
 #pragma unroll
   for (int it = 0; it < PT; ++it) {
     const size_t k2 = (threadIdx.x + it * T) / NC;
@@ -799,9 +813,9 @@ template <int LOGM, int LAY>
 void launch_1p_lay(const l2c_dct_plan *p, const double *in, double *out, int kind, size_t count,
                    const LineMap &lm, hipStream_t st) {
   constexpr int M = 1 << LOGM, NV = kElems / M;
+  const int ld = kind == 2 ? Cols1<2, LOGM, LAY>::LD : Cols1<3, LOGM, LAY>::LD;
   const size_t shmem =
-      (size_t(NV) * Cols<LOGM, NV>::LD + (LOGM > 3 ? M / 4 : 0)) * sizeof(double2) +
-      NV * sizeof(size_t);
+      (size_t(NV) * ld + (LOGM > 3 ? M / 4 : 0)) * sizeof(double2) + NV * sizeof(size_t);
   const dim3 grid(unsigned((count + NV - 1) / NV)), blk(kElems / 8);
   if (kind == 2)
     hipLaunchKernelGGL((k_dct2_1p<LOGM, NV, LAY>), grid, blk, shmem, st, in, out, count, lm, p->tb);

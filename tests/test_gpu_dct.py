@@ -252,3 +252,27 @@ def test_lines_errors(amd):
     small = amd.DCTPlan(64)
     assert lib.l2c_execute_dct_lines_device(small._plan, buf.ptr, buf.ptr, 2, 0, 1, 0, 0, 1, None) == -1
     assert lib.l2c_execute_dct_lines_device(small._plan, buf.ptr, buf.ptr, 5, 1, 1, 0, 0, 1, None) == -1
+
+
+@pytest.mark.parametrize("kind", [2, 3])
+@pytest.mark.parametrize("N", [32, 64, 512, 1024, 2048, 4096])
+def test_full_work_groups(amd, orc, N, kind):
+    """Every column of the one-pass kernels' LDS filled, and one line more: 2048 / (N / 2)
+    lines fill a work-group.  Vectors, lines along rows and lines along columns."""
+    nl = 4096 // N * 2 + 1
+    check(amd, orc, N, nl, kind, 7 * N + kind)
+    for shape, axis in (((nl, N + 2), 1), ((N, nl), 0)):
+        announce(f"dct full work-groups kind={kind} {shape} axis={axis}")
+        x = np.random.default_rng(N + axis).uniform(-1, 1, shape)
+        plan = amd.DCTPlan(N)
+        din, dout = amd.DeviceBuffer(x.size), amd.DeviceBuffer(x.size)
+        din.upload(x.ravel())
+        dout.upload(np.zeros(x.size))
+        ls, es = ((shape[1], 1) if axis else (1, nl))
+        plan.execute_lines_device(din.ptr, dout.ptr, kind, nl, nl, ls, 0, es)
+        plan.synchronize()
+        lines = (lambda a: a[:, :N]) if axis else (lambda a: a.T)
+        ref = orc.redft(np.ascontiguousarray(lines(x)), kind)
+        y = lines(dout.download().reshape(shape))
+        err = max(relerr(a, b) for a, b in zip(y, ref))
+        assert err < tol(N), (axis, err)
