@@ -7,15 +7,22 @@
 //   k_up    leaf moments (step 1) on FP64 MFMA and the upward pass (step 2)
 //           inside a subtree of 2^gu <= 16 leaf chunks; writes the multipole
 //           store for levels >= lu and, for each level l < lu, the subtree
-//           root's contribution P(lu-l, .) w_root to its level-l ancestor.
+//           root's contribution P(lu-l, .) w_root to its level-l ancestor.  At
+//           rank 18 and s <= 64 other work-groups of the same launch do the
+//           near field (band_group, FP64 VALU): the raw band sums go to the
+//           output, or to the workspace where the output is strided.
 //   k_m2l   M2L (step 3) of every block of every level, streaming the M2L
-//           matrices through LDS with coalesced loads (each matrix read once
-//           for both parities); blocks above lu first sum the k_up
-//           contributions into their multipoles.  HBM-bound.
-//   k_down  per subtree of 2^gd leaf chunks: L2L (step 4) down the ancestor
-//           chain and the subtree, the near-field band (FP64 VALU), leaf
-//           evaluation (step 5), final scaling, one coalesced store of the
-//           output (which is overwritten, not accumulated).
+//           matrices (k_m2l_t: block rows in registers, k_m2l: through LDS,
+//           k_m2l_mma: FP64 MFMA for many lines; each matrix read once for both
+//           parities); blocks above lu first sum the k_up contributions into
+//           their multipoles.  HBM-bound.
+//   k_far   per subtree of 2^gd leaf chunks: L2L (step 4) down the ancestor
+//           chain and the subtree, leaf evaluation (step 5) on FP64 MFMA, added
+//           to the band sums, final scaling, one store of the output (which is
+//           overwritten, not accumulated).
+//
+// Other ranks and s > 64: k_up_any, and k_down8r, k_down8 or k_down, which do the
+// near field and k_far's work in one launch.
 //
 // Workspace per line: [multipoles: slot_base(L) x 2M][contributions:
 // lu x 2^(lu+2) x 2M][M2L results: slot_base(L) x 2M]; chunk slot
@@ -3074,7 +3081,6 @@ size_t dband_shared_bytes(int N) {
   const int w = dband_pad(dband_win(std::min((N + 1) / 2, kDbChunk))) + 1;
   return 8 * (size_t)(3 * w + 24);  // windows, the other parts' row sums (G = 1)
 }
-// G = 1 while two work-groups' windows fit one CU's 160 KB of LDS, else 4
 // Entries per thread and batch of the window loads: nine where that saves the
 // first work-groups a batch (N = 4096 7.0 -> 6.3 us a call, 8192 10.9 -> 10.4), else
 // eight (nine: 5000 8.6 -> 8.8, 7000 9.0 -> 9.3)
@@ -3083,6 +3089,7 @@ inline int dband_batch(int N) {
   const int w = dband_win((N + 1) / 2);
   return (w + 2303) / 2304 < (w + 2047) / 2048 ? 9 : 8;
 }
+// G = 1 while two work-groups' windows fit one CU's 160 KB of LDS, else 4
 inline int dband_groups(int N) { return dband_shared_bytes(N) <= 80 * 1024 ? 1 : 4; }
 
 // Columns [t0, t1) of the lane's 8 rows, t0 a multiple of 8; xq, pq, hq: the

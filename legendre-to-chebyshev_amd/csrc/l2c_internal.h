@@ -303,9 +303,8 @@ struct fmm_plan_s {
   // lines with L >= 10; L2C_DOWN_SPLIT
   int down_split = 0;
   // the downward pass of other ranks at s = 16, 32, 64 with wave roles
-  // (k_down8r: tree and far field on
-  // half the waves, the band on the other half; default) or without (0:
-  // k_down8); L2C_DOWN_ROLES
+  // (k_down8r: tree and far field on half the waves, the band on the other
+  // half; default) or without (0: k_down8); L2C_DOWN_ROLES
   int down_roles = 1;
   // band columns moved from k_down8r's band role to its tree role (negative:
   // the other way); L2C_ROLES_SHIFT
